@@ -5,10 +5,9 @@ on one GPU through one batched engine plan (``aimdhf_batch_create``).
 Per geometry of the whole batch:
 
 * one set-up (pairs, Schwarz bounds, screened quartets of every replica) and
-  one integral-evaluation launch per quartet class for all replicas, expanded
-  into one dense two-electron tensor per replica;
+  one integral-evaluation launch per quartet class for all replicas;
 * an SCF whose iteration is one captured HIP graph for all replicas: J/K of
-  every replica in one launch, Fock matrices, energies and commutators as
+  every replica in one or two launches, Fock matrices, energies and commutators as
   batched products, Pulay DIIS with its small systems solved on the device
   (one launch), and the aufbau densities of every replica and spin by
   purification in one launch; one host read per iteration checks convergence;
@@ -67,9 +66,9 @@ class ReplicaBatch:
     screening; ``precision`` "fp64" or "mixed" (FP32 for quartets below the
     switch thresholds in the integral evaluation and the derivative
     integrals, as the single-molecule engine). ``jk_lanes`` (16, 32 or 64)
-    fixes how many lanes digest one J/K element; None lets :meth:`autotune`
-    time the choices on the first geometry. The choice sets the summation
-    order, so runs that must agree bit for bit across processes fix it.
+    fixes the J/K workgroups (four threads per lane); None lets :meth:`autotune`
+    time the choices on the first geometry. Lane sums depend on it in their
+    last bits, so runs that must agree bit for bit across processes fix it.
     """
 
     def __init__(self, molecules: Sequence[tuple], basis: str = "6-31g**", conv_tol: float = 1e-10,
@@ -247,8 +246,8 @@ class ReplicaBatch:
         _lib.check(_lib.lib().aimdhf_jk(self._h, 2, _ptr(D), _ptr(self.J), _ptr(self.K), _stream()))
 
     def autotune(self, reps: int = 5) -> dict[int, float]:
-        """Time the batched J/K digestion at 64, 32 and 16 lanes per output element on the
-        current geometry's integral tensors (reps builds each, HIP events on the current
+        """Time the batched J/K digestion at 64, 32 and 16 lanes (256, 128 and 64 threads a
+        workgroup) on the current geometry's integrals (reps builds each, HIP events on the current
         stream), keep the fastest, and drop the captured SCF graph so the next iteration
         records the new launch. Returns {lanes: ms per build}."""
         L = _lib.lib()

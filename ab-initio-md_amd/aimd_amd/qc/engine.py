@@ -108,7 +108,7 @@ class Engine:
         self.jk_mode = mode
 
     def set_store_units(self, items: int) -> None:
-        """Lane items per store-mode digestion work unit (from the next set_geometry)."""
+        """Least quartets a workgroup of the store-mode digestion takes from a long run of kets."""
         _lib.check(_lib.lib().aimdhf_set_store_units(self._h, int(items)))
         self.store_units = int(items)
 
@@ -117,8 +117,8 @@ class Engine:
     def set_precision(self, precision: str = "fp64", jk_switch: float = 0.0, grad_switch: float = 0.0,
                       delta_switch: float = 0.0) -> None:
         """"fp64", or "mixed": FP32 for quartets whose Schwarz bound (J/K store, from the next
-        set_geometry) or Schwarz-Gamma bound (derivative integrals) is below the switch, and
-        for every stored integral in density-difference builds with max |dD| <= delta_switch."""
+        set_geometry) or Schwarz-Gamma bound (derivative integrals) is below the switch.
+        delta_switch is accepted and has no effect: difference builds sum in FP64."""
         if precision not in self.PRECISIONS:
             raise ValueError(f"precision must be one of {sorted(self.PRECISIONS)}, got {precision!r}")
         _lib.check(_lib.lib().aimdhf_set_precision(self._h, self.PRECISIONS[precision], float(jk_switch),
@@ -131,8 +131,8 @@ class Engine:
         _lib.check(_lib.lib().aimdhf_set_streams(self._h, int(bool(concurrent))))
 
     def jk_info(self) -> dict:
-        """Store state of the current geometry: stored, bytes, K and J gather-list entries and
-        the bytes of integral data one J/K build streams (gather_bytes)."""
+        """Store state of the current geometry: stored, bytes, the quartets one J/K build digests
+        (k_entries; j_entries is 0) and the bytes of integrals it streams (gather_bytes)."""
         st = ctypes.c_int()
         b, ke, je, gd = ctypes.c_int64(), ctypes.c_int64(), ctypes.c_int64(), ctypes.c_int64()
         _lib.check(_lib.lib().aimdhf_jk_info(self._h, ctypes.byref(st), ctypes.byref(b), ctypes.byref(ke),
@@ -141,8 +141,9 @@ class Engine:
                 "j_entries": int(je.value), "gather_bytes": int(gd.value)}
 
     def jk_type_info(self) -> dict:
-        """Store traffic per exchange output type (9), Coulomb pair class (6) and the unique
-        integral bytes per quartet class (21) of the current geometry (zeros in direct mode)."""
+        """Unique integral bytes per quartet class (21) of the current geometry, which one J/K
+        build streams once (zeros in direct mode; the arrays per exchange output type and
+        Coulomb pair class are zero, no reordered copies are kept)."""
         kb, ke = np.zeros(9, np.int64), np.zeros(9, np.int64)
         jb, je = np.zeros(6, np.int64), np.zeros(6, np.int64)
         ub = np.zeros(21, np.int64)
@@ -161,9 +162,8 @@ class Engine:
     def jk_delta(self, ddens: torch.Tensor, threshold: float) -> tuple[torch.Tensor, torch.Tensor]:
         """J, K of density differences for an incremental Fock build.
 
-        In store mode, work units whose largest Schwarz product times max |dD|
-        is below ``threshold`` are skipped, and in mixed precision the integrals
-        are digested in FP32. In direct mode this is :meth:`jk`.
+        In store mode, quartets whose Schwarz product times max |dD| is below
+        ``threshold`` may be skipped. In direct mode this is :meth:`jk`.
         """
         single = ddens.dim() == 2
         D = ddens.reshape(-1, self.nao, self.nao).to(device=self.device, dtype=torch.float64).contiguous()
@@ -222,19 +222,18 @@ class Engine:
     PAIR_CLASS_NAMES = ["ss", "ps", "pp", "ds", "dp", "dd"]
     KIND_NAMES = ([f"jengine_bra_{c}" for c in PAIR_CLASS_NAMES]
                   + [f"exchange_{'spd'[t // 3]}{'spd'[t % 3]}" for t in range(9)]
-                  + ["gather_copies"] + [f"unused_{k}" for k in range(16, 21)]
+                  + [f"unused_{k}" for k in range(15, 21)]
                   + [f"grad_class_{k}" for k in range(21)]
                   + ["geometry", "one_electron", "grad_one", "jk_prologue_epilogue", "jk_hermite_density",
-                     "eri_store", "gather_lists"]
-                  + [f"jstore_{c}" for c in PAIR_CLASS_NAMES]
-                  + [f"kstore_{'spd'[t // 3]}{'spd'[t % 3]}" for t in range(9)]
+                     "eri_store"] + [f"unused_{k}" for k in range(48, 64)]
                   + [f"grad_screen_{k}" for k in range(21)]
                   + ["host_energy_list", "host_owner_lists", "host_store_build", "host_gradient_list"]
-                  + ["host_store_counts", "host_store_bands", "host_store_fill", "host_store_units"]
-                  + ["kstore_reduce", "jstore_reduce", "generic_jk", "generic_grad_two", "unused_97"])
-    NKIND = 98
-    FOCK_KINDS = list(range(0, 15)) + [45, 46] + list(range(49, 64)) + [93, 94, 95]   # per-iteration J/K work
-    STORE_KINDS = [15, 47, 48]                                          # per-geometry store build
+                  + [f"unused_{k}" for k in range(89, 93)]
+                  + ["jk_finish", "digest_all", "generic_jk", "generic_grad_two", "unused_97"]
+                  + [f"digest_class_{k}" for k in range(21)])
+    NKIND = 119
+    FOCK_KINDS = list(range(0, 15)) + [45, 46, 93, 94, 95] + list(range(98, 119))   # per-iteration J/K work
+    STORE_KINDS = [47]                                                  # per-geometry store build
     GRAD_KINDS = list(range(21, 42)) + list(range(64, 85)) + [96]       # derivative ERIs
 
     def profile(self, on: bool = True) -> None:
@@ -250,7 +249,7 @@ class Engine:
 
     def profile_replay(self, kind: int, reps: int = 20) -> float:
         """Average milliseconds of `reps` back-to-back launches of a store-mode digestion
-        kernel (kind 49..63) with the arguments of the last J/K build."""
+        kernel (kind 98 + quartet class) with the arguments of the last J/K build."""
         out = ctypes.c_double()
         _lib.check(_lib.lib().aimdhf_profile_replay(self._h, int(kind), int(reps), _stream(), ctypes.byref(out)))
         return float(out.value)

@@ -61,12 +61,12 @@ class SCFOptions:
     the free device memory). ``incremental_fock`` (default: on in mixed
     precision, off in FP64) builds J and K of every iteration after the first
     from the density difference, J(D) = J(D_prev) + J(D - D_prev), skipping in
-    store mode the work units whose largest Schwarz product times max |dD| is
-    below ``incremental_threshold`` (default: the Schwarz threshold in FP64; in
+    store mode quartets whose Schwarz product times max |dD| is below
+    ``incremental_threshold`` (default: the Schwarz threshold in FP64; in
     mixed precision a tenth of ``conv_energy`` when that is larger, so the
-    skipped contributions stay an order below the SCF's own energy tolerance)
-    and, in mixed precision once max |dD| <= ``delta_fp32_switch``, digesting
-    the difference in FP32.
+    skipped contributions stay an order below the SCF's own energy tolerance).
+    ``delta_fp32_switch`` is accepted and has no effect: difference builds sum
+    the stored integrals in FP64 in both precisions.
     """
     conv_energy: float = 1e-10
     conv_commutator: float = 1e-7

@@ -3,6 +3,7 @@
 
 #include "../../include/aimdhf.h"
 #include "aimdhf_internal.h"
+#include "jk_digest.h"
 
 #include <algorithm>
 #include <chrono>
@@ -69,6 +70,9 @@ int ncart(int l) { return (l + 1) * (l + 2) / 2; }
 int nherm(int L) { return (L + 1) * (L + 2) * (L + 3) / 6; }
 constexpr int NQCLASS = 21;
 constexpr int REC_HDR = 8;
+// single molecules up to nset nao^2 of this digest all classes in one launch: measured per
+// build, (1, 19 AOs) 30 against 174 us, (1, 114) 132 against 187; (2, 100) 183 against 169
+constexpr int SMALL_JK = 200 * 200;
 
 // Boys grid table F_n(k/10), n < 43 (aimd/qc/boys.py:57-75): series for the
 // highest order, then the downward recursion.
@@ -92,9 +96,9 @@ std::vector<double> boys_table() {
 }
 
 // Optional per-launch timing with HIP events on the caller's stream.
-// Kinds as listed at aimdhf_profile_enable in aimdhf.h (0..63).
+// Kinds as listed at aimdhf_profile_enable in aimdhf.h.
 struct Profiler {
-    static constexpr int NKIND = 98;
+    static constexpr int NKIND = 119;
     bool on = false;
     struct Rec {
         int kind;
@@ -238,27 +242,25 @@ struct aimdhf_plan {
     int jk_mode = 0;
     long long store_limit = 0;
     bool stored = false;
-    long long store_base[NQCLASS + 1] = {0};
-    long long store_bytes = 0, k_entries = 0, j_entries = 0;
+    long long store_bytes = 0;
+    // ranked pairs (jk_digest.h): component base of every pair class, the quartet list's
+    // runs, and the byte offset of every class's FP64 and FP32 blocks in the store
+    long long koff[7] = {0}, npao = 0, runbase[NQCLASS + 1] = {0};
+    int list_parts = 1;
+    long long list_off[NQCLASS + 1] = {0}, base64[NQCLASS] = {0}, base32[NQCLASS] = {0};
+    size_t store_need = 0;
+    int lds_limit = 65536;
+    DevBuf d_oab, d_rank_rep, d_rep_shell, d_seg, d_rq, d_gcell, d_lcnt, d_loff, d_lsum, d_lbra, d_lket;
+    DevBuf d_dket, d_kacc, d_jacc, d_dcell, d_geo;
+    aimdhf::DigestArgs last_dig[NQCLASS];
     DevBuf d_gkeep, d_gsel, d_nsel, d_gblk;
     // precision: 0 FP64 everywhere; 1 mixed (FP32 below the switches)
     int precision = 0;
     double jk_switch = 0.0, grad_switch = 0.0;
-    DevBuf d_store, d_qmap, d_kcnt, d_jcnt, d_kseg, d_jseg, d_klist, d_jlist, d_lerr;
-    DevBuf d_kdata, d_jdata, d_kdoff, d_jdoff, d_kdata32, d_jdata32, d_kdoff32, d_jdoff32, d_kbig, d_jbig;
-    long long kdata_total = 0, jdata_total = 0, kdata32_total = 0, jdata32_total = 0;
-    // work units of the store kernels: at most unit_items lane items each
+    DevBuf d_store;
+    // least quartets a workgroup of the J/K digestion takes from a long run
     int unit_items = 1024;
-    int kunit_base[10] = {0}, junit_base[7] = {0};
-    DevBuf d_kunit_os, d_kunit_e, d_out_unit, d_kpart2, d_junit_pc, d_junit_e, d_pair_unit, d_jpart2;
-    // density-difference builds: per-unit largest Schwarz products, max |dD|,
-    // and in mixed precision FP32 copies of the FP64 parts
-    DevBuf d_kunit_q, d_junit_q, d_dmax, d_kdata32b, d_jdata32b;
-    bool have_32b = false;
-    // largest max |dD| at which mixed-precision difference builds digest every
-    // unit in FP32 (larger differences use the FP64 parts of the store)
-    double delta_fp32_max = 1e-3;
-    DevBuf d_tab;                   // store-table temporaries (sizes, unit counts, scan blocks)
+    double delta_fp32_max = 1e-3;   // accepted; every difference build sums in FP64
     DevBuf d_gdmax;                 // per shell pair density maxima for the gradient screening
     long long* h_pin = nullptr;     // pinned host words for the totals and the error flag
     // pinned host staging of the per-geometry list transfers: asynchronous copies on
@@ -267,15 +269,13 @@ struct aimdhf_plan {
     size_t h_stage_cap = 0, h_stage_used = 0;
     // batched plans: independent molecules (replicas) sharing one plan; shells and
     // atoms grouped by replica, pairs and quartets only within a replica, matrices
-    // in the padded layout (replica r's ld x ld block at r ld^2), two-electron
-    // integrals as one dense n_r^4 tensor per replica
+    // in the padded layout (replica r's ld x ld block at r ld^2)
     bool batched = false;
     int nrep = 1, bld = 0;
-    int batch_jk_lanes = 64;        // lanes per output element of the batched J/K digestion
+    int batch_jk_lanes = 64;        // batched J/K digestion: four threads per lane of this and workgroup
     std::vector<int> rep_shell, rep_atom, rep_nao, shell_rep, shell_first, shell_pair0, pair_lo;
-    std::vector<long long> rep_toff, rep_item;
-    long long tens_total = 0;
-    DevBuf d_shell_rep, d_shell_first, d_shell_pair0, d_pair_lo, d_rep_atom, d_rep_nao, d_rep_toff, d_rep_item, d_tens;
+    long long tens_total = 0;       // elements of one dense n_r^4 tensor per replica (aimdhf_batch_layout)
+    DevBuf d_shell_rep, d_shell_first, d_shell_pair0, d_pair_lo, d_rep_atom, d_rep_nao;
     // elements of one stack of matrices (nao^2, or nrep ld^2 for a batch)
     size_t mat_elems() const { return batched ? (size_t)nrep * bld * bld : (size_t)nao * nao; }
     // device address and size of the fixed scratch array of the allocation-free
@@ -285,10 +285,7 @@ struct aimdhf_plan {
     // runtime-l path (a shell with l = 3 or 4): every shell pair i >= j in index
     // order; the energy quartets in d_list / qtotal, the last gradient list in
     // d_glist / gen_gq; bounds per shell pair in d_qshell, per block pair in d_qblock
-    // arguments of the last store-mode J/K build (kernel replays for timing)
-    aimdhf::KSArgs last_ka{};
-    aimdhf::JSArgs last_ja{};
-    bool have_last_store = false;
+    bool have_last_store = false;   // last_dig holds a build at the current geometry
     bool generic = false;
     std::vector<int> gpair_i, gpair_j, gpair_bp, gen_npp;
     std::vector<double> gen_qb;
@@ -378,13 +375,11 @@ struct aimdhf_plan {
                           &d_qshell, &d_qblock, &d_qscr, &d_counts, &d_offsets, &d_list, &d_fx, &d_dsym,
                           &d_charges, &d_glist, &d_gfx, &d_gden, &d_scratch, &d_out_x, &d_out_y, &d_ao_shell,
                           &d_ket_q, &d_kpre, &d_krec, &d_kpair, &d_part_off, &d_part_shell, &d_part_pair,
-                          &d_part_q, &d_dh, &d_jpart, &d_kpart, &d_ket_pair, &d_store, &d_qmap, &d_kcnt,
-                          &d_jcnt, &d_kseg, &d_jseg, &d_klist, &d_jlist, &d_lerr, &d_gkeep, &d_gsel, &d_nsel, &d_gblk,
-                          &d_kdata, &d_jdata, &d_kdoff, &d_jdoff, &d_kdata32, &d_jdata32, &d_kdoff32, &d_jdoff32,
-                          &d_kbig, &d_jbig, &d_kunit_os, &d_kunit_e, &d_out_unit,
-                          &d_kpart2, &d_junit_pc, &d_junit_e, &d_pair_unit, &d_jpart2, &d_kunit_q, &d_junit_q,
-                          &d_dmax, &d_kdata32b, &d_jdata32b, &d_tab, &d_gdmax, &d_shell_rep, &d_shell_first,
-                          &d_shell_pair0, &d_pair_lo, &d_rep_atom, &d_rep_nao, &d_rep_toff, &d_rep_item, &d_tens,
+                          &d_part_q, &d_dh, &d_jpart, &d_kpart, &d_ket_pair, &d_store, &d_oab, &d_rank_rep, &d_rep_shell,
+                          &d_seg, &d_rq, &d_gcell, &d_lcnt, &d_loff, &d_lsum, &d_lbra, &d_lket, &d_dket, &d_kacc,
+                          &d_jacc, &d_dcell, &d_geo, &d_gkeep, &d_gsel, &d_nsel, &d_gblk,
+                          &d_gdmax, &d_shell_rep, &d_shell_first,
+                          &d_shell_pair0, &d_pair_lo, &d_rep_atom, &d_rep_nao,
                           &d_gpair_i, &d_gpair_j})
             b->release();
         if (h_pin) (void)hipHostFree(h_pin);
@@ -419,12 +414,6 @@ struct aimdhf_plan {
         g.boys = d_boys.as<double>();
         g.pair_lo = batched ? d_pair_lo.as<int>() : nullptr;
         return g;
-    }
-
-    const int2* list_of_class(int k) const {
-        long long off = 0;
-        for (int i = 0; i < k; ++i) off += qcount[i];
-        return d_list.as<int2>() + off;
     }
 
     // Class-binned list of unique shell quartets with q_P q_Q >= thr into buf;
@@ -552,370 +541,214 @@ struct aimdhf_plan {
         upload_async(d_part_q, part_q, st);
     }
 
-    // Bytes the integral store of the current list would take: the blocks, up
-    // to six gather-ordered copies of them (four exchange, two Coulomb), the
-    // pair-pair map and the gather lists (about six entries per quartet).
-    long long store_estimate() const {
-        long long dbl = 0;
-        for (int k = 0; k < NQCLASS; ++k) dbl += qcount[k] * aimdhf::store_block(k);
-        long long keys = (long long)npair * (npair + 1) / 2;
-        return 8 * 7 * dbl + 4 * keys + 8 * 6 * qtotal;
-    }
+    int matrix_ld() const { return batched ? bld : nao; }
 
-    aimdhf::KSArgs ks_args(int nset, const double* dens, double* K) const {
-        aimdhf::KSArgs ka;
-        ka.nao = nao;
-        ka.nset = nset;
-        for (int t = 0; t < 10; ++t) ka.out_off[t] = out_off[t];
-        ka.out_x = d_out_x.as<int>();
-        ka.out_y = d_out_y.as<int>();
-        ka.shell_ao = d_shell_ao.as<int>();
-        ka.kseg = d_kseg.as<long long>();
-        ka.klist = d_klist.as<long long>();
-        ka.store = d_store.as<double>();
-        for (int k = 0; k < NQCLASS; ++k) ka.store_base[k] = store_base[k];
-        ka.kdata = d_kdata.as<double>();
-        ka.kdoff = d_kdoff.as<long long>();
-        ka.kdata32 = d_kdata32.as<float>();
-        ka.kdoff32 = d_kdoff32.as<long long>();
-        ka.kbig = d_kbig.as<long long>();
-        for (int t = 0; t < 10; ++t) ka.unit_base[t] = kunit_base[t];
-        long long pb = 0;
-        for (int t = 0; t < 9; ++t) {
-            ka.part_base[t] = pb;
-            pb += (long long)(kunit_base[t + 1] - kunit_base[t]) * std::max(nset, 1) * ncart(t / 3) * ncart(t % 3);
-        }
-        ka.unit_os = d_kunit_os.as<int>();
-        ka.unit_e = d_kunit_e.as<long long>();
-        ka.out_unit = d_out_unit.as<int>();
-        ka.kpart = d_kpart2.as<double>();
-        ka.dens = dens;
-        ka.K = K;
-        ka.delta = 0;
-        ka.unit_q = d_kunit_q.as<double>();
-        ka.dmax = d_dmax.as<double>();
-        ka.dthr = 0.0;
-        ka.d32 = 0.0;
-        ka.kdata32b = have_32b ? d_kdata32b.as<float>() : nullptr;
-        return ka;
-    }
-
-    aimdhf::JSArgs js_args(int nset, const double* dens, double* J) const {
-        aimdhf::JSArgs ja;
-        ja.nao = nao;
-        ja.nset = nset;
-        ja.cls_off = 0;
-        ja.cls_pairs = d_cls_pairs.as<int>();
-        ja.pair_a = d_pair_a.as<int>();
-        ja.pair_b = d_pair_b.as<int>();
-        ja.shell_ao = d_shell_ao.as<int>();
-        ja.jseg = d_jseg.as<long long>();
-        ja.jlist = d_jlist.as<long long>();
-        ja.store = d_store.as<double>();
-        for (int k = 0; k < NQCLASS; ++k) ja.store_base[k] = store_base[k];
-        ja.jdata = d_jdata.as<double>();
-        ja.jdoff = d_jdoff.as<long long>();
-        ja.jdata32 = d_jdata32.as<float>();
-        ja.jdoff32 = d_jdoff32.as<long long>();
-        ja.jbig = d_jbig.as<long long>();
-        for (int c = 0; c < 7; ++c) ja.unit_base[c] = junit_base[c];
-        static const int ncp[6] = {1, 3, 9, 6, 18, 36};
-        long long pb = 0;
-        for (int c = 0; c < 6; ++c) {
-            ja.part_base[c] = pb;
-            pb += (long long)(junit_base[c + 1] - junit_base[c]) * std::max(nset, 1) * ncp[c];
-        }
-        ja.unit_pc = d_junit_pc.as<int>();
-        ja.unit_e = d_junit_e.as<long long>();
-        ja.pair_unit = d_pair_unit.as<int>();
-        ja.jpart = d_jpart2.as<double>();
-        ja.dens = dens;
-        ja.J = J;
-        ja.delta = 0;
-        ja.unit_q = d_junit_q.as<double>();
-        ja.dmax = d_dmax.as<double>();
-        ja.dthr = 0.0;
-        ja.d32 = 0.0;
-        ja.jdata32b = have_32b ? d_jdata32b.as<float>() : nullptr;
-        return ja;
-    }
-
-    // Evaluate the screened quartets into the store and build the J and K
-    // gather lists. Synchronises the stream.
-    void build_store(hipStream_t st) {
-        long long off = 0;
+    // Screened quartets of the current geometry (quartet_list.hip): rank-ordered
+    // screening values, runs of kets per bra and class, totals to the host.
+    // Synchronises the stream.
+    void build_quartets(double thr, double sw, hipStream_t st) {
+        if (!h_pin) HIPCHECK(hipHostMalloc((void**)&h_pin, sizeof(long long) * 64 + sizeof(aimdhf::DigestGeo) * NQCLASS));
+        aimdhf::GeoArgs g;
+        g.nshell = nshell;
+        g.npair = npair;
+        g.shell_l = d_shell_l.as<int>();
+        g.shell_rep = batched ? d_shell_rep.as<int>() : nullptr;
+        g.shell_first = batched ? d_shell_first.as<int>() : nullptr;
+        g.shell_pair0 = batched ? d_shell_pair0.as<int>() : nullptr;
+        g.rep_shell = batched ? d_rep_shell.as<int>() : nullptr;
+        g.cls_pairs = d_cls_pairs.as<int>();
+        g.qscr = d_qscr.as<double>();
+        g.rq = d_rq.as<double>();
+        g.gcell = d_gcell.as<unsigned long long>();
+        g.nrep = nrep;
+        aimdhf::launch_geo_bounds(g, st);
+        list_parts = sw > 0.0 ? 2 : 1;
+        long long runs = 0;
         for (int k = 0; k < NQCLASS; ++k) {
-            store_base[k] = off;
-            off += qcount[k] * aimdhf::store_block(k);
+            runbase[k] = runs;
+            runs += (long long)list_parts * ncls[bra_class(k)];
         }
-        store_base[NQCLASS] = off;
-        const long long keys = (long long)npair * (npair + 1) / 2;
-        d_store.ensure(sizeof(double) * std::max<long long>(off, 1));
-        d_qmap.ensure(sizeof(int) * std::max<long long>(keys, 1));
-        d_lerr.ensure(sizeof(int));
-        // the integrals run on the library streams while the caller's stream builds
-        // the gather lists (they need only the pair-pair map); joined before the copies
-        fan.fork(st);
-        {
-            aimdhf::StoreArgs sa;
-            sa.recs = d_recs.as<double>();
-            sa.rec_off = d_rec_off.as<long long>();
-            sa.npp = d_npp.as<int>();
-            sa.boys = d_boys.as<double>();
-            for (int k = 0, i = 0; k < NQCLASS; ++k) {
-                if (!qcount[k]) continue;
-                sa.store = d_store.as<double>() + store_base[k];
-                hipStream_t s2 = fan.on(1 + i++ % Fan::NAUX);
-                prof.time(47, s2, [&] { aimdhf::launch_eri_store(k, sa, list_of_class(k), qcount[k], q64count[k], s2); });
-            }
-        }
-        {
-            // partner and ket lists on the host while the integrals run
-            auto t0 = Profiler::clock::now();
-            build_owner_lists(threshold, false, st);
-            prof.host(86, t0);
-        }
-        prof.time(48, st, [&] {
-            aimdhf::launch_fill_int(d_qmap.as<int>(), (size_t)keys, -1, st);
-            aimdhf::launch_fill_int(d_lerr.as<int>(), 1, 0, st);
-            aimdhf::QmapArgs qa;
-            qa.list = d_list.as<int2>();
-            qa.qoff[0] = 0;
-            for (int k = 0; k < NQCLASS; ++k) qa.qoff[k + 1] = qa.qoff[k] + qcount[k];
-            qa.qmap = d_qmap.as<int>();
-            aimdhf::launch_qmap(qa, st);
-        });
-        HIPCHECK(hipGetLastError());
-        aimdhf::ListArgs la;
+        runbase[NQCLASS] = runs;
+        const long long cells = runs * aimdhf::LIST_WAVES;
+        d_lcnt.ensure(sizeof(long long) * cells);
+        d_loff.ensure(sizeof(long long) * (cells + 1));
+        d_lsum.ensure(sizeof(long long) * (aimdhf::list_scan_blocks(cells) + 64));
+        long long* picked = d_lsum.as<long long>() + aimdhf::list_scan_blocks(cells);
+        aimdhf::QListArgs la;
         la.npair = npair;
-        la.thr = threshold;
-        // mixed precision: bands two decades apart from the FP64 / FP32 switch down, the
-        // first held in FP64; FP64: one band (finer units only slow the complete builds)
-        const bool split = precision == 1 && jk_switch > threshold;
-        const int nbig = split ? 1 : aimdhf::NBAND;   // leading bands held in FP64
-        for (int b = 0; b < aimdhf::NBAND - 1; ++b)
-            la.band_lo[b] = split ? std::max(jk_switch * std::pow(1e-2, b), threshold) : threshold;
-        la.band_lo[aimdhf::NBAND - 1] = threshold;
-        la.out_x = d_out_x.as<int>();
-        la.out_y = d_out_y.as<int>();
-        la.shell_l = d_shell_l.as<int>();
-        la.shell_ao = d_shell_ao.as<int>();
-        la.pair_a = d_pair_a.as<int>();
-        la.pair_b = d_pair_b.as<int>();
-        la.pair_cls = d_pair_cls.as<int>();
-        la.part_off = d_part_off.as<int>();
-        la.part_shell = d_part_shell.as<int>();
-        la.part_pair = d_part_pair.as<int>();
-        la.part_q = d_part_q.as<double>();
-        la.qscr = d_qscr.as<double>();
-        la.ket_pair = d_ket_pair.as<int>();
-        la.ket_q = d_ket_q.as<double>();
-        for (int c = 0; c < 7; ++c) la.ket_off[c] = ket_off[c];
-        la.qmap = d_qmap.as<int>();
-        for (int k = 0; k < NQCLASS; ++k) la.qcount[k] = qcount[k];
-        la.err = d_lerr.as<int>();
-        const int nout = out_off[9];
-        constexpr int NB = aimdhf::NBAND;
-        const long long nks = (long long)nout * 9, njs = (long long)npair * 6;
-        if (nks * NB + 1 > aimdhf::scan_max_items() || njs * NB + 1 > aimdhf::scan_max_items()) {
-            g_err = "integral store: too many gather segments for the table scans";
-            throw HipError{AIMDHF_E_UNSUPPORTED};
+        la.nrep = nrep;
+        la.nparts = list_parts;
+        la.thr = thr;
+        la.sw = sw;
+        for (int c = 0; c < 7; ++c) la.cls_off[c] = cls_pair_off[c];
+        for (int k = 0; k < NQCLASS; ++k) la.runbase[k] = runbase[k];
+        la.seg = d_seg.as<int>();
+        la.rank_rep = batched ? d_rank_rep.as<int>() : nullptr;
+        la.rq = d_rq.as<double>();
+        la.cnt = d_lcnt.as<long long>();
+        la.off = d_loff.as<long long>();
+        la.lbra = la.lket = nullptr;
+        aimdhf::launch_qlist_count(la, st);
+        aimdhf::launch_list_scan(la.cnt, d_loff.as<long long>(), cells, d_lsum.as<long long>(), st);
+        aimdhf::PickArgs pk;
+        pk.n = 0;
+        for (int k = 0; k < NQCLASS; ++k) {
+            pk.at[pk.n++] = runbase[k] * aimdhf::LIST_WAVES;
+            pk.at[pk.n++] = (runbase[k] + ncls[bra_class(k)]) * aimdhf::LIST_WAVES;
         }
-        // device tables: per-band counts -> sizes -> scans -> units; only totals come back
-        d_kcnt.ensure(sizeof(long long) * (NB + 1) * std::max<long long>(nks, 1));   // bands, then totals
-        d_jcnt.ensure(sizeof(long long) * (NB + 1) * std::max<long long>(njs, 1));
-        d_kseg.ensure(sizeof(long long) * (nks + 1));
-        d_jseg.ensure(sizeof(long long) * (njs + 1));
-        d_kdoff.ensure(sizeof(long long) * (nks + 1));
-        d_kdoff32.ensure(sizeof(long long) * (nks + 1));
-        d_jdoff.ensure(sizeof(long long) * (njs + 1));
-        d_jdoff32.ensure(sizeof(long long) * (njs + 1));
-        d_kbig.ensure(sizeof(long long) * std::max<long long>(nks, 1));
-        d_jbig.ensure(sizeof(long long) * std::max<long long>(njs, 1));
-        const long long nku_slots = nks * NB + 1, nju_slots = njs * NB + 1;
-        const long long nbsum = (std::max(nku_slots, nju_slots) + 4095) / 4096 + 1;
-        const long long tab_n = 3 * nks + (nks * NB) + nku_slots + 3 * njs + (njs * NB) + nju_slots + nbsum + 32;
-        d_tab.ensure(sizeof(long long) * tab_n);
-        d_out_unit.ensure(sizeof(int) * (nout + 1));
-        d_pair_unit.ensure(sizeof(int) * (npair + 1));
-        aimdhf::TabArgs ta;
-        ta.nout = nout;
-        ta.npair = npair;
-        ta.nbig = nbig;
-        ta.unit_items = unit_items;
-        for (int t = 0; t < 10; ++t) ta.out_off[t] = out_off[t];
-        for (int c = 0; c < 7; ++c) ta.cls_pair_off[c] = cls_pair_off[c];
-        ta.out_x = d_out_x.as<int>();
-        ta.out_y = d_out_y.as<int>();
-        ta.shell_l = d_shell_l.as<int>();
-        ta.pair_cls = d_pair_cls.as<int>();
-        ta.cls_pairs = d_cls_pairs.as<int>();
-        ta.kband = d_kcnt.as<long long>();
-        ta.jband = d_jcnt.as<long long>();
-        long long* tp = d_tab.as<long long>();
-        auto take = [&](long long n) { long long* r = tp; tp += n; return r; };
-        ta.kcount = take(nks);
-        ta.ksz64 = take(nks);
-        ta.ksz32 = take(nks);
-        ta.knu = take(nks * NB);
-        ta.kustart = take(nku_slots);
-        ta.jcount = take(njs);
-        ta.jsz64 = take(njs);
-        ta.jsz32 = take(njs);
-        ta.jnu = take(njs * NB);
-        ta.justart = take(nju_slots);
-        long long* bsum = take(nbsum);
-        long long* tot = take(32);      // totals and check flag of launch_tab_totals
-        ta.kbig = d_kbig.as<long long>();
-        ta.jbig = d_jbig.as<long long>();
-        ta.kseg = d_kseg.as<long long>();
-        ta.kdoff = d_kdoff.as<long long>();
-        ta.kdoff32 = d_kdoff32.as<long long>();
-        ta.jseg = d_jseg.as<long long>();
-        ta.jdoff = d_jdoff.as<long long>();
-        ta.jdoff32 = d_jdoff32.as<long long>();
-        ta.out_unit = d_out_unit.as<int>();
-        ta.pair_unit = d_pair_unit.as<int>();
-        ta.kunit_os = nullptr;
-        ta.kunit_e = nullptr;
-        ta.junit_pc = nullptr;
-        ta.junit_e = nullptr;
-        la.kband = d_kcnt.as<long long>();
-        if (!h_pin) HIPCHECK(hipHostMalloc((void**)&h_pin, sizeof(long long) * 64));
-        auto th = Profiler::clock::now();
-        prof.time(48, st, [&] {
-            aimdhf::launch_klist_count(la, nout, d_kcnt.as<long long>() + NB * nks, d_kcnt.as<long long>(), st);
-            aimdhf::launch_jlist_count(la, d_jcnt.as<long long>() + NB * njs, d_jcnt.as<long long>(), st);
-            aimdhf::launch_seg_sizes(ta, st);
-            aimdhf::launch_scan(ta.kcount, ta.kseg, nks, bsum, st);
-            aimdhf::launch_scan(ta.ksz64, ta.kdoff, nks, bsum, st);
-            aimdhf::launch_scan(ta.ksz32, ta.kdoff32, nks, bsum, st);
-            aimdhf::launch_scan(ta.knu, ta.kustart, nks * NB, bsum, st);
-            aimdhf::launch_scan(ta.jcount, ta.jseg, njs, bsum, st);
-            aimdhf::launch_scan(ta.jsz64, ta.jdoff, njs, bsum, st);
-            aimdhf::launch_scan(ta.jsz32, ta.jdoff32, njs, bsum, st);
-            aimdhf::launch_scan(ta.jnu, ta.justart, njs * NB, bsum, st);
-            aimdhf::launch_tab_totals(ta, tot, st);
-        });
+        pk.at[pk.n++] = cells;
+        aimdhf::launch_pick(pk, d_loff.as<long long>(), picked, st);
         HIPCHECK(hipGetLastError());
-        HIPCHECK(hipMemcpyAsync(h_pin, tot, sizeof(long long) * 26, hipMemcpyDeviceToHost, st));
+        HIPCHECK(hipMemcpyAsync(h_pin, picked, sizeof(long long) * pk.n, hipMemcpyDeviceToHost, st));
         HIPCHECK(hipStreamSynchronize(st));
-        if (h_pin[25]) {
-            g_err = "integral store: inconsistent gather-segment tables";
-            throw HipError{AIMDHF_E_STATE};
+        qcount.assign(NQCLASS, 0);
+        q64count.assign(NQCLASS, 0);
+        for (int k = 0; k < NQCLASS; ++k) {
+            list_off[k] = h_pin[2 * k];
+            q64count[k] = h_pin[2 * k + 1] - h_pin[2 * k];
+            qcount[k] = h_pin[2 * k + 2] - h_pin[2 * k];
         }
-        prof.host(89, th);
-        th = Profiler::clock::now();
-        k_entries = h_pin[0];
-        j_entries = h_pin[1];
-        const long long ko = h_pin[2], ko32 = h_pin[3], jo = h_pin[4], jo32 = h_pin[5];
-        const long long nku = h_pin[6], nju = h_pin[7];
-        for (int t = 0; t < 10; ++t) kunit_base[t] = (int)h_pin[8 + t];
-        for (int c = 0; c < 7; ++c) junit_base[c] = (int)h_pin[18 + c];
-        kdata_total = ko;
-        jdata_total = jo;
-        kdata32_total = ko32;
-        jdata32_total = jo32;
-        d_klist.ensure(sizeof(long long) * std::max<long long>(k_entries, 1));
-        d_jlist.ensure(sizeof(long long) * std::max<long long>(j_entries, 1));
-        d_kunit_os.ensure(sizeof(int) * std::max<long long>(nku, 1));
-        d_kunit_e.ensure(sizeof(long long) * 2 * std::max<long long>(nku, 1));
-        d_junit_pc.ensure(sizeof(int) * std::max<long long>(nju, 1));
-        d_junit_e.ensure(sizeof(long long) * 2 * std::max<long long>(nju, 1));
-        d_kpart2.ensure(sizeof(double) * 2 * 36 * std::max<long long>(nku, 1));
-        d_jpart2.ensure(sizeof(double) * 2 * 36 * std::max<long long>(nju, 1));
-        d_kdata.ensure(sizeof(double) * std::max<long long>(ko, 1));
-        d_jdata.ensure(sizeof(double) * std::max<long long>(jo, 1));
-        have_32b = precision == 1;
-        if (have_32b) {
-            d_kdata32b.ensure(sizeof(float) * std::max<long long>(ko, 1));
-            d_jdata32b.ensure(sizeof(float) * std::max<long long>(jo, 1));
-        }
-        d_kdata32.ensure(sizeof(float) * std::max<long long>(ko32, 1));
-        d_jdata32.ensure(sizeof(float) * std::max<long long>(jo32, 1));
-        ta.kunit_os = d_kunit_os.as<int>();
-        ta.kunit_e = d_kunit_e.as<long long>();
-        ta.junit_pc = d_junit_pc.as<int>();
-        ta.junit_e = d_junit_e.as<long long>();
-        la.kseg = d_kseg.as<long long>();
-        la.klist = d_klist.as<long long>();
-        la.jseg = d_jseg.as<long long>();
-        la.jlist = d_jlist.as<long long>();
-        prof.host(90, th);
-        th = Profiler::clock::now();
-        prof.time(48, st, [&] {
-            aimdhf::launch_klist_fill(la, nout, st);
-            aimdhf::launch_jlist_fill(la, st);
-            aimdhf::launch_units(ta, st);
-        });
+        qtotal = list_off[NQCLASS] = h_pin[2 * NQCLASS];
+        d_lbra.ensure(sizeof(int) * std::max<long long>(qtotal, 1));
+        d_lket.ensure(sizeof(int) * std::max<long long>(qtotal, 1));
+        la.lbra = d_lbra.as<int>();
+        la.lket = d_lket.as<int>();
+        if (qtotal) aimdhf::launch_qlist_fill(la, st);
         HIPCHECK(hipGetLastError());
-        HIPCHECK(hipMemcpyAsync(h_pin + 32, d_lerr.p, sizeof(int), hipMemcpyDeviceToHost, st));
-        HIPCHECK(hipStreamSynchronize(st));
-        if (*(const int*)(h_pin + 32)) {
-            g_err = "integral store: a gather-list quartet is missing from the screened list";
-            throw HipError{AIMDHF_E_STATE};
+        // the store's layout: per class its FP64 blocks, then its FP32 blocks, in tiles of 64 quartets
+        size_t b = 0;
+        for (int k = 0; k < NQCLASS; ++k) {
+            const size_t blk = (size_t)aimdhf::store_block(k);
+            base64[k] = (long long)b;
+            b += sizeof(double) * ((q64count[k] + 63) / 64 * 64) * blk;
+            base32[k] = (long long)b;
+            b += sizeof(float) * ((qcount[k] - q64count[k] + 63) / 64 * 64) * blk;
         }
-        prof.host(91, th);
-        th = Profiler::clock::now();
-        prof.host(92, th);
-        fan.join();
-        prof.time(15, st, [&] {
-            fan.fork(st);
-            int i = 0;
-            aimdhf::KSArgs ka = ks_args(1, nullptr, nullptr);
-            for (int t = 0; t < 9; ++t) {
-                const int no = out_off[t + 1] - out_off[t];
-                if (no > 0) aimdhf::launch_kcopy(t, ka, no, fan.on(i++));
-            }
-            aimdhf::JSArgs ja = js_args(1, nullptr, nullptr);
-            for (int c = 0; c < 6; ++c) {
-                if (!ncls[c]) continue;
-                ja.cls_off = cls_pair_off[c];
-                aimdhf::launch_jcopy(c, ja, ncls[c], fan.on(i++));
-            }
-            fan.join();
-        });
-        HIPCHECK(hipGetLastError());
-        have_unit_q = false;   // unit bounds: on the first density-difference build
-        store_bytes = 8 * (off + ko + jo) + 4 * (ko32 + jo32) + (have_32b ? 4 * (ko + jo) : 0) + 4 * keys +
-                      8 * (k_entries + j_entries + 4 * nks + 4 * njs);
+        store_need = b;
     }
 
-    // Largest Schwarz product of every work unit of the integral store, which
-    // density-difference builds screen with; computed once per store, on the first
-    // such build (stream-ordered, no synchronisation).
-    bool have_unit_q = false;
-    void ensure_unit_q(hipStream_t st) {
-        if (have_unit_q) return;
-        const int nku = kunit_base[9], nju = junit_base[6];
-        d_kunit_q.ensure(sizeof(double) * std::max(nku, 1));
-        d_junit_q.ensure(sizeof(double) * std::max(nju, 1));
-        d_dmax.ensure(sizeof(double));
-        aimdhf::UnitQArgs ua;
-        ua.list = d_list.as<int2>();
-        long long qo = 0;
-        for (int k = 0; k < NQCLASS; ++k) {
-            ua.qoff[k] = qo;
-            qo += qcount[k];
+    static int bra_class(int k) {
+        int hi = 0;
+        while ((hi + 1) * (hi + 2) / 2 <= k) ++hi;
+        return hi;
+    }
+    static int ket_class(int k) { return k - bra_class(k) * (bra_class(k) + 1) / 2; }
+
+    // Evaluate the screened quartets into the store.
+    void build_store(hipStream_t st) {
+        d_store.ensure(std::max<size_t>(store_need, 1));
+        aimdhf::EriArgs ea;
+        ea.recs = d_recs.as<double>();
+        ea.rec_off = d_rec_off.as<long long>();
+        ea.npp = d_npp.as<int>();
+        ea.cls_pairs = d_cls_pairs.as<int>();
+        ea.boys = d_boys.as<double>();
+        fan.fork(st);
+        for (int k = 0, i = 0; k < NQCLASS; ++k) {
+            if (!qcount[k]) continue;
+            ea.lbra = d_lbra.as<int>() + list_off[k];
+            ea.lket = d_lket.as<int>() + list_off[k];
+            ea.out64 = (double*)(d_store.as<char>() + base64[k]);
+            ea.out32 = (float*)(d_store.as<char>() + base32[k]);
+            hipStream_t s2 = fan.on(i++);
+            prof.time(47, s2, [&] { aimdhf::launch_eri(k, ea, q64count[k], qcount[k] - q64count[k], s2); });
         }
-        ua.qscr = d_qscr.as<double>();
-        ua.shell_l = d_shell_l.as<int>();
-        ua.out_x = d_out_x.as<int>();
-        ua.out_y = d_out_y.as<int>();
-        ua.pair_cls = d_pair_cls.as<int>();
-        ua.klist = d_klist.as<long long>();
-        ua.kunit_os = d_kunit_os.as<int>();
-        ua.kunit_e = d_kunit_e.as<long long>();
-        ua.nkunit = nku;
-        ua.kunit_q = d_kunit_q.as<double>();
-        ua.jlist = d_jlist.as<long long>();
-        ua.junit_pc = d_junit_pc.as<int>();
-        ua.junit_e = d_junit_e.as<long long>();
-        ua.njunit = nju;
-        ua.junit_q = d_junit_q.as<double>();
-        prof.time(48, st, [&] { aimdhf::launch_unit_q(ua, st); });
+        fan.join();
         HIPCHECK(hipGetLastError());
-        have_unit_q = true;
+        // the digestion's view of the store (the stream was synchronised when the list was
+        // built: no earlier copy from this pinned block is pending)
+        aimdhf::DigestGeo* geo = (aimdhf::DigestGeo*)(h_pin + 64);
+        for (int k = 0; k < NQCLASS; ++k) {
+            geo[k].t64 = list_off[k];
+            geo[k].t32 = list_off[k] + q64count[k];
+            geo[k].off = d_loff.as<long long>() + runbase[k] * aimdhf::LIST_WAVES;
+            geo[k].lket = d_lket.as<int>();
+            geo[k].s64 = (const double*)(d_store.as<char>() + base64[k]);
+            geo[k].s32 = (const float*)(d_store.as<char>() + base32[k]);
+        }
+        d_geo.ensure(sizeof(aimdhf::DigestGeo) * NQCLASS);
+        HIPCHECK(hipMemcpyAsync(d_geo.p, geo, sizeof(aimdhf::DigestGeo) * NQCLASS, hipMemcpyHostToDevice, st));
+        store_bytes = (long long)store_need + 8 * qtotal;
+        ensure_digest(1);
+    }
+
+    // copies of the global J/K accumulators: one per XCD where the matrices are few
+    int digest_copies() const { return batched ? 1 : 8; }
+
+    // one launch for all classes where the runs are short (see jk_digest_all.hip)
+    bool digest_in_one(int nset) const {
+        return (batched || (long long)nset * nao * nao <= SMALL_JK) && aimdhf::digest_all_fits(matrix_ld(), lds_limit);
+    }
+
+    void ensure_digest(int nset) {
+        const size_t mats = mat_elems() * nset, c = digest_copies();
+        d_dsym.ensure(sizeof(double) * mats);
+        d_dket.ensure(sizeof(double) * std::max<long long>(npao * nset, 1));
+        d_kacc.ensure(sizeof(long long) * mats * c);
+        d_jacc.ensure(sizeof(long long) * std::max<long long>(npao * nset, 1) * c);
+        d_dcell.ensure(sizeof(long long) * aimdhf::JK_CELLS * nrep * nset);
+    }
+
+    aimdhf::PrepArgs prep_args(int nset, const double* dens, double* J, double* K) const {
+        aimdhf::PrepArgs a;
+        a.ld = matrix_ld();
+        a.nset = nset;
+        a.nrep = nrep;
+        a.ncopy = digest_copies();
+        a.npair = npair;
+        for (int c = 0; c < 7; ++c) {
+            a.cls_off[c] = cls_pair_off[c];
+            a.koff[c] = koff[c];
+        }
+        a.npao = npao;
+        a.kstride = (long long)(mat_elems() * nset);
+        a.oab = d_oab.as<int>();
+        a.rank_rep = batched ? d_rank_rep.as<int>() : nullptr;
+        a.rep_nao = batched ? d_rep_nao.as<int>() : nullptr;
+        a.dens = dens;
+        a.dsym = d_dsym.as<double>();
+        a.dket = d_dket.as<double>();
+        a.kacc = d_kacc.as<unsigned long long>();
+        a.jacc = d_jacc.as<unsigned long long>();
+        a.dcell = d_dcell.as<unsigned long long>();
+        a.gcell = d_gcell.as<unsigned long long>();
+        a.J = J;
+        a.K = K;
+        a.rq = d_rq.as<double>();
+        return a;
+    }
+
+    // class k, or every class (k < 0) for launch_digest_all
+    aimdhf::DigestArgs digest_args(int k, int nset, bool delta, double dthr) const {
+        aimdhf::DigestArgs a;
+        a.geo = d_geo.as<aimdhf::DigestGeo>();
+        const int nk = k < 0 ? 0 : ncls[ket_class(k)];
+        a.ld = matrix_ld();
+        a.nset = nset;
+        a.ncopy = digest_copies();
+        a.lds_limit = lds_limit;
+        a.nparts = list_parts;
+        a.unit = unit_items;
+        a.nchunk = batched ? 1 : (int)std::min<long long>(16, std::max<long long>(1, nk / (8LL * unit_items)));
+        a.oab = d_oab.as<int>();
+        a.rank_rep = batched ? d_rank_rep.as<int>() : nullptr;
+        a.dsym = d_dsym.as<double>();
+        a.dket = d_dket.as<double>();
+        a.npao = npao;
+        for (int c = 0; c < 7; ++c) {
+            a.cls_off[c] = cls_pair_off[c];
+            a.koff[c] = koff[c];
+        }
+        a.kacc = d_kacc.as<unsigned long long>();
+        a.jacc = d_jacc.as<unsigned long long>();
+        a.kstride = (long long)(mat_elems() * nset);
+        a.dcell = d_dcell.as<unsigned long long>();
+        a.gcell = d_gcell.as<unsigned long long>();
+        a.rep_nao = batched ? d_rep_nao.as<int>() : nullptr;
+        a.delta = delta ? 1 : 0;
+        a.dthr = dthr;
+        a.rq = d_rq.as<double>();
+        return a;
     }
 
     aimdhf::OneElArgs oneel_args() const {
@@ -947,64 +780,6 @@ struct aimdhf_plan {
         return g;
     }
 
-    aimdhf::BatchArgs batch_args() const {
-        aimdhf::BatchArgs b;
-        b.nrep = nrep;
-        b.ld = bld;
-        b.rep_nao = d_rep_nao.as<int>();
-        b.rep_toff = d_rep_toff.as<long long>();
-        b.rep_item = d_rep_item.as<long long>();
-        b.shell_rep = d_shell_rep.as<int>();
-        b.shell_ao = d_shell_ao.as<int>();
-        b.shell_l = d_shell_l.as<int>();
-        b.pair_a = d_pair_a.as<int>();
-        b.pair_b = d_pair_b.as<int>();
-        b.list = d_list.as<int2>();
-        b.qoff[0] = 0;
-        for (int k = 0; k < NQCLASS; ++k) {
-            b.qoff[k + 1] = b.qoff[k] + qcount[k];
-            b.store_base[k] = store_base[k];
-            b.blk[k] = (int)aimdhf::store_block(k);
-            int hi = 0;
-            while ((hi + 1) * (hi + 2) / 2 <= k) ++hi;
-            const int lo = k - hi * (hi + 1) / 2, lc = lo == 0 ? 0 : lo <= 2 ? 1 : 2, ld_ = lo - lc * (lc + 1) / 2;
-            b.ncd[k] = ncart(lc) * ncart(ld_);
-        }
-        b.store_base[NQCLASS] = store_base[NQCLASS];
-        b.store = d_store.as<double>();
-        b.tens = d_tens.as<double>();
-        return b;
-    }
-
-    // Batch geometry: every screened quartet of every replica into the store (one
-    // launch per class, FP64), then into the replicas' dense tensors
-    void build_batch_tensors(hipStream_t st) {
-        long long off = 0;
-        for (int k = 0; k < NQCLASS; ++k) {
-            store_base[k] = off;
-            off += qcount[k] * aimdhf::store_block(k);
-        }
-        store_base[NQCLASS] = off;
-        d_store.ensure(sizeof(double) * std::max<long long>(off, 1));
-        d_tens.ensure(sizeof(double) * std::max<long long>(tens_total, 1));
-        aimdhf::StoreArgs sa;
-        sa.recs = d_recs.as<double>();
-        sa.rec_off = d_rec_off.as<long long>();
-        sa.npp = d_npp.as<int>();
-        sa.boys = d_boys.as<double>();
-        prof.time(47, st, [&] {
-            for (int k = 0; k < NQCLASS; ++k) {
-                if (!qcount[k]) continue;
-                sa.store = d_store.as<double>() + store_base[k];
-                aimdhf::launch_eri_store(k, sa, list_of_class(k), qcount[k], q64count[k], st);
-            }
-        });
-        prof.time(15, st, [&] {
-            aimdhf::launch_zero_d(d_tens.as<double>(), (size_t)tens_total, st);
-            aimdhf::launch_batch_scatter(batch_args(), off, st);
-        });
-        HIPCHECK(hipGetLastError());
-    }
 };
 
 static int pair_class(int la, int lb) { return la * (la + 1) / 2 + lb; }
@@ -1144,14 +919,10 @@ static int create_plan(int natm, int nshell, const int64_t* shell_atom, const in
             for (int sh = 0; sh < nshell; ++sh) local[sh] = p->shell_ao[sh] - p->shell_ao[p->shell_first[sh]];
             local[nshell] = 0;
             p->shell_ao = local;
-            p->rep_toff.assign(p->nrep + 1, 0);
-            p->rep_item.assign(p->nrep + 1, 0);
             for (int r = 0; r < p->nrep; ++r) {
                 const long long n = p->rep_nao[r];
-                p->rep_toff[r + 1] = p->rep_toff[r] + n * n * n * n;
-                p->rep_item[r + 1] = p->rep_item[r] + n * n;
+                p->tens_total += n * n * n * n;
             }
-            p->tens_total = p->rep_toff[p->nrep];
         }
         p->nblock = p->shell_block[nshell - 1] + 1;
         p->prim_exp.assign(prim_exp, prim_exp + nprim);
@@ -1206,12 +977,70 @@ static int create_plan(int natm, int nshell, const int64_t* shell_atom, const in
             }
         p->rec_off[p->npair] = off;
         p->rec_total = off;
+        // rank order of the pairs (jk_digest.h): per class, replica by replica, the most
+        // contracted first, then along the diagonals of the pair triangle
+        {
+            std::vector<int> first(p->npair), second(p->npair);
+            for (int r = 0, Q = 0; r < p->nrep; ++r)
+                for (int s1 = p->rep_shell[r]; s1 < p->rep_shell[r + 1]; ++s1)
+                    for (int s2 = p->rep_shell[r]; s2 <= s1; ++s2, ++Q) {
+                        first[Q] = s1;
+                        second[Q] = s2;
+                    }
+            auto nprim_of = [&](int sh) { return (int)(shell_prim[sh + 1] - shell_prim[sh]); };
+            for (auto& v : bylcls)
+                std::stable_sort(v.begin(), v.end(), [&](int x, int y) {
+                    const int rx = p->shell_rep[first[x]], ry = p->shell_rep[first[y]];
+                    if (rx != ry) return rx < ry;
+                    const int cx = nprim_of(first[x]) * nprim_of(second[x]), cy = nprim_of(first[y]) * nprim_of(second[y]);
+                    if (cx != cy) return cx > cy;
+                    const int dx = p->pair_a[x] - p->pair_b[x], dy = p->pair_a[y] - p->pair_b[y];
+                    return dx != dy ? dx < dy : first[x] < first[y];
+                });
+        }
         p->cls_pair_off.assign(7, 0);
         p->ncls.assign(6, 0);
         for (int c = 0; c < 6; ++c) {
             p->cls_pair_off[c + 1] = p->cls_pair_off[c] + (int)bylcls[c].size();
             p->ncls[c] = (int)bylcls[c].size();
             p->cls_pairs.insert(p->cls_pairs.end(), bylcls[c].begin(), bylcls[c].end());
+        }
+        // AO offsets and replica of every rank, rank range of every (class, replica), and
+        // the base of every class's components
+        std::vector<int> oab(p->npair), rank_rep(p->npair), seg(6 * p->nrep + 1, p->npair);
+        for (int r = p->npair - 1; r >= 0; --r) {
+            const int Q = p->cls_pairs[r], a = p->pair_a[Q], b = p->pair_b[Q];
+            oab[r] = (p->shell_ao[a] & aimdhf::OAB_MASK) | (p->shell_ao[b] & aimdhf::OAB_MASK) << 14 |
+                     (a == b ? aimdhf::OAB_SAME : 0);
+            rank_rep[r] = p->shell_rep[a];
+            seg[p->pair_cls[Q] * p->nrep + rank_rep[r]] = r;
+        }
+        // segments without pairs start where the next one does
+        for (int i = 6 * p->nrep - 1; i >= 0; --i) {
+            const int c = i / p->nrep;
+            const bool any = seg[i] < p->npair && p->pair_cls[p->cls_pairs[seg[i]]] == c &&
+                             rank_rep[seg[i]] == i % p->nrep;
+            if (!any) seg[i] = seg[i + 1];
+        }
+        p->koff[0] = 0;
+        for (int c = 0; c < 6; ++c) {
+            const int la = c == 0 ? 0 : c <= 2 ? 1 : 2, lb = c - la * (la + 1) / 2;
+            p->koff[c + 1] = p->koff[c] + (long long)p->ncls[c] * ncart(la) * ncart(lb);
+        }
+        p->npao = p->koff[6];
+        upload(p->d_oab, oab);
+        upload(p->d_seg, seg);
+        if (p->batched) {
+            upload(p->d_rank_rep, rank_rep);
+            upload(p->d_rep_shell, p->rep_shell);
+        }
+        p->d_rq.ensure(sizeof(double) * p->npair);
+        p->d_gcell.ensure(sizeof(long long) * 3 * p->nrep);
+        {
+            int dev = 0, lim = 0;
+            HIPCHECK(hipGetDevice(&dev));
+            HIPCHECK(hipDeviceGetAttribute(&lim, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+            p->lds_limit = std::max(lim, 65536);
         }
         p->bp_off.assign(p->nbpair + 1, 0);
         for (int i = 0; i < p->nbpair; ++i) {
@@ -1267,8 +1096,6 @@ static int create_plan(int natm, int nshell, const int64_t* shell_atom, const in
             upload(p->d_pair_lo, p->pair_lo);
             upload(p->d_rep_atom, p->rep_atom);
             upload(p->d_rep_nao, p->rep_nao);
-            upload(p->d_rep_toff, p->rep_toff);
-            upload(p->d_rep_item, p->rep_item);
         }
         p->d_scratch.ensure(sizeof(double) * 1024);
         p->d_pos.ensure(sizeof(double) * 3 * natm);
@@ -1330,7 +1157,7 @@ static int set_geometry_generic(aimdhf_plan* p, const double* positions, double 
         p->qtotal = p->gen_build_list(thr, p->d_list);
         p->threshold = thr;
         p->stored = false;
-        p->store_bytes = p->k_entries = p->j_entries = 0;
+        p->store_bytes = 0;
         p->prof.host(85, t0);
         p->have_geometry = true;
     } catch (const HipError& e) {
@@ -1467,17 +1294,14 @@ int aimdhf_set_geometry(aimdhf_plan* p, const double* positions, double thr, voi
         });
         HIPCHECK(hipGetLastError());
         auto t0 = Profiler::clock::now();
-        p->build_list(thr, p->precision == 1 && p->jk_switch > thr ? p->jk_switch : 0.0, p->d_list, p->qcount,
-                      p->q64count, st);
-        p->qtotal = 0;
-        for (long long c : p->qcount) p->qtotal += c;
+        p->build_quartets(thr, p->precision == 1 && p->jk_switch > thr ? p->jk_switch : 0.0, st);
         p->threshold = thr;
         p->prof.host(85, t0);
         p->stored = false;
-        p->store_bytes = p->k_entries = p->j_entries = 0;
+        p->store_bytes = 0;
         if (p->batched) {
             auto t1 = Profiler::clock::now();
-            p->build_batch_tensors(st);
+            p->build_store(st);
             p->prof.host(87, t1);
             p->have_geometry = true;
             return AIMDHF_OK;
@@ -1490,7 +1314,7 @@ int aimdhf_set_geometry(aimdhf_plan* p, const double* positions, double thr, voi
                 HIPCHECK(hipMemGetInfo(&fr, &tot));
                 limit = (long long)(fr / 2);
             }
-            store = p->jk_mode == 2 || p->store_estimate() <= limit;
+            store = p->jk_mode == 2 || (long long)p->store_need <= limit;
         }
         if (!store) {
             t0 = Profiler::clock::now();
@@ -1537,7 +1361,14 @@ int aimdhf_quartets(aimdhf_plan* p, int64_t* out, int64_t cap, int64_t* count) {
     try {
         long long n = std::min<long long>(cap, p->qtotal);
         std::vector<int2> tmp(n);
-        if (n) HIPCHECK(hipMemcpy(tmp.data(), p->d_list.p, sizeof(int2) * n, hipMemcpyDeviceToHost));
+        if (p->generic) {
+            if (n) HIPCHECK(hipMemcpy(tmp.data(), p->d_list.p, sizeof(int2) * n, hipMemcpyDeviceToHost));
+        } else if (n) {
+            std::vector<int> b(n), k(n);
+            HIPCHECK(hipMemcpy(b.data(), p->d_lbra.p, sizeof(int) * n, hipMemcpyDeviceToHost));
+            HIPCHECK(hipMemcpy(k.data(), p->d_lket.p, sizeof(int) * n, hipMemcpyDeviceToHost));
+            for (long long i = 0; i < n; ++i) tmp[i] = make_int2(p->cls_pairs[b[i]], p->cls_pairs[k[i]]);
+        }
         for (long long i = 0; i < n; ++i) {
             int a = tmp[i].x, b = tmp[i].y;
             out[2 * i] = std::max(a, b);
@@ -1588,44 +1419,36 @@ int aimdhf_grad_quartets(aimdhf_plan* p, int64_t* out, int64_t cap, int64_t* cou
     return AIMDHF_OK;
 }
 
-// J and K from the integral store; delta: dens is a density difference and
-// units below dthr (largest Schwarz product times max |dens|) are skipped
+// J and K from the integral store (one molecule, or every replica of a batch);
+// delta: dens is a density difference and quartets below dthr may be skipped
 static int jk_from_store(aimdhf_plan* p, int nset, const double* dens, double* J, double* K, bool delta, double dthr,
                          hipStream_t st) {
     try {
-        const size_t nn = (size_t)p->nao * p->nao;
-        p->d_dsym.ensure(sizeof(double) * nset * nn);
-        if (delta) p->ensure_unit_q(st);
-        p->prof.time(45, st, [&] {
-            aimdhf::launch_symmetrize(dens, nset, p->nao, p->d_dsym.as<double>(), st);
-            if (delta) aimdhf::launch_absmax(p->d_dsym.as<double>(), nset * nn, p->d_dmax.as<double>(), st);
-        });
-        // the 15 J and K launches are independent (disjoint outputs): spread over the fan's streams
-        p->fan.fork(st);
-        int i = 0;
-        aimdhf::KSArgs ka = p->ks_args(nset, p->d_dsym.as<double>(), K);
-        aimdhf::JSArgs ja = p->js_args(nset, p->d_dsym.as<double>(), J);
-        ka.delta = ja.delta = delta ? 1 : 0;
-        ka.dthr = ja.dthr = dthr;
-        ka.d32 = ja.d32 = p->delta_fp32_max;
-        p->last_ka = ka;
-        p->last_ja = ja;
+        p->ensure_digest(nset);
+        const aimdhf::PrepArgs pa = p->prep_args(nset, dens, J, K);
+        p->prof.time(45, st, [&] { aimdhf::launch_jk_prep(pa, st); });
+        // the classes add to the same accumulators in any order
+        const int threads = p->batched ? 4 * p->batch_jk_lanes : 256;
+        if (p->digest_in_one(nset)) {
+            const aimdhf::DigestArgs da = p->digest_args(-1, nset, delta, dthr);
+            for (int k = 0; k < NQCLASS; ++k) p->last_dig[k] = p->digest_args(k, nset, delta, dthr);
+            p->prof.time(94, st, [&] { aimdhf::launch_digest_all(da, threads, st); });
+        } else {
+            // spread over the fan's streams; a batch's launches stay on the caller's stream, which
+            // may be capturing (its graph outlives calls and must not depend on the plan's
+            // streams), and cover every class, as the graph is replayed at other geometries
+            if (!p->batched) p->fan.fork(st);
+            int i = 0;
+            for (int k = NQCLASS - 1; k >= 0; --k) {
+                if (!p->qcount[k] && !p->batched) continue;
+                p->last_dig[k] = p->digest_args(k, nset, delta, dthr);
+                hipStream_t s2 = p->batched ? st : p->fan.on(i++);
+                p->prof.time(98 + k, s2, [&] { aimdhf::launch_digest(k, p->last_dig[k], threads, s2); });
+            }
+            if (!p->batched) p->fan.join();
+        }
         p->have_last_store = true;
-        for (int t = 8; t >= 0; --t) {
-            int nout = p->out_off[t + 1] - p->out_off[t];
-            if (nout <= 0) continue;
-            hipStream_t s2 = p->fan.on(i++);
-            p->prof.time(55 + t, s2, [&] { aimdhf::launch_kstore(t, ka, nout, s2); });
-            p->prof.time(93, s2, [&] { aimdhf::launch_kreduce(t, ka, nout, s2); });
-        }
-        for (int c = 5; c >= 0; --c) {
-            if (!p->ncls[c]) continue;
-            ja.cls_off = p->cls_pair_off[c];
-            hipStream_t s2 = p->fan.on(i++);
-            p->prof.time(49 + c, s2, [&] { aimdhf::launch_jstore(c, ja, p->ncls[c], s2); });
-            p->prof.time(94, s2, [&] { aimdhf::launch_jreduce(c, ja, p->ncls[c], s2); });
-        }
-        p->fan.join();
+        p->prof.time(93, st, [&] { aimdhf::launch_jk_finish(pa, st); });
         HIPCHECK(hipGetLastError());
     } catch (const HipError& e) {
         return e.code;
@@ -1643,34 +1466,12 @@ int aimdhf_jk_delta(aimdhf_plan* p, int nset, const double* ddens, double* dJ, d
     return jk_from_store(p, nset, ddens, dJ, dK, true, threshold, (hipStream_t)stream);
 }
 
-// J and K of every replica of a batch from its dense tensor; dens, J, K in the
-// padded layout (nrep, nset, ld, ld)
-static int jk_batch(aimdhf_plan* p, int nset, const double* dens, double* J, double* K, hipStream_t st) {
-    try {
-        const size_t n = (size_t)nset * p->mat_elems();
-        p->d_dsym.ensure(sizeof(double) * n);
-        p->prof.time(45, st, [&] {
-            aimdhf::launch_symmetrize(dens, p->nrep * nset, p->bld, p->d_dsym.as<double>(), st);
-            aimdhf::launch_zero_d(J, n, st);
-            aimdhf::launch_zero_d(K, n, st);
-        });
-        p->prof.time(49, st, [&] {
-            aimdhf::launch_batch_jk(p->batch_args(), nset, p->d_dsym.as<double>(), J, K, p->rep_item[p->nrep],
-                                    p->batch_jk_lanes, st);
-        });
-        HIPCHECK(hipGetLastError());
-    } catch (const HipError& e) {
-        return e.code;
-    }
-    return AIMDHF_OK;
-}
-
 int aimdhf_jk(aimdhf_plan* p, int nset, const double* dens, double* J, double* K, void* stream) {
     if (!p || !dens || !J || !K) return fail(AIMDHF_E_ARG, "NULL argument");
     if (nset < 1 || nset > 2) return fail(AIMDHF_E_ARG, "nset must be 1 or 2");
     if (!p->have_geometry) return fail(AIMDHF_E_STATE, "no geometry set");
     hipStream_t st = (hipStream_t)stream;
-    if (p->batched) return jk_batch(p, nset, dens, J, K, st);
+    if (p->batched) return jk_from_store(p, nset, dens, J, K, false, 0.0, st);
     if (p->generic) return jk_generic(p, nset, dens, J, K, st);
     if (p->stored) return jk_from_store(p, nset, dens, J, K, false, 0.0, st);
     try {
@@ -2077,11 +1878,10 @@ int aimdhf_jk_info(aimdhf_plan* p, int* stored, int64_t* store_bytes, int64_t* k
     if (!p) return fail(AIMDHF_E_ARG, "NULL plan");
     if (!p->have_geometry) return fail(AIMDHF_E_STATE, "no geometry set");
     if (stored) *stored = p->stored ? 1 : 0;
-    if (gather_bytes)
-        *gather_bytes = p->stored ? 8 * (p->kdata_total + p->jdata_total) + 4 * (p->kdata32_total + p->jdata32_total) : 0;
+    if (gather_bytes) *gather_bytes = p->stored ? (int64_t)p->store_need : 0;
     if (store_bytes) *store_bytes = p->store_bytes;
-    if (k_entries) *k_entries = p->k_entries;
-    if (j_entries) *j_entries = p->j_entries;
+    if (k_entries) *k_entries = p->stored ? p->qtotal : 0;
+    if (j_entries) *j_entries = 0;
     return AIMDHF_OK;
 }
 
@@ -2089,45 +1889,15 @@ int aimdhf_jk_type_info(aimdhf_plan* p, int64_t* k_bytes, int64_t* k_entries, in
                         int64_t* unique_bytes) {
     if (!p) return fail(AIMDHF_E_ARG, "NULL plan");
     if (!p->have_geometry) return fail(AIMDHF_E_STATE, "no geometry set");
-    try {
-        if (unique_bytes)
-            for (int k = 0; k < NQCLASS; ++k)
-                unique_bytes[k] = p->stored ? 8 * (p->store_base[k + 1] - p->store_base[k]) : 0;
-        for (int t = 0; t < 9; ++t) {
-            if (k_bytes) k_bytes[t] = 0;
-            if (k_entries) k_entries[t] = 0;
-        }
-        for (int c = 0; c < 6; ++c) {
-            if (j_bytes) j_bytes[c] = 0;
-            if (j_entries) j_entries[c] = 0;
-        }
-        if (!p->stored || p->batched) return AIMDHF_OK;
-        // K segments are (output block, subclass) with the output blocks grouped by type
-        auto at = [&](const DevBuf& b, long long i) {
-            long long v = 0;
-            HIPCHECK(hipMemcpy(&v, b.as<long long>() + i, sizeof(long long), hipMemcpyDeviceToHost));
-            return v;
-        };
-        for (int t = 0; t < 9; ++t) {
-            const long long a = 9LL * p->out_off[t], b = 9LL * p->out_off[t + 1];
-            if (k_bytes)
-                k_bytes[t] = 8 * (at(p->d_kdoff, b) - at(p->d_kdoff, a)) + 4 * (at(p->d_kdoff32, b) - at(p->d_kdoff32, a));
-            if (k_entries) k_entries[t] = at(p->d_kseg, b) - at(p->d_kseg, a);
-        }
-        // J segments are indexed by pair; each pair's six segments go to its class
-        const size_t njs = (size_t)p->npair * 6 + 1;
-        std::vector<long long> seg(njs), d64(njs), d32(njs);
-        HIPCHECK(hipMemcpy(seg.data(), p->d_jseg.p, sizeof(long long) * njs, hipMemcpyDeviceToHost));
-        HIPCHECK(hipMemcpy(d64.data(), p->d_jdoff.p, sizeof(long long) * njs, hipMemcpyDeviceToHost));
-        HIPCHECK(hipMemcpy(d32.data(), p->d_jdoff32.p, sizeof(long long) * njs, hipMemcpyDeviceToHost));
-        for (int P = 0; P < p->npair; ++P) {
-            const int c = p->pair_cls[P];
-            const size_t a = (size_t)P * 6, b = a + 6;
-            if (j_bytes) j_bytes[c] += 8 * (d64[b] - d64[a]) + 4 * (d32[b] - d32[a]);
-            if (j_entries) j_entries[c] += seg[b] - seg[a];
-        }
-    } catch (const HipError& e) {
-        return e.code;
+    for (int k = 0; unique_bytes && k < NQCLASS; ++k)
+        unique_bytes[k] = p->stored ? aimdhf::store_block(k) * (8 * p->q64count[k] + 4 * (p->qcount[k] - p->q64count[k])) : 0;
+    for (int t = 0; t < 9; ++t) {
+        if (k_bytes) k_bytes[t] = 0;
+        if (k_entries) k_entries[t] = 0;
+    }
+    for (int c = 0; c < 6; ++c) {
+        if (j_bytes) j_bytes[c] = 0;
+        if (j_entries) j_entries[c] = 0;
     }
     return AIMDHF_OK;
 }
@@ -2146,27 +1916,18 @@ int aimdhf_profile_enable(aimdhf_plan* p, int on) {
 int aimdhf_profile_replay(aimdhf_plan* p, int kind, int reps, void* stream, double* avg_ms) {
     if (!p || !avg_ms) return fail(AIMDHF_E_ARG, "NULL argument");
     if (reps < 1) return fail(AIMDHF_E_ARG, "reps must be >= 1");
-    const bool ks = kind >= 55 && kind < 64, js = kind >= 49 && kind < 55;
-    if (!ks && !js) return fail(AIMDHF_E_UNSUPPORTED, "replay covers the store-mode digestion kinds 49..63");
-    if (!p->have_geometry || !p->stored || !p->have_last_store)
+    const int k = kind - 98;
+    if (k < 0 || k >= NQCLASS) return fail(AIMDHF_E_UNSUPPORTED, "replay covers the store-mode digestion kinds 98..118");
+    if (!p->have_geometry || !p->stored || !p->have_last_store || !p->qcount[k])
         return fail(AIMDHF_E_STATE, "replay needs a store-mode J/K build at the current geometry");
     hipStream_t st = (hipStream_t)stream;
     hipEvent_t a = nullptr, b = nullptr;
     try {
         HIPCHECK(hipEventCreate(&a));
         HIPCHECK(hipEventCreate(&b));
-        aimdhf::JSArgs ja = p->last_ja;
-        const int t = kind - 55, c = kind - 49;
-        if (js) ja.cls_off = p->cls_pair_off[c];
-        const int nout = ks ? p->out_off[t + 1] - p->out_off[t] : p->ncls[c];
-        // the digestion writes only its unit partials: replays leave J and K alone
+        // the digestion adds to accumulators that every build clears: replays leave J and K alone
         HIPCHECK(hipEventRecord(a, st));
-        for (int r = 0; r < reps; ++r) {
-            if (ks)
-                aimdhf::launch_kstore(t, p->last_ka, nout, st);
-            else
-                aimdhf::launch_jstore(c, ja, nout, st);
-        }
+        for (int r = 0; r < reps; ++r) aimdhf::launch_digest(k, p->last_dig[k], 256, st);
         HIPCHECK(hipEventRecord(b, st));
         HIPCHECK(hipEventSynchronize(b));
         float ms = 0.0f;

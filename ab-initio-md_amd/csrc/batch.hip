@@ -1,8 +1,7 @@
 // Batched plans: many independent small molecules (replicas) in one plan. Their
-// screened quartets are evaluated into the class-binned store by the ordinary
-// per-class store kernels (one launch per class for all replicas); this file
-// expands the stored blocks into one dense (n_r^4) integral tensor per replica
-// and digests those into J and K for every replica in a single launch.
+// screened quartets are evaluated and digested by the per-class kernels that
+// single molecules use (one launch per class for all replicas); this file holds
+// the density and DIIS solvers of all replicas at once.
 //
 // Matrices of a batch live in a padded layout: replica r's (nset x) ld x ld
 // block starts at (r * nset + x) * ld^2; rows and columns past n_r stay zero.
@@ -12,99 +11,6 @@
 namespace aimdhf {
 
 namespace {
-
-__device__ __forceinline__ int ncart_of(int l) { return (l + 1) * (l + 2) / 2; }
-
-// one thread per stored integral: class by binary search over the class
-// offsets, then the integral's four AOs; the value goes to all eight
-// permutation-equivalent places of its replica's tensor (the same value where
-// places coincide)
-__global__ __launch_bounds__(256) void k_batch_scatter(BatchArgs b, long long total) {
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= total) return;
-    int k = 0;
-    for (int step = 16; step > 0; step >>= 1)
-        if (k + step <= NQCLASS_B - 1 && b.store_base[k + step] <= t) k += step;
-    const long long local = t - b.store_base[k];
-    const int blk = b.blk[k], ncd = b.ncd[k];
-    const long long q = b.qoff[k] + local / blk;
-    const int e = (int)(local % blk), ab = e / ncd, cd = e % ncd;
-    const int2 pq = b.list[q];
-    const int A = b.pair_a[pq.x], B = b.pair_b[pq.x], C = b.pair_a[pq.y], D = b.pair_b[pq.y];
-    const int nb = ncart_of(b.shell_l[B]), nd = ncart_of(b.shell_l[D]);
-    const long long m = b.shell_ao[A] + ab / nb, n = b.shell_ao[B] + ab % nb;
-    const long long l = b.shell_ao[C] + cd / nd, s = b.shell_ao[D] + cd % nd;
-    const int r = b.shell_rep[A];
-    const long long N = b.rep_nao[r];
-    double* T = b.tens + b.rep_toff[r];
-    const double v = b.store[t];
-    const long long mn = m * N + n, nm = n * N + m, ls = l * N + s, sl = s * N + l, NN = N * N;
-    T[mn * NN + ls] = v;
-    T[nm * NN + ls] = v;
-    T[mn * NN + sl] = v;
-    T[nm * NN + sl] = v;
-    T[ls * NN + mn] = v;
-    T[sl * NN + mn] = v;
-    T[ls * NN + nm] = v;
-    T[sl * NN + nm] = v;
-}
-
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-
-// G lanes (64, 32 or 16) per output element (r, m, c), lanes over (l, s):
-//   J_x[m][c] = sum_{l,s} (m c|l s) D_x[l][s]     (the contiguous slab T[m][c])
-//   K_x[m][c] = sum_{l,s} (m l|c s) D_x[l][s]     (rows T[m][l][c][.])
-// both against the same density element; fixed per-lane order and a butterfly
-// sum within the G lanes: bitwise reproducible for a given G
-template <int G>
-__global__ __launch_bounds__(256) void k_batch_jk(BatchArgs b, int nset, const double* __restrict__ dens,
-                                                  double* __restrict__ J, double* __restrict__ K, long long nitems) {
-    const long long item = ((long long)blockIdx.x * blockDim.x + threadIdx.x) / G;
-    const int lane = threadIdx.x % G;
-    if (item >= nitems) return;                 // whole groups of G lanes leave together
-    int r = 0;
-    for (int step = 1 << 20; step > 0; step >>= 1)
-        if (r + step < b.nrep && b.rep_item[r + step] <= item) r += step;
-    const long long loc = item - b.rep_item[r];
-    const int N = b.rep_nao[r];
-    const int m = (int)(loc / N), c = (int)(loc % N);
-    const double* T = b.tens + b.rep_toff[r];
-    const size_t ld = b.ld, ld2 = ld * ld;
-    const double* D0 = dens + (size_t)r * nset * ld2;
-    double ja[2] = {0.0, 0.0}, ka[2] = {0.0, 0.0};
-    const double* slab = T + ((size_t)m * N + c) * N * N;
-    const double* krow = T + (size_t)m * N * N * N + (size_t)c * N;   // + l N^2 + s
-    for (int e = lane; e < N * N; e += G) {
-        const int l = e / N, s = e % N;
-        const size_t de = (size_t)l * ld + s;
-        const double tj = slab[e], tk = krow[(size_t)l * N * N + s];
-        const double d0 = D0[de];
-        ja[0] += tj * d0;
-        ka[0] += tk * d0;
-        if (nset == 2) {
-            const double d1 = D0[ld2 + de];
-            ja[1] += tj * d1;
-            ka[1] += tk * d1;
-        }
-    }
-    for (int x = 0; x < nset; ++x) {
-        double jv = ja[x], kv = ka[x];
-#pragma unroll
-        for (int o = G / 2; o >= 1; o >>= 1) {
-            jv += __shfl_xor(jv, o, 64);
-            kv += __shfl_xor(kv, o, 64);
-        }
-        if (lane == 0) {
-            const size_t o = ((size_t)r * nset + x) * ld2 + (size_t)m * ld + c;
-            J[o] = jv;
-            K[o] = kv;
-        }
-    }
-}
 
 // Trace-correcting purification of nmat symmetric ld x ld matrices (ld <= 64), one
 // workgroup per matrix held in LDS for all steps: X0 = (e_max - F) / (e_max -
@@ -272,23 +178,6 @@ void launch_batch_purify(int nmat, int ld, const double* F, const double* nocc, 
 
 void launch_batch_diis_solve(int nrep, int m, const double* G, const double* r, double* c, hipStream_t st) {
     if (nrep > 0) k_batch_diis_solve<<<dim3((nrep + 63) / 64), dim3(64), 0, st>>>(nrep, m, G, r, c);
-}
-
-void launch_batch_scatter(const BatchArgs& b, long long total, hipStream_t st) {
-    if (total > 0) k_batch_scatter<<<dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st>>>(b, total);
-}
-
-void launch_batch_jk(const BatchArgs& b, int nset, const double* dens, double* J, double* K, long long nitems,
-                     int lanes, hipStream_t st) {
-    if (nitems <= 0) return;
-    const long long per = 256 / lanes;          // output elements per workgroup
-    const dim3 grid((unsigned)((nitems + per - 1) / per));
-    if (lanes == 16)
-        k_batch_jk<16><<<grid, dim3(256), 0, st>>>(b, nset, dens, J, K, nitems);
-    else if (lanes == 32)
-        k_batch_jk<32><<<grid, dim3(256), 0, st>>>(b, nset, dens, J, K, nitems);
-    else
-        k_batch_jk<64><<<grid, dim3(256), 0, st>>>(b, nset, dens, J, K, nitems);
 }
 
 }  // namespace aimdhf

@@ -1,12 +1,15 @@
-// Per-geometry evaluation of the screened unique quartets of one class
-// (compiled once per class with -DAIMDHF_QCLASS=k) into the HBM integral
-// store. Quartet t of the class list (bra = heavier pair, ties: higher pair
-// index) keeps its contracted block at store[t * NAB * NCD + ab * NCD + cd],
-// ab / cd over the bra / ket pair records. The list holds the class's FP64
-// quartets first; in mixed precision the rest (q_P q_Q below the switch, held
-// and digested in FP32 afterwards) are also evaluated in FP32.
+// Evaluation of screened unique quartets of one class (compiled once per class
+// with -DAIMDHF_QCLASS=k) into the integral store. Quartet t of a list part
+// (bra = heavier pair) keeps value v = cd NAB + ab (ab / cd over the bra / ket
+// pair records) at (t / 64) 64 NAB NCD + 64 v + t % 64: tiles of 64 quartets,
+// value-major, so that every store of a wavefront here and every load of the J/K
+// digestion covers 64 consecutive words. In mixed precision the quartets below
+// the switch are evaluated and held in FP32. The lanes of a wavefront take 64
+// consecutive quartets (one bra run of the list: the same bra records for most
+// of them); classes whose block does not fit the registers take one ket
+// component per wavefront.
 
-#include "aimdhf_internal.h"
+#include "jk_digest.h"
 #include "md_eri.h"
 
 #ifndef AIMDHF_QCLASS
@@ -29,27 +32,31 @@ constexpr int BLK = Qt::NAB * Qt::NCD;
 constexpr int NSPLIT = SPLIT ? Qt::NCD : 1;
 
 template <int LA_, int LB_, int LC_, int LD_, typename Real>
-__global__ __launch_bounds__(256) void k_eri_store(StoreArgs a, const int2* __restrict__ list, long long nq) {
+__global__ __launch_bounds__(256) void k_eri(EriArgs a, Real* __restrict__ store, long long nq) {
     __shared__ double btab[BOYS_NGRID * BOYS_SROW];
     boys_stage(a.boys, LA_ + LB_ + LC_ + LD_, btab);
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nq * NSPLIT) return;
-    const long long q = t / NSPLIT;
-    const int2 pq = list[q];
-    const double* rb = a.recs + a.rec_off[pq.x];
-    const double* rk = a.recs + a.rec_off[pq.y];
-    double* out = a.store + q * BLK;
+    const long long it = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long long g = it >> 6;                    // wavefront: tile g / NSPLIT, ket component g % NSPLIT
+    const int lane = (int)(it & 63);
+    const long long q = g / NSPLIT * 64 + lane;
+    if (q >= nq) return;
+    const int P = a.cls_pairs[a.lbra[q]], Q = a.cls_pairs[a.lket[q]];
+    const double* rb = a.recs + a.rec_off[P];
+    const double* rk = a.recs + a.rec_off[Q];
+    Real* out = store + (q >> 6) * (64 * BLK) + lane;
     if constexpr (SPLIT) {
-        const int cd = (int)(t % NSPLIT);
+        const int cd = (int)(g % NSPLIT);
         Real acc[Qt::NAB];
-        eri_quartet_cd<LA_, LB_, LC_, LD_, true, Real>(rb, a.npp[pq.x], rk, a.npp[pq.y], btab, cd, acc);
+        eri_quartet_cd<LA_, LB_, LC_, LD_, true, Real>(rb, a.npp[P], rk, a.npp[Q], btab, cd, acc);
 #pragma unroll
-        for (int ab = 0; ab < Qt::NAB; ++ab) out[ab * Qt::NCD + cd] = double(acc[ab]);
+        for (int ab = 0; ab < Qt::NAB; ++ab) out[(cd * Qt::NAB + ab) * 64] = acc[ab];
     } else {
         Real acc[BLK];
-        eri_quartet<LA_, LB_, LC_, LD_, true, Real>(rb, a.npp[pq.x], rk, a.npp[pq.y], btab, acc);
+        eri_quartet<LA_, LB_, LC_, LD_, true, Real>(rb, a.npp[P], rk, a.npp[Q], btab, acc);
 #pragma unroll
-        for (int i = 0; i < BLK; ++i) out[i] = double(acc[i]);
+        for (int ab = 0; ab < Qt::NAB; ++ab)
+#pragma unroll
+            for (int cd = 0; cd < Qt::NCD; ++cd) out[(cd * Qt::NAB + ab) * 64] = acc[ab * Qt::NCD + cd];
     }
 }
 }  // namespace
@@ -57,18 +64,15 @@ __global__ __launch_bounds__(256) void k_eri_store(StoreArgs a, const int2* __re
 #define CAT2(a, b) a##b
 #define CAT(a, b) CAT2(a, b)
 
-// quartets [0, n64) of the class list in FP64, [n64, nq) in FP32
-void CAT(launch_eri_store_, AIMDHF_QCLASS)(const StoreArgs& a, const int2* list, long long nq, long long n64,
-                                           hipStream_t st) {
-    const long long nt = n64 * NSPLIT;
-    if (nt > 0)
-        k_eri_store<LA, LB, LC, LD, double><<<dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, st>>>(a, list, n64);
-    const long long nt32 = (nq - n64) * NSPLIT;
-    if (nt32 > 0) {
-        StoreArgs a32 = a;
-        a32.store = a.store + n64 * BLK;
-        k_eri_store<LA, LB, LC, LD, float><<<dim3((unsigned)((nt32 + 255) / 256)), dim3(256), 0, st>>>(
-            a32, list + n64, nq - n64);
+// n64 quartets from a.lbra in FP64, the n32 after them in FP32
+void CAT(launch_eri_, AIMDHF_QCLASS)(const EriArgs& a, long long n64, long long n32, hipStream_t st) {
+    auto blocks = [](long long n) { return dim3((unsigned)(((n + 63) / 64 * 64 * NSPLIT + 255) / 256)); };
+    if (n64 > 0) k_eri<LA, LB, LC, LD, double><<<blocks(n64), dim3(256), 0, st>>>(a, a.out64, n64);
+    if (n32 > 0) {
+        EriArgs b = a;
+        b.lbra += n64;
+        b.lket += n64;
+        k_eri<LA, LB, LC, LD, float><<<blocks(n32), dim3(256), 0, st>>>(b, a.out32, n32);
     }
 }
 

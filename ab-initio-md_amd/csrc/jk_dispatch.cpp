@@ -1,6 +1,7 @@
 // Dispatch tables over the per-class / per-type kernel objects (one object
 // per template configuration, see the Makefile).
 #include "aimdhf_internal.h"
+#include "jk_digest.h"
 
 namespace aimdhf {
 
@@ -66,84 +67,38 @@ void launch_kown(int type, const KOArgs& a, int nout, const int* has_l, hipStrea
     fns[type](a, nout, has_l, st);
 }
 
-#define DECLS(k) void launch_eri_store_##k(const StoreArgs&, const int2*, long long, long long, hipStream_t);
+#define DECLS(k) void launch_eri_##k(const EriArgs&, long long, long long, hipStream_t); \
+    void launch_digest_##k(const DigestArgs&, int, hipStream_t);
 DECLS(0) DECLS(1) DECLS(2) DECLS(3) DECLS(4) DECLS(5) DECLS(6) DECLS(7) DECLS(8) DECLS(9) DECLS(10)
 DECLS(11) DECLS(12) DECLS(13) DECLS(14) DECLS(15) DECLS(16) DECLS(17) DECLS(18) DECLS(19) DECLS(20)
 #undef DECLS
-#define DECLJS(c) void launch_jstore_##c(const JSArgs&, int, hipStream_t); \
-    void launch_jreduce_##c(const JSArgs&, int, hipStream_t); \
-    void launch_jcopy_##c(const JSArgs&, int, hipStream_t);
-DECLJS(0) DECLJS(1) DECLJS(2) DECLJS(3) DECLJS(4) DECLJS(5)
-#undef DECLJS
-#define DECLKS(x, y) void launch_kstore_##x##_##y(const KSArgs&, int, hipStream_t); \
-    void launch_kreduce_##x##_##y(const KSArgs&, int, hipStream_t); \
-    void launch_kcopy_##x##_##y(const KSArgs&, int, hipStream_t);
-DECLKS(0, 0) DECLKS(0, 1) DECLKS(0, 2) DECLKS(1, 0) DECLKS(1, 1) DECLKS(1, 2) DECLKS(2, 0) DECLKS(2, 1) DECLKS(2, 2)
-#undef DECLKS
 
-void launch_eri_store(int k, const StoreArgs& a, const int2* list, long long nq, long long n64, hipStream_t st) {
-    typedef void (*Fn)(const StoreArgs&, const int2*, long long, long long, hipStream_t);
+void launch_eri(int k, const EriArgs& a, long long n64, long long n32, hipStream_t st) {
+    typedef void (*Fn)(const EriArgs&, long long, long long, hipStream_t);
     static const Fn fns[21] = {
-        launch_eri_store_0, launch_eri_store_1, launch_eri_store_2, launch_eri_store_3, launch_eri_store_4,
-        launch_eri_store_5, launch_eri_store_6, launch_eri_store_7, launch_eri_store_8, launch_eri_store_9,
-        launch_eri_store_10, launch_eri_store_11, launch_eri_store_12, launch_eri_store_13, launch_eri_store_14,
-        launch_eri_store_15, launch_eri_store_16, launch_eri_store_17, launch_eri_store_18, launch_eri_store_19,
-        launch_eri_store_20};
-    fns[k](a, list, nq, n64, st);
+        launch_eri_0, launch_eri_1, launch_eri_2, launch_eri_3, launch_eri_4, launch_eri_5, launch_eri_6,
+        launch_eri_7, launch_eri_8, launch_eri_9, launch_eri_10, launch_eri_11, launch_eri_12, launch_eri_13,
+        launch_eri_14, launch_eri_15, launch_eri_16, launch_eri_17, launch_eri_18, launch_eri_19, launch_eri_20};
+    fns[k](a, n64, n32, st);
 }
 
-void launch_jcopy(int pclass, const JSArgs& a, int npairs, hipStream_t st) {
-    typedef void (*Fn)(const JSArgs&, int, hipStream_t);
-    static const Fn fns[6] = {launch_jcopy_0, launch_jcopy_1, launch_jcopy_2,
-                              launch_jcopy_3, launch_jcopy_4, launch_jcopy_5};
-    fns[pclass](a, npairs, st);
+void launch_digest(int k, const DigestArgs& a, int threads, hipStream_t st) {
+    typedef void (*Fn)(const DigestArgs&, int, hipStream_t);
+    static const Fn fns[21] = {
+        launch_digest_0, launch_digest_1, launch_digest_2, launch_digest_3, launch_digest_4, launch_digest_5,
+        launch_digest_6, launch_digest_7, launch_digest_8, launch_digest_9, launch_digest_10, launch_digest_11,
+        launch_digest_12, launch_digest_13, launch_digest_14, launch_digest_15, launch_digest_16, launch_digest_17,
+        launch_digest_18, launch_digest_19, launch_digest_20};
+    fns[k](a, threads, st);
 }
 
-void launch_kcopy(int type, const KSArgs& a, int nout, hipStream_t st) {
-    typedef void (*Fn)(const KSArgs&, int, hipStream_t);
-    static const Fn fns[9] = {launch_kcopy_0_0, launch_kcopy_0_1, launch_kcopy_0_2,
-                              launch_kcopy_1_0, launch_kcopy_1_1, launch_kcopy_1_2,
-                              launch_kcopy_2_0, launch_kcopy_2_1, launch_kcopy_2_2};
-    fns[type](a, nout, st);
-}
-
-// doubles per stored block of quartet class k (heavier pair as bra)
+// integrals per block of quartet class k (heavier pair as bra)
 long long store_block(int k) {
     static const int ncp[6] = {1, 3, 9, 6, 18, 36};
     int hi = 0;
     while ((hi + 1) * (hi + 2) / 2 <= k) ++hi;
     int lo = k - hi * (hi + 1) / 2;
     return (long long)ncp[hi] * ncp[lo];
-}
-
-void launch_jstore(int pclass, const JSArgs& a, int npairs, hipStream_t st) {
-    typedef void (*Fn)(const JSArgs&, int, hipStream_t);
-    static const Fn fns[6] = {launch_jstore_0, launch_jstore_1, launch_jstore_2,
-                              launch_jstore_3, launch_jstore_4, launch_jstore_5};
-    fns[pclass](a, npairs, st);
-}
-
-void launch_kstore(int type, const KSArgs& a, int nout, hipStream_t st) {
-    typedef void (*Fn)(const KSArgs&, int, hipStream_t);
-    static const Fn fns[9] = {launch_kstore_0_0, launch_kstore_0_1, launch_kstore_0_2,
-                              launch_kstore_1_0, launch_kstore_1_1, launch_kstore_1_2,
-                              launch_kstore_2_0, launch_kstore_2_1, launch_kstore_2_2};
-    fns[type](a, nout, st);
-}
-
-void launch_jreduce(int pclass, const JSArgs& a, int npairs, hipStream_t st) {
-    typedef void (*Fn)(const JSArgs&, int, hipStream_t);
-    static const Fn fns[6] = {launch_jreduce_0, launch_jreduce_1, launch_jreduce_2,
-                              launch_jreduce_3, launch_jreduce_4, launch_jreduce_5};
-    fns[pclass](a, npairs, st);
-}
-
-void launch_kreduce(int type, const KSArgs& a, int nout, hipStream_t st) {
-    typedef void (*Fn)(const KSArgs&, int, hipStream_t);
-    static const Fn fns[9] = {launch_kreduce_0_0, launch_kreduce_0_1, launch_kreduce_0_2,
-                              launch_kreduce_1_0, launch_kreduce_1_1, launch_kreduce_1_2,
-                              launch_kreduce_2_0, launch_kreduce_2_1, launch_kreduce_2_2};
-    fns[type](a, nout, st);
 }
 
 }  // namespace aimdhf

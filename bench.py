@@ -13,7 +13,7 @@ tests/golden/water16.xyz (16 randomly rotated waters in an 8 A cube, O-O >=
 
 By default the FP64 trajectory runs first; the mixed-precision path (FP32 for
 quartets below the Schwarz switches, and incremental Fock builds whose
-density differences are screened and digested in FP32) then computes the same geometries with
+density differences are screened) then computes the same geometries with
 its own density reuse, and its energies and forces are compared with the
 FP64 ones at every step. ``value`` is the mixed step time when it stays
 within |dE| <= 1e-6 Eh and |dF| <= 1e-5 Eh/bohr at every step, else FP64.
@@ -195,8 +195,7 @@ def main() -> int:
                   for k in range(eng.NKIND) if n_kind[k] > 0}
     roofline = dominant_kernel_roofline(eng, ms_kind, n_kind, tinfo, gw)
     unique_b = int(tinfo["unique_bytes"].sum())
-    streamed_b = int(tinfo["k_bytes"].sum() + tinfo["j_bytes"].sum()
-                     + 8 * (tinfo["k_entries"].sum() + tinfo["j_entries"].sum()))
+    streamed_b = unique_b + 4 * info["k_entries"]
     use_mixed = mixed is not None and mixed["within_bounds"]
     value = mixed["ms_per_step"] if use_mixed else ms_per_step
     out = {
@@ -215,8 +214,8 @@ def main() -> int:
         "config": {
             "workload": "(H2O)16 RHF/6-31G* (304 AOs), velocity-Verlet NVE BOMD step at 0.5 fs, 300 K, "
                         "SCF conv 1e-10 Eh / 1e-7, Schwarz 1e-12, gradient screening 1e-14; value: the mixed "
-                        "path (FP32 below the Schwarz switches, incremental Fock with FP32 density-difference "
-                        "builds) over the FP64 trajectory's geometries when it "
+                        "path (FP32 below the Schwarz switches, incremental Fock) "
+                        "over the FP64 trajectory's geometries when it "
                         "stays within |dE| <= 1e-6 Eh and |dF| <= 1e-5 Eh/bohr of FP64 at every step, else FP64; "
                         "per-kernel figures from the FP64 run",
             "geometry": "tests/golden/water16.xyz",
@@ -236,8 +235,7 @@ def main() -> int:
         "jk_traffic": {"unique_integral_bytes": unique_b, "streamed_bytes_per_build": streamed_b,
                        "streamed_over_unique": round(streamed_b / unique_b, 3) if unique_b else None,
                        "stream_gbs": round(streamed_b / (jk_ms * 1e-3) / 1e9, 1) if jk_ms > 0 and unique_b else None,
-                       "note": "streamed = gather-ordered integral copies plus 8-byte list entries that one "
-                               "J/K build reads; unique = the screened integrals stored once"},
+                       "note": "streamed = the screened integrals, each read once, plus 4-byte list entries"},
         "store_build_ms_per_step": round(store_ms, 3),
         "store_bytes": info["store_bytes"],
         "gradient_kernels_ms_per_step": round(float(grad_ms), 3),
@@ -428,47 +426,37 @@ def bench_replicas(args):
 def dominant_kernel_roofline(eng, ms_kind, n_kind, tinfo, gw):
     """Roofline of the kernel with the largest time per step in the serialised profiling
     step, among the kinds that time one kernel per launch: the derivative-ERI classes
-    (FP64 VALU, flops from flopmodel.grad_work), and the store-mode exchange and Coulomb
-    digestion (HBM, the gather-ordered integral copies and list entries one launch
-    streams)."""
+    (FP64 VALU, flops from flopmodel.grad_work), and the store-mode J/K digestion per
+    quartet class (HBM, the integrals and list entries one launch streams)."""
     from aimd_amd.qc import flopmodel
-    kstore = {55 + t: t for t in range(9)}
-    jstore = {49 + c: c for c in range(6)}
-    cands = list(range(21, 42)) + list(kstore) + list(jstore)
+    cands = list(range(21, 42)) + list(range(98, 119))
     k = max(cands, key=lambda i: float(ms_kind[i]))
     avg_ms = float(ms_kind[k]) / max(int(n_kind[k]), 1)
     name = eng.KIND_NAMES[k]
     out = {"kind": name, "ms_per_step": round(float(ms_kind[k]), 4), "launches_per_step": int(n_kind[k]),
            "event_avg_launch_ms": round(avg_ms, 4)}
-    if k >= 49:
+    if k >= 98:
         # store digestion: 20 back-to-back launches with the last build's arguments between
         # one event pair (the per-launch event pairs of the step add dispatch gaps)
         avg_ms = eng.profile_replay(k, 20)
         out["replay_launches"] = 20
     out["avg_launch_ms"] = round(avg_ms, 4)
+    c = k - 21 if k < 42 else k - 98
+    ls = "/".join(str(v) for v in flopmodel.class_ls(c))
     if k < 42:
-        c = k - 21
         achieved = gw["per_class"][c] / (avg_ms * 1e-3) / 1e12
         out.update({"bound": "valu", "unit": "TFLOP/s", "peak": PEAK_FP64_TFLOPS,
-                    "kernel": f"k_grad_class<{c}, double> (derivative ERIs, quartet class "
-                              f"({'/'.join(str(v) for v in flopmodel.class_ls(c))}))",
+                    "kernel": f"k_grad_class<{c}, double> (derivative ERIs, quartet class ({ls}))",
                     "flops_per_launch": float(gw["per_class"][c]),
                     "note": "FP64 vector-ALU kernel (no MFMA instructions) against MI355X's FP64 vector peak"})
     else:
-        if k in kstore:
-            t = kstore[k]
-            nbytes = int(tinfo["k_bytes"][t] + 8 * tinfo["k_entries"][t])
-            kern = f"k_kstore<{t // 3}, {t % 3}, 1> (exchange from the integral store, output blocks " \
-                   f"{'spd'[t // 3]}{'spd'[t % 3]})"
-        else:
-            c = jstore[k]
-            nbytes = int(tinfo["j_bytes"][c] + 8 * tinfo["j_entries"][c])
-            kern = f"k_jstore<{c}, 1> (Coulomb from the integral store, pair class {eng.PAIR_CLASS_NAMES[c]})"
+        nbytes = int(tinfo["unique_bytes"][c] + 4 * eng.class_counts()[0][c])
         achieved = nbytes / (avg_ms * 1e-3) / 1e9
-        out.update({"bound": "hbm", "unit": "GB/s", "peak": PEAK_HBM_GBS, "kernel": kern,
+        out.update({"bound": "hbm", "unit": "GB/s", "peak": PEAK_HBM_GBS,
+                    "kernel": f"k_digest<{c}, 1, true> (J/K from the integral store, quartet class ({ls}))",
                     "bytes_per_launch": nbytes,
-                    "note": "bytes = gather-ordered integral copies (8 B FP64, 4 B FP32) and 8-byte list "
-                            "entries one launch streams; density reads hit L2 and are not counted"})
+                    "note": "bytes = the class's integrals (8 B FP64, 4 B FP32), each read once, and 4-byte list "
+                            "entries; density reads and K sums are in LDS and not counted"})
     out["achieved"] = round(achieved, 4)
     out["frac"] = round(achieved / out["peak"], 5)
     out["traffic"] = measured_traffic(out["kind"])

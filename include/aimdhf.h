@@ -67,8 +67,9 @@ int aimdhf_plan_destroy(aimdhf_plan* plan);
  * and each replica's nuclei act only on its own electrons, so every replica is
  * the molecule it would be alone. The entry points then work on all replicas at
  * once: set_geometry takes the concatenated positions and evaluates every
- * screened quartet of every replica (one launch per quartet class) into one dense
- * two-electron tensor per replica; jk digests all tensors in one launch;
+ * screened quartet of every replica into the integral store (one launch per
+ * quartet class); jk digests all replicas in one or two launches, which stay
+ * valid in a captured graph when the geometry moves;
  * one_electron, grad_one(_terms) and grad_two take and fill matrices in the
  * padded layout: nset (or 1) matrices of ld x ld per replica, replica by replica
  * ((nrep, nset, ld, ld); ld = the largest replica's AO count, see
@@ -83,8 +84,9 @@ int aimdhf_batch_create(int nrep, const int64_t* rep_atom, const int64_t* rep_sh
                         const double* charges, aimdhf_plan** out);
 
 /* Replicas (0 for a single-molecule plan), padded matrix dimension ld (nao for a
- * single molecule) and bytes of the dense tensors of a batch (any pointer may be
- * NULL). No counterpart in the reference. */
+ * single molecule) and the bytes that one dense n_r^4 integral tensor per replica
+ * would take, a measure of the batch's size (any pointer may be NULL). No
+ * counterpart in the reference. */
 int aimdhf_batch_layout(aimdhf_plan* plan, int* nrep, int* ld, int64_t* tensor_bytes);
 
 /*
@@ -93,8 +95,8 @@ int aimdhf_batch_layout(aimdhf_plan* plan, int* nrep, int* ld, int64_t* tensor_b
  * Schwarz bounds Q = max |(ab|ab)|^(1/2), and the class-binned list of unique
  * shell quartets whose contraction-block pairs satisfy Q_P Q_Q >= threshold.
  * In store mode (aimdhf_set_jk_mode) the screened quartets are also evaluated
- * here into a device-resident integral store, with the gather lists of the
- * J and K kernels. Synchronises the stream (the list sizes come back to the host).
+ * here into a device-resident integral store that every J/K build reads once.
+ * Synchronises the stream (the list sizes come back to the host).
  * Replaces: BasisSet.with_positions (aimd/qc/basis.py:242-246), _build_pairs
  * (aimd/qc/integrals.py:525-599), schwarz_bounds (aimd/qc/integrals.py:970-983)
  * and the screening loop of _eri_tensor_kernel (aimd/qc/integrals.py:900-903);
@@ -118,11 +120,13 @@ int aimdhf_quartets(aimdhf_plan* plan, int64_t* out_host, int64_t cap, int64_t* 
 /*
  * Coulomb and exchange matrices of nset densities (device (nset,nao,nao)):
  *   J_mn = sum_ls (mn|ls) D_ls,   K_mn = sum_ls (ml|ns) D_ls
- * of the symmetric part of each D over the screened quartets. Every output
- * block is owned by one wavefront that sums its contributions in a fixed
- * order (no atomics), so J and K are bitwise reproducible run to run.
- * Direct mode recomputes the integrals (J-engine in Hermite space for J,
- * per-block exchange owners for K); store mode reads them from the store.
+ * of the symmetric part of each D over the screened quartets, bitwise
+ * reproducible run to run. Direct mode recomputes the integrals (J-engine in
+ * Hermite space for J, per-block exchange owners for K), every output block
+ * owned by one wavefront; store mode reads each stored integral once and sums in
+ * 64-bit fixed point whose exponent follows the density and the Schwarz bounds
+ * (resolution 2^-62 of a bound of the largest element; a density with a NaN or
+ * infinity gives NaN in its J and K).
  * Replaces: jk_from_eri (aimd/qc/integrals.py:1009-1044) and, in direct mode,
  * eri_tensor (aimd/qc/integrals.py:986-1006).
  */
@@ -130,12 +134,11 @@ int aimdhf_jk(aimdhf_plan* plan, int nset, const double* dens, double* J, double
 
 /*
  * J and K of density differences dD (device (nset,nao,nao)) for an
- * incremental Fock build, J(D) = J(D_prev) + J(dD). In store mode a work unit
- * whose largest Q_P Q_Q times max |dD| is below threshold is skipped (each of
- * its integral-density products is below threshold), and in mixed precision
- * every stored integral is digested in FP32, the large-bound ones from FP32
- * copies made at set_geometry; threshold 0 skips nothing. In direct mode the
- * same as aimdhf_jk. Replaces the full jk_from_eri rebuild of every SCF
+ * incremental Fock build, J(D) = J(D_prev) + J(dD). In store mode quartets
+ * whose Q_P Q_Q times max |dD| is below threshold may be skipped (a wavefront
+ * skips 64 of them together; each integral-density product is below
+ * threshold); threshold 0 skips nothing. Sums are FP64 products of the stored
+ * integrals in both precisions. In direct mode the same as aimdhf_jk. Replaces the full jk_from_eri rebuild of every SCF
  * iteration (aimd/qc/scf.py:863-867, aimd/qc/integrals.py:1009-1044).
  */
 int aimdhf_jk_delta(aimdhf_plan* plan, int nset, const double* ddens, double* dJ, double* dK, double threshold,
@@ -154,9 +157,9 @@ int aimdhf_set_jk_mode(aimdhf_plan* plan, int mode, int64_t max_store_bytes);
  * derivative integrals of quartets with Q_P Q_Q max|Gamma| < grad_switch are
  * evaluated in FP32 (accumulated per quartet in FP32, summed in exact fixed
  * point), and, in store mode, integrals of quartets with Q_P Q_Q < jk_switch
- * are held and digested in FP32 (taking effect at the next set_geometry);
- * aimdhf_jk_delta digests every stored integral in FP32 once max |dD| <=
- * delta_switch. Large-bound quartets, the SCF algebra and all sums stay FP64.
+ * are evaluated and held in FP32 (taking effect at the next set_geometry).
+ * Large-bound quartets, the digestion, the SCF algebra and all sums stay FP64;
+ * delta_switch is accepted and has no effect (difference builds sum in FP64).
  * No counterpart in the reference (FP64 only).
  */
 int aimdhf_set_precision(aimdhf_plan* plan, int mode, double jk_switch, double grad_switch, double delta_switch);
@@ -198,9 +201,9 @@ int aimdhf_batch_purify(int nmat, int ld, const double* F, const double* nocc, d
                         double* err, void* stream);
 
 /*
- * Lanes (16, 32 or 64; default 64) that digest one output element of a
- * batched plan's J/K, for batches of small replicas where a full wavefront per
- * element leaves lanes idle. A tuning knob with no counterpart in the
+ * Lanes (16, 32 or 64; default 64): a workgroup of a batched plan's J/K has four
+ * threads per lane, for batches of small replicas whose runs of kets would
+ * leave larger workgroups idle. Results do not depend on it. A tuning knob with no counterpart in the
  * reference; aimd_amd.batch.ReplicaBatch.autotune times the choices.
  */
 int aimdhf_batch_set_jk_lanes(aimdhf_plan* plan, int lanes);
@@ -229,28 +232,26 @@ int aimdhf_tc2_error(int n, const double* X, double* err, void* stream);
  */
 int aimdhf_set_streams(aimdhf_plan* plan, int concurrent);
 
-/* Whether the current geometry has an integral store, its size in bytes, the
- * gather-list lengths of the K and J kernels and the bytes of their
- * gather-ordered integral data (FP64 and, in mixed precision, FP32), i.e. what
- * one J/K build streams (any pointer may be NULL). */
 /*
- * Lane items per work unit of the store-mode J/K digestion (64 .. 65536,
- * default 1024; one wavefront digests one unit), from the next
- * aimdhf_set_geometry on. A tuning knob with no counterpart in the
- * reference; results do not depend on it beyond the order of the unit sums.
+ * Least quartets (64 .. 65536, default 1024) a workgroup of the store-mode J/K
+ * digestion takes from a long run of kets. A tuning knob with no counterpart in
+ * the reference; results do not depend on it.
  */
 int aimdhf_set_store_units(aimdhf_plan* plan, int items);
 
+/* Whether the current geometry has an integral store, its size in bytes, the
+ * quartets one J/K build digests (k_entries; j_entries is 0: J and K come from
+ * the same reading) and the bytes of integrals it streams (any pointer may be
+ * NULL). */
 int aimdhf_jk_info(aimdhf_plan* plan, int* stored, int64_t* store_bytes, int64_t* k_entries, int64_t* j_entries,
                    int64_t* gather_bytes);
 
 /*
  * The integral store of the current geometry broken down for traffic
- * accounting: per exchange output type t = 3 l_X + l_Y (9) the gather-ordered
- * bytes one build streams and the gather-list entries, the same per Coulomb
- * pair class (6: ss ps pp ds dp dd), and the bytes of the unique screened
- * integrals per quartet class (21). All zero in direct mode (any pointer may
- * be NULL). No counterpart in the reference (its integrals are not stored);
+ * accounting: the bytes of the unique screened integrals per quartet class
+ * (21), which one build streams once, next to 4 bytes of list per quartet. The
+ * arrays per exchange output type (9) and Coulomb pair class (6) are zero: no
+ * reordered copies are kept. All zero in direct mode (any pointer may be NULL). No counterpart in the reference (its integrals are not stored);
  * for profilers and benchmarks.
  */
 int aimdhf_jk_type_info(aimdhf_plan* plan, int64_t* k_bytes, int64_t* k_entries, int64_t* j_bytes,
@@ -319,14 +320,13 @@ int aimdhf_grad_two(aimdhf_plan* plan, const double* Dc, int nx, const double* D
  * type (l_X, l_Y), 21..41 derivative-ERI kernels of the 21 quartet classes,
  * 42 geometry set-up, 43 one-electron integrals, 44 one-electron gradient,
  * 45 J/K prologue and epilogue, 46 Hermite densities, 47 integral store
- * evaluation, 15 gather-ordered copies, 48 gather-list build, 49..54 store J
- * per pair class, 55..63 store K per output type, 64..84 derivative-ERI
- * screening pre-pass per class; 85..88 host wall-clock phases (energy list,
- * owner lists, store build incl. its device work, gradient list) and 89..92
- * sub-phases of the store build (list counts, band tables, list fill, unit
- * tables; milliseconds of the calling thread, not events). aimdhf_profile_read synchronises, returns the
- * summed milliseconds and launch counts per kind (nkind <= 96) and optionally
- * resets.
+ * evaluation, 64..84 derivative-ERI screening pre-pass per class; 85..88 host
+ * wall-clock phases (energy list, owner lists, store build incl. its device
+ * work, gradient list; milliseconds of the calling thread, not events), 93 J/K
+ * from the store's accumulators, 94 the digestion of every class in one or two
+ * launches (small systems and batches), 98..118 the digestion per quartet class.
+ * aimdhf_profile_read synchronises, returns the summed milliseconds and launch
+ * counts per kind (nkind <= 119) and optionally resets.
  */
 int aimdhf_profile_enable(aimdhf_plan* plan, int on);
 int aimdhf_profile_read(aimdhf_plan* plan, double* ms, int64_t* launches, int nkind, int reset);
@@ -334,9 +334,8 @@ int aimdhf_profile_read(aimdhf_plan* plan, double* ms, int64_t* launches, int nk
 /*
  * Average duration in milliseconds of `reps` back-to-back launches, on
  * `stream`, of one store-mode digestion kernel with the arguments of the last
- * J/K build at the current geometry: kind 55 + t (exchange, output type t) or
- * 49 + c (Coulomb, pair class c). The kernels write only their unit partials,
- * so J and K are left as they were. No counterpart in the reference; for
+ * J/K build at the current geometry: kind 98 + quartet class. The kernels add to
+ * accumulators that every build clears, so J and K are left as they were. No counterpart in the reference; for
  * benchmarks (one event pair around many launches times the kernel without
  * the per-launch event and dispatch gaps).
  */
