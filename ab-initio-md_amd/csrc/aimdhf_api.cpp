@@ -247,6 +247,8 @@ struct aimdhf_plan {
     // runs, and the byte offset of every class's FP64 and FP32 blocks in the store
     long long koff[7] = {0}, npao = 0, runbase[NQCLASS + 1] = {0};
     int list_parts = 1;
+    int nheavy[6] = {0};            // leading ranks of each class with ERI_HEAVY primitive pairs or more
+    long long h64count[NQCLASS] = {0}, h32count[NQCLASS] = {0};
     long long list_off[NQCLASS + 1] = {0}, base64[NQCLASS] = {0}, base32[NQCLASS] = {0};
     size_t store_need = 0;
     int lds_limit = 65536;
@@ -547,7 +549,7 @@ struct aimdhf_plan {
     // screening values, runs of kets per bra and class, totals to the host.
     // Synchronises the stream.
     void build_quartets(double thr, double sw, hipStream_t st) {
-        if (!h_pin) HIPCHECK(hipHostMalloc((void**)&h_pin, sizeof(long long) * 64 + sizeof(aimdhf::DigestGeo) * NQCLASS));
+        if (!h_pin) HIPCHECK(hipHostMalloc((void**)&h_pin, sizeof(long long) * 128 + sizeof(aimdhf::DigestGeo) * NQCLASS));
         aimdhf::GeoArgs g;
         g.nshell = nshell;
         g.npair = npair;
@@ -572,7 +574,7 @@ struct aimdhf_plan {
         const long long cells = runs * aimdhf::LIST_WAVES;
         d_lcnt.ensure(sizeof(long long) * cells);
         d_loff.ensure(sizeof(long long) * (cells + 1));
-        d_lsum.ensure(sizeof(long long) * (aimdhf::list_scan_blocks(cells) + 64));
+        d_lsum.ensure(sizeof(long long) * (aimdhf::list_scan_blocks(cells) + 128));
         long long* picked = d_lsum.as<long long>() + aimdhf::list_scan_blocks(cells);
         aimdhf::QListArgs la;
         la.npair = npair;
@@ -597,6 +599,11 @@ struct aimdhf_plan {
             pk.at[pk.n++] = (runbase[k] + ncls[bra_class(k)]) * aimdhf::LIST_WAVES;
         }
         pk.at[pk.n++] = cells;
+        // where each part's contracted bras end
+        for (int k = 0; k < NQCLASS; ++k)
+            for (int part = 0; part < list_parts; ++part)
+                pk.at[pk.n++] = (runbase[k] + (long long)part * ncls[bra_class(k)] + nheavy[bra_class(k)]) *
+                                aimdhf::LIST_WAVES;
         aimdhf::launch_pick(pk, d_loff.as<long long>(), picked, st);
         HIPCHECK(hipGetLastError());
         HIPCHECK(hipMemcpyAsync(h_pin, picked, sizeof(long long) * pk.n, hipMemcpyDeviceToHost, st));
@@ -609,6 +616,11 @@ struct aimdhf_plan {
             qcount[k] = h_pin[2 * k + 2] - h_pin[2 * k];
         }
         qtotal = list_off[NQCLASS] = h_pin[2 * NQCLASS];
+        for (int k = 0; k < NQCLASS; ++k) {
+            const long long* h = h_pin + 2 * NQCLASS + 1 + list_parts * k;
+            h64count[k] = h[0] - list_off[k];
+            h32count[k] = list_parts == 2 ? h[1] - list_off[k] - q64count[k] : 0;
+        }
         d_lbra.ensure(sizeof(int) * std::max<long long>(qtotal, 1));
         d_lket.ensure(sizeof(int) * std::max<long long>(qtotal, 1));
         la.lbra = d_lbra.as<int>();
@@ -651,13 +663,13 @@ struct aimdhf_plan {
             ea.out64 = (double*)(d_store.as<char>() + base64[k]);
             ea.out32 = (float*)(d_store.as<char>() + base32[k]);
             hipStream_t s2 = fan.on(i++);
-            prof.time(47, s2, [&] { aimdhf::launch_eri(k, ea, q64count[k], qcount[k] - q64count[k], s2); });
+            prof.time(47, s2, [&] { aimdhf::launch_eri(k, ea, q64count[k], h64count[k], qcount[k] - q64count[k], h32count[k], s2); });
         }
         fan.join();
         HIPCHECK(hipGetLastError());
         // the digestion's view of the store (the stream was synchronised when the list was
         // built: no earlier copy from this pinned block is pending)
-        aimdhf::DigestGeo* geo = (aimdhf::DigestGeo*)(h_pin + 64);
+        aimdhf::DigestGeo* geo = (aimdhf::DigestGeo*)(h_pin + 128);
         for (int k = 0; k < NQCLASS; ++k) {
             geo[k].t64 = list_off[k];
             geo[k].t32 = list_off[k] + q64count[k];
@@ -997,6 +1009,13 @@ static int create_plan(int natm, int nshell, const int64_t* shell_atom, const in
                     const int dx = p->pair_a[x] - p->pair_b[x], dy = p->pair_a[y] - p->pair_b[y];
                     return dx != dy ? dx < dy : first[x] < first[y];
                 });
+            // in a batch the contracted pairs of a class come replica by replica: all of them
+            // count as contracted where any is
+            for (int c = 0; c < 6; ++c) {
+                int n = 0;
+                for (int x : bylcls[c]) n += nprim_of(first[x]) * nprim_of(second[x]) >= aimdhf::ERI_HEAVY;
+                p->nheavy[c] = p->batched && n > 0 ? (int)bylcls[c].size() : n;
+            }
         }
         p->cls_pair_off.assign(7, 0);
         p->ncls.assign(6, 0);

@@ -61,6 +61,8 @@ constexpr int NT_MAX = NT<double> > NT<float> ? NT<double> : NT<float>;
 // LDS words for the per-atom sums: with the 35 KB Boys slice, a workgroup stays
 // within 64 KB of LDS
 constexpr int GRAD_LDS_WORDS = 3600;
+// most parts a bra's (or, in a ket pass, a ket's) primitive pairs are cut into
+constexpr int MAXPART = pc_lo() == 0 || pc_hi() <= 1 ? (pc_hi() == 0 ? 16 : pc_hi() == 1 ? 8 : 4) : pc_hi() <= 3 ? 4 : 2;
 
 __device__ __forceinline__ void lds_add(long long* lds, int atom, int d, double x) {
     long long h, l;
@@ -208,10 +210,21 @@ __global__ __launch_bounds__(256) void k_grad_scatter(const unsigned char* __res
     if (k == 2) sel32[o2 + __popcll(m2 & below)] = (int)q;
 }
 
+// part `part` of np primitive pairs; false if it is empty
+__device__ __forceinline__ bool prim_part(int np, int part, int nparts, int& b0, int& nb) {
+    const int ch = (np + nparts - 1) / nparts;
+    b0 = part * ch;
+    nb = b0 + ch < np ? ch : np - b0;
+    return nb > 0;
+}
+
 // The folded item for ket columns KC0 .. KC0+FOLD<Real>-1 of quartet pq: A, B and C
 // derivatives from one pass, D by translational invariance
 template <int KC0, typename Real>
-__device__ __forceinline__ void fold_item(const GradArgs& a, int2 pq, const double* btab, long long* lds) {
+__device__ __forceinline__ void fold_item(const GradArgs& a, int2 pq, int part, int nparts, const double* btab,
+                                          long long* lds) {
+    int b0, nb;
+    if (!prim_part(a.npp[pq.x], part, nparts, b0, nb)) return;
     const int sA = a.pair_a[pq.x], sB = a.pair_b[pq.x], sC = a.pair_a[pq.y], sD = a.pair_b[pq.y];
     const int aA = a.shell_atom[sA], aB = a.shell_atom[sB], aC = a.shell_atom[sC], aD = a.shell_atom[sD];
     double deg = 0.5;
@@ -228,7 +241,7 @@ __device__ __forceinline__ void fold_item(const GradArgs& a, int2 pq, const doub
             gam[ab * F + c] =
                 Real(gamma_el(a, rep, oA + ab / NB, oB + ab % NB, oC + (KC0 + c) / ND, oD + (KC0 + c) % ND, deg));
     double gA[3], gB[3], gC[3];
-    grad_pass_c<LA, LB, LC, LD, F, KC0, true, Real>(a.recs + a.rec_off[pq.x], a.npp[pq.x],
+    grad_pass_c<LA, LB, LC, LD, F, KC0, true, Real>(a.recs + a.rec_off[pq.x] + (size_t)b0 * Qt::RSB, nb,
                                                        a.recs + a.rec_off[pq.y], a.npp[pq.y], btab, a.pos + 3 * aA,
                                                        a.pos + 3 * aB, a.pos + 3 * aC, aC != aD, gam, gA, gB, gC);
     for (int d = 0; d < 3; ++d) {
@@ -242,7 +255,7 @@ __device__ __forceinline__ void fold_item(const GradArgs& a, int2 pq, const doub
 // Work item = (selected quartet, pass column group), derivative integrals in Real
 template <int Q, typename Real>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(grad_waves<Real>()))) void k_grad_class(
-    GradArgs a, const int2* __restrict__ list, const int* __restrict__ sel, const int* __restrict__ nsel) {
+    GradArgs a, const int2* __restrict__ list, const int* __restrict__ sel, const int* __restrict__ nsel, int nparts) {
     extern __shared__ long long lds_acc[];
     __shared__ double btab[BOYS_NGRID * BOYS_SROW];
     // per-atom sums staged in LDS when they fit next to the Boys slice, else added
@@ -255,18 +268,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(grad_waves<
     // items wave by wave: the 64 lanes of a wave take 64 consecutive selected
     // quartets and one pass / column group, so the pass dispatch is uniform
     constexpr int NTR = NT<Real>;
-    const long long ns = *nsel, nitems = (ns + 63) / 64 * 64 * NTR;
+    const int ntp = NTR * nparts;
+    const long long ns = *nsel, nitems = (ns + 63) / 64 * 64 * ntp;
     for (long long it = (long long)blockIdx.x * blockDim.x + threadIdx.x; it < nitems;
          it += (long long)gridDim.x * blockDim.x) {
         const long long g = it >> 6;
-        const int j = (int)(g % NTR);
-        const long long qi = g / NTR * 64 + (it & 63);
+        const int jp = (int)(g % ntp), j = jp / nparts, part = jp - j * nparts;
+        const long long qi = g / ntp * 64 + (it & 63);
         if (qi >= ns) continue;
         const int2 pq = list[sel[qi]];
         if constexpr (FOLD<Real> > 0) {
             static_for<0, NTR>([&](auto jj) {
                 constexpr int J = decltype(jj)::value;
-                if (j == J) fold_item<J * FOLD<Real>, Real>(a, pq, btab, lds);
+                if (j == J) fold_item<J * FOLD<Real>, Real>(a, pq, part, nparts, btab, lds);
             });
             continue;
         }
@@ -284,6 +298,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(grad_waves<
         const size_t rep = a.shell_rep ? (size_t)a.shell_rep[sA] : 0;
         const double* rb = a.recs + a.rec_off[pq.x];
         const double* rk = a.recs + a.rec_off[pq.y];
+        int b0, nb;
+        if (!prim_part(a.npp[bra ? pq.x : pq.y], part, nparts, b0, nb)) continue;
         double g1[3], g2[3];
         if (bra) {
             const int kc0 = j * NCB;
@@ -293,7 +309,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(grad_waves<
                 for (int c = 0; c < NCB; ++c)
                     gam[ab * NCB + c] =
                         Real(gamma_el(a, rep, oA + ab / NB, oB + ab % NB, oC + (kc0 + c) / ND, oD + (kc0 + c) % ND, deg));
-            grad_pass<LA, LB, LC, LD, NCB, true, Real>(rb, a.npp[pq.x], rk, a.npp[pq.y], btab, a.pos + 3 * aA,
+            grad_pass<LA, LB, LC, LD, NCB, true, Real>(rb + (size_t)b0 * Qt::RSB, nb, rk, a.npp[pq.y], btab, a.pos + 3 * aA,
                                                        a.pos + 3 * aB, kc0, gam, g1, g2);
             for (int d = 0; d < 3; ++d) {
                 if (need_bra) {
@@ -313,7 +329,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(grad_waves<
                 for (int c = 0; c < NCK; ++c)
                     gam[cd * NCK + c] =
                         Real(gamma_el(a, rep, oA + (ab0 + c) / NB, oB + (ab0 + c) % NB, oC + cd / ND, oD + cd % ND, deg));
-            grad_pass<LC, LD, LA, LB, NCK, true, Real>(rk, a.npp[pq.y], rb, a.npp[pq.x], btab, a.pos + 3 * aC,
+            grad_pass<LC, LD, LA, LB, NCK, true, Real>(rk + (size_t)b0 * Qt::RSK, nb, rb, a.npp[pq.x], btab, a.pos + 3 * aC,
                                                        a.pos + 3 * aD, ab0, gam, g1, g2);
             for (int d = 0; d < 3; ++d) {
                 if (need_ket) {
@@ -351,14 +367,21 @@ void CAT(launch_grad_keep_, AIMDHF_QCLASS)(const GradArgs& a, const int2* list, 
 // FP64 items, then FP32 items (the grid is sized for the whole list; each kernel
 // reads its selection count on the device)
 void CAT(launch_grad_class_, AIMDHF_QCLASS)(const GradArgs& a, const int2* list, long long nq, hipStream_t st) {
+    // primitive parts per item: a lane's loop over a contracted quartet (36 x 36 for
+    // (ss|ss) in 6-31G*, 64 x 64 in cc-pVDZ) is what a small system waits for; with too few
+    // items to fill the card it is cut into parts (their sums are exact integers). Up to
+    // 16 parts, while the items stay below 16 wavefronts a CU
     long long items = nq * NT_MAX;
     if (items <= 0) return;
+    int nparts = 1;
+    while (nparts < MAXPART && items * nparts * 2 <= 262144) nparts *= 2;
+    items *= nparts;
     long long blocks = (items + 255) / 256;
     if (blocks > 1024) blocks = 1024;
     const size_t shm = 6 * a.natm <= GRAD_LDS_WORDS ? sizeof(long long) * 6 * a.natm : 0;
-    k_grad_class<QC, double><<<dim3((unsigned)blocks), dim3(256), shm, st>>>(a, list, a.sel64, a.nsel);
+    k_grad_class<QC, double><<<dim3((unsigned)blocks), dim3(256), shm, st>>>(a, list, a.sel64, a.nsel, nparts);
     if (a.fp32_switch > 0.0)
-        k_grad_class<QC, float><<<dim3((unsigned)blocks), dim3(256), shm, st>>>(a, list, a.sel32, a.nsel + 1);
+        k_grad_class<QC, float><<<dim3((unsigned)blocks), dim3(256), shm, st>>>(a, list, a.sel32, a.nsel + 1, nparts);
 }
 
 }  // namespace aimdhf

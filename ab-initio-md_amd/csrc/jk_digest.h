@@ -117,14 +117,17 @@ void launch_qlist_count(const QListArgs& a, hipStream_t st);
 void launch_qlist_fill(const QListArgs& a, hipStream_t st);
 void launch_list_scan(const long long* in, long long* out, long long n, long long* bsum, hipStream_t st);
 long long list_scan_blocks(long long n);
-// out[i] = off[at[i]] of n (<= 64) list cells, at by value
+// out[i] = off[at[i]] of n (<= 128) list cells, at by value
 struct PickArgs {
     int n;
-    long long at[64];
+    long long at[128];
 };
 void launch_pick(const PickArgs& a, const long long* off, long long* out, hipStream_t st);
 
-void launch_eri(int k, const EriArgs& a, long long n64, long long n32, hipStream_t st);
+// n64 FP64 quartets from the list position of a, n32 FP32 ones after them; the first h64 / h32
+// of each have contracted bras (ERI_HEAVY primitive pairs or more)
+constexpr int ERI_HEAVY = 6;
+void launch_eri(int k, const EriArgs& a, long long n64, long long h64, long long n32, long long h32, hipStream_t st);
 long long store_block(int k);       // integrals per block of quartet class k
 void launch_jk_prep(const PrepArgs& a, hipStream_t st);
 void launch_jk_finish(const PrepArgs& a, hipStream_t st);

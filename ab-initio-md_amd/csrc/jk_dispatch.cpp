@@ -67,19 +67,19 @@ void launch_kown(int type, const KOArgs& a, int nout, const int* has_l, hipStrea
     fns[type](a, nout, has_l, st);
 }
 
-#define DECLS(k) void launch_eri_##k(const EriArgs&, long long, long long, hipStream_t); \
+#define DECLS(k) void launch_eri_##k(const EriArgs&, long long, long long, long long, long long, hipStream_t); \
     void launch_digest_##k(const DigestArgs&, int, hipStream_t);
 DECLS(0) DECLS(1) DECLS(2) DECLS(3) DECLS(4) DECLS(5) DECLS(6) DECLS(7) DECLS(8) DECLS(9) DECLS(10)
 DECLS(11) DECLS(12) DECLS(13) DECLS(14) DECLS(15) DECLS(16) DECLS(17) DECLS(18) DECLS(19) DECLS(20)
 #undef DECLS
 
-void launch_eri(int k, const EriArgs& a, long long n64, long long n32, hipStream_t st) {
-    typedef void (*Fn)(const EriArgs&, long long, long long, hipStream_t);
+void launch_eri(int k, const EriArgs& a, long long n64, long long h64, long long n32, long long h32, hipStream_t st) {
+    typedef void (*Fn)(const EriArgs&, long long, long long, long long, long long, hipStream_t);
     static const Fn fns[21] = {
         launch_eri_0, launch_eri_1, launch_eri_2, launch_eri_3, launch_eri_4, launch_eri_5, launch_eri_6,
         launch_eri_7, launch_eri_8, launch_eri_9, launch_eri_10, launch_eri_11, launch_eri_12, launch_eri_13,
         launch_eri_14, launch_eri_15, launch_eri_16, launch_eri_17, launch_eri_18, launch_eri_19, launch_eri_20};
-    fns[k](a, n64, n32, st);
+    fns[k](a, n64, h64, n32, h32, st);
 }
 
 void launch_digest(int k, const DigestArgs& a, int threads, hipStream_t st) {

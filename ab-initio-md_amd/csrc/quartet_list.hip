@@ -238,7 +238,7 @@ void launch_list_scan(const long long* in, long long* out, long long n, long lon
 }
 
 void launch_pick(const PickArgs& a, const long long* off, long long* out, hipStream_t st) {
-    k_pick<<<dim3(1), dim3(64), 0, st>>>(a, off, out);
+    k_pick<<<dim3(1), dim3(128), 0, st>>>(a, off, out);
 }
 
 void launch_geo_bounds(const GeoArgs& a, hipStream_t st) {
