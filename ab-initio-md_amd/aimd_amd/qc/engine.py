@@ -220,11 +220,9 @@ class Engine:
 
     # ------------------------------------------------------------ profiling
     PAIR_CLASS_NAMES = ["ss", "ps", "pp", "ds", "dp", "dd"]
-    KIND_NAMES = ([f"jengine_bra_{c}" for c in PAIR_CLASS_NAMES]
-                  + [f"exchange_{'spd'[t // 3]}{'spd'[t % 3]}" for t in range(9)]
-                  + [f"unused_{k}" for k in range(15, 21)]
+    KIND_NAMES = ([f"unused_{k}" for k in range(21)]
                   + [f"grad_class_{k}" for k in range(21)]
-                  + ["geometry", "one_electron", "grad_one", "jk_prologue_epilogue", "jk_hermite_density",
+                  + ["geometry", "one_electron", "grad_one", "jk_prologue_epilogue", "direct_eri",
                      "eri_store"] + [f"unused_{k}" for k in range(48, 64)]
                   + [f"grad_screen_{k}" for k in range(21)]
                   + ["host_energy_list", "host_owner_lists", "host_store_build", "host_gradient_list"]
@@ -232,7 +230,7 @@ class Engine:
                   + ["jk_finish", "digest_all", "generic_jk", "generic_grad_two", "unused_97"]
                   + [f"digest_class_{k}" for k in range(21)])
     NKIND = 119
-    FOCK_KINDS = list(range(0, 15)) + [45, 46, 93, 94, 95] + list(range(98, 119))   # per-iteration J/K work
+    FOCK_KINDS = [45, 46, 93, 94, 95] + list(range(98, 119))   # per-iteration J/K work
     STORE_KINDS = [47]                                                  # per-geometry store build
     GRAD_KINDS = list(range(21, 42)) + list(range(64, 85)) + [96]       # derivative ERIs
 

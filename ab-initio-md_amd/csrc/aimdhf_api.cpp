@@ -226,18 +226,6 @@ struct aimdhf_plan {
     DevBuf d_recs, d_npp, d_qshell, d_qblock, d_qscr, d_counts, d_offsets, d_list;
     DevBuf d_fx, d_dsym, d_charges, d_glist, d_gfx, d_gden, d_scratch;
     std::vector<long long> gcount;
-    // owner-computes J/K: static output lists and per-geometry streams / partner lists
-    std::vector<int> out_x, out_y, ao_shell;
-    int out_off[10] = {0};
-    int has_l[3] = {0, 0, 0};
-    DevBuf d_out_x, d_out_y, d_ao_shell;
-    std::vector<int> ket_pair, ket_off, part_off, part_shell, part_pair, kpair;
-    std::vector<double> ket_q, part_q;
-    std::vector<long long> kpre, krec;
-    long long pbase[7] = {0}, dh_base2[7] = {0};
-    int nket[6] = {0};
-    DevBuf d_ket_q, d_kpre, d_krec, d_kpair, d_part_off, d_part_shell, d_part_pair, d_part_q;
-    DevBuf d_dh, d_jpart, d_kpart, d_ket_pair;
     // integral store: mode (0 auto, 1 direct, 2 store), byte limit (0: half the free device memory)
     int jk_mode = 0;
     long long store_limit = 0;
@@ -265,10 +253,6 @@ struct aimdhf_plan {
     double delta_fp32_max = 1e-3;   // accepted; every difference build sums in FP64
     DevBuf d_gdmax;                 // per shell pair density maxima for the gradient screening
     long long* h_pin = nullptr;     // pinned host words for the totals and the error flag
-    // pinned host staging of the per-geometry list transfers: asynchronous copies on
-    // the caller's stream, which do not wait for the integrals on the library streams
-    char* h_stage = nullptr;
-    size_t h_stage_cap = 0, h_stage_used = 0;
     // batched plans: independent molecules (replicas) sharing one plan; shells and
     // atoms grouped by replica, pairs and quartets only within a replica, matrices
     // in the padded layout (replica r's ld x ld block at r ld^2)
@@ -340,44 +324,12 @@ struct aimdhf_plan {
         return (long long)out.size();
     }
 
-    // make room for `bytes` of staging (no transfer may be pending) and start over
-    void stage_reset(size_t bytes) {
-        if (bytes > h_stage_cap) {
-            if (h_stage) HIPCHECK(hipHostFree(h_stage));
-            h_stage = nullptr;
-            h_stage_cap = 0;
-            const size_t want = bytes + bytes / 8 + 4096;
-            HIPCHECK(hipHostMalloc((void**)&h_stage, want));
-            h_stage_cap = want;
-        }
-        h_stage_used = 0;
-    }
-    char* stage_take(size_t bytes) {
-        const size_t at = h_stage_used;
-        h_stage_used += (bytes + 255) & ~(size_t)255;
-        if (h_stage_used > h_stage_cap) {
-            g_err = "staging buffer overflow";
-            throw HipError{AIMDHF_E_STATE};
-        }
-        return h_stage + at;
-    }
-    template <class T>
-    void upload_async(DevBuf& b, const std::vector<T>& v, hipStream_t st) {
-        b.ensure(sizeof(T) * std::max<size_t>(v.size(), 1));
-        if (v.empty()) return;
-        char* h = stage_take(sizeof(T) * v.size());
-        std::memcpy(h, v.data(), sizeof(T) * v.size());
-        HIPCHECK(hipMemcpyAsync(b.p, h, sizeof(T) * v.size(), hipMemcpyHostToDevice, st));
-    }
-
     ~aimdhf_plan() {
         for (DevBuf* b : {&d_shell_atom, &d_shell_l, &d_shell_prim, &d_shell_ao, &d_prim_exp, &d_prim_coef,
                           &d_pos, &d_pair_a, &d_pair_b, &d_pair_cls, &d_rec_size, &d_rec_off, &d_cls_pairs,
                           &d_cls_pair_off, &d_ncls, &d_bp_off, &d_bp_list, &d_boys, &d_recs, &d_npp,
                           &d_qshell, &d_qblock, &d_qscr, &d_counts, &d_offsets, &d_list, &d_fx, &d_dsym,
-                          &d_charges, &d_glist, &d_gfx, &d_gden, &d_scratch, &d_out_x, &d_out_y, &d_ao_shell,
-                          &d_ket_q, &d_kpre, &d_krec, &d_kpair, &d_part_off, &d_part_shell, &d_part_pair,
-                          &d_part_q, &d_dh, &d_jpart, &d_kpart, &d_ket_pair, &d_store, &d_oab, &d_rank_rep, &d_rep_shell,
+                          &d_charges, &d_glist, &d_gfx, &d_gden, &d_scratch, &d_store, &d_oab, &d_rank_rep, &d_rep_shell,
                           &d_seg, &d_rq, &d_gcell, &d_lcnt, &d_loff, &d_lsum, &d_lbra, &d_lket, &d_dket, &d_kacc,
                           &d_jacc, &d_dcell, &d_geo, &d_gkeep, &d_gsel, &d_nsel, &d_gblk,
                           &d_gdmax, &d_shell_rep, &d_shell_first,
@@ -385,7 +337,6 @@ struct aimdhf_plan {
                           &d_gpair_i, &d_gpair_j})
             b->release();
         if (h_pin) (void)hipHostFree(h_pin);
-        if (h_stage) (void)hipHostFree(h_stage);
     }
 
     aimdhf::PairArgs pair_args() const {
@@ -448,99 +399,6 @@ struct aimdhf_plan {
         buf.ensure(sizeof(int2) * std::max<long long>(total, 1));
         aimdhf::launch_fill_quartets(g, thr, sw, offs, base, buf.as<int2>(), st);
         HIPCHECK(hipGetLastError());
-    }
-
-    // Sorted ket streams (J-engine) and per-shell partner lists (exchange
-    // owners) from the screening values of the current geometry. Synchronous.
-    // direct: also the ket primitive records and Hermite-density layout the
-    // direct-mode J-engine streams (not needed when the integrals are stored)
-    void build_owner_lists(double thr, bool direct, hipStream_t st) {
-        HIPCHECK(hipStreamSynchronize(st));
-        stage_reset(12 * (size_t)npair + 512);
-        double* hq = (double*)stage_take(sizeof(double) * npair);
-        int* hn = (int*)stage_take(sizeof(int) * npair);
-        HIPCHECK(hipMemcpyAsync(hq, d_qscr.p, sizeof(double) * npair, hipMemcpyDeviceToHost, st));
-        HIPCHECK(hipMemcpyAsync(hn, d_npp.p, sizeof(int) * npair, hipMemcpyDeviceToHost, st));
-        HIPCHECK(hipStreamSynchronize(st));
-        std::vector<double> q(hq, hq + npair);
-        std::vector<int> np(hn, hn + npair);
-        double qmax = 0.0;
-        for (double v : q) qmax = std::max(qmax, v);
-        // kets by class, q descending (ties: pair index)
-        ket_pair.clear();
-        ket_q.clear();
-        ket_off.assign(7, 0);
-        for (int c = 0; c < 6; ++c) {
-            std::vector<int> ps(cls_pairs.begin() + cls_pair_off[c], cls_pairs.begin() + cls_pair_off[c + 1]);
-            std::stable_sort(ps.begin(), ps.end(), [&](int a, int b) { return q[a] > q[b] || (q[a] == q[b] && a < b); });
-            for (int P : ps) {
-                ket_pair.push_back(P);
-                ket_q.push_back(q[P]);
-            }
-            ket_off[c + 1] = (int)ket_pair.size();
-            nket[c] = ket_off[c + 1] - ket_off[c];
-        }
-        kpre.assign(ket_pair.size() + 1, 0);
-        krec.clear();
-        kpair.clear();
-        for (size_t m = 0; direct && m < ket_pair.size(); ++m) {
-            int P = ket_pair[m];
-            kpre[m + 1] = kpre[m] + np[P];
-            for (int k = 0; k < np[P]; ++k) {
-                krec.push_back(rec_off[P] + (long long)k * rec_size[P]);
-                kpair.push_back(P);
-            }
-        }
-        long long db = 0;
-        for (int c = 0; c < 6; ++c) {
-            int lc = c == 0 ? 0 : c <= 2 ? 1 : 2, ld = c - lc * (lc + 1) / 2;
-            pbase[c] = kpre[ket_off[c]];
-            dh_base2[c] = db;
-            db += (kpre[ket_off[c + 1]] - kpre[ket_off[c]]) * 2 * nherm(lc + ld);
-        }
-        pbase[6] = kpre[ket_off[6]];
-        dh_base2[6] = db;
-        // partner lists: shell X -> shells J of each l with q_XJ qmax >= thr (the exact
-        // test: no quartet of a pair failing it can pass q_P q_Q >= thr), q descending
-        part_off.assign(nshell * 3 + 1, 0);
-        part_shell.clear();
-        part_pair.clear();
-        part_q.clear();
-        std::vector<std::pair<double, int>> tmp;
-        for (int X = 0; X < nshell; ++X)
-            for (int l = 0; l < 3; ++l) {
-                tmp.clear();
-                for (int J = 0; J < nshell; ++J) {
-                    if (shell_l[J] != l) continue;
-                    int P = X >= J ? X * (X + 1) / 2 + J : J * (J + 1) / 2 + X;
-                    if (!(q[P] * qmax < thr)) tmp.push_back({q[P], J});
-                }
-                std::stable_sort(tmp.begin(), tmp.end(), [](const std::pair<double, int>& a, const std::pair<double, int>& b) {
-                    return a.first > b.first || (a.first == b.first && a.second < b.second);
-                });
-                for (auto& e : tmp) {
-                    int J = e.second;
-                    part_shell.push_back(J);
-                    part_pair.push_back(X >= J ? X * (X + 1) / 2 + J : J * (J + 1) / 2 + X);
-                    part_q.push_back(e.first);
-                }
-                part_off[X * 3 + l + 1] = (int)part_shell.size();
-            }
-        size_t bytes = 12 * ket_q.size() + 4 * part_off.size() + 16 * part_shell.size() + 8 * 1024;
-        if (direct) bytes += 8 * kpre.size() + 12 * krec.size();
-        stage_reset(bytes);   // the downloads above have completed
-        upload_async(d_ket_q, ket_q, st);
-        upload_async(d_ket_pair, ket_pair, st);
-        if (direct) {
-            upload_async(d_kpre, kpre, st);
-            upload_async(d_krec, krec, st);
-            upload_async(d_kpair, kpair, st);
-            d_dh.ensure(sizeof(double) * std::max<long long>(db, 1));
-        }
-        upload_async(d_part_off, part_off, st);
-        upload_async(d_part_shell, part_shell, st);
-        upload_async(d_part_pair, part_pair, st);
-        upload_async(d_part_q, part_q, st);
     }
 
     int matrix_ld() const { return batched ? bld : nao; }
@@ -649,19 +507,10 @@ struct aimdhf_plan {
     // Evaluate the screened quartets into the store.
     void build_store(hipStream_t st) {
         d_store.ensure(std::max<size_t>(store_need, 1));
-        aimdhf::EriArgs ea;
-        ea.recs = d_recs.as<double>();
-        ea.rec_off = d_rec_off.as<long long>();
-        ea.npp = d_npp.as<int>();
-        ea.cls_pairs = d_cls_pairs.as<int>();
-        ea.boys = d_boys.as<double>();
         fan.fork(st);
         for (int k = 0, i = 0; k < NQCLASS; ++k) {
             if (!qcount[k]) continue;
-            ea.lbra = d_lbra.as<int>() + list_off[k];
-            ea.lket = d_lket.as<int>() + list_off[k];
-            ea.out64 = (double*)(d_store.as<char>() + base64[k]);
-            ea.out32 = (float*)(d_store.as<char>() + base32[k]);
+            const aimdhf::EriArgs ea = eri_args(k, list_off[k]);
             hipStream_t s2 = fan.on(i++);
             prof.time(47, s2, [&] { aimdhf::launch_eri(k, ea, q64count[k], h64count[k], qcount[k] - q64count[k], h32count[k], s2); });
         }
@@ -673,6 +522,10 @@ struct aimdhf_plan {
         for (int k = 0; k < NQCLASS; ++k) {
             geo[k].t64 = list_off[k];
             geo[k].t32 = list_off[k] + q64count[k];
+            geo[k].lo64 = geo[k].t64;
+            geo[k].hi64 = geo[k].t32;
+            geo[k].lo32 = geo[k].t32;
+            geo[k].hi32 = list_off[k] + qcount[k];
             geo[k].off = d_loff.as<long long>() + runbase[k] * aimdhf::LIST_WAVES;
             geo[k].lket = d_lket.as<int>();
             geo[k].s64 = (const double*)(d_store.as<char>() + base64[k]);
@@ -682,6 +535,78 @@ struct aimdhf_plan {
         HIPCHECK(hipMemcpyAsync(d_geo.p, geo, sizeof(aimdhf::DigestGeo) * NQCLASS, hipMemcpyHostToDevice, st));
         store_bytes = (long long)store_need + 8 * qtotal;
         ensure_digest(1);
+    }
+
+    // Direct mode: the list cut into pieces whose integrals fit a bounded buffer (a class is
+    // split at multiples of 64 quartets); a J/K build evaluates and digests piece by piece
+    struct Piece {
+        long long lo[NQCLASS], hi[NQCLASS];
+        size_t at[NQCLASS];
+    };
+    std::vector<Piece> pieces;
+    void build_direct(hipStream_t) {
+        size_t fr = 0, tot = 0;
+        HIPCHECK(hipMemGetInfo(&fr, &tot));
+        size_t cap = std::min<size_t>((size_t)1 << 30, std::max<size_t>(fr / 8 + d_store.bytes, (size_t)1 << 20));
+        if (store_limit > 0) cap = std::min<size_t>(cap, std::max<size_t>((size_t)store_limit, (size_t)1 << 26));
+        pieces.clear();
+        Piece cur{};
+        size_t used = 0, most = 1;
+        for (int k = 0; k < NQCLASS; ++k) {
+            const size_t tile = sizeof(double) * 64 * (size_t)aimdhf::store_block(k);
+            long long pos = list_off[k], left = qcount[k];
+            while (left > 0) {
+                const long long room = (long long)((cap - used) / tile) * 64;
+                if (room == 0) {
+                    pieces.push_back(cur);
+                    cur = Piece{};
+                    used = 0;
+                    continue;
+                }
+                const long long n = std::min(left, room);
+                cur.lo[k] = pos;
+                cur.hi[k] = pos + n;
+                cur.at[k] = used;
+                used += (size_t)((n + 63) / 64) * tile;
+                most = std::max(most, used);
+                pos += n;
+                left -= n;
+                if (left > 0) {         // one range of a class per piece
+                    pieces.push_back(cur);
+                    cur = Piece{};
+                    used = 0;
+                }
+            }
+        }
+        if (used > 0) pieces.push_back(cur);
+        d_store.ensure(most);
+        std::vector<aimdhf::DigestGeo> geo(std::max<size_t>(pieces.size(), 1) * NQCLASS);
+        for (size_t c = 0; c < pieces.size(); ++c)
+            for (int k = 0; k < NQCLASS; ++k) {
+                aimdhf::DigestGeo& g = geo[c * NQCLASS + k];
+                g.t64 = g.lo64 = pieces[c].lo[k];
+                g.hi64 = g.t32 = g.lo32 = g.hi32 = pieces[c].hi[k];
+                g.off = d_loff.as<long long>() + runbase[k] * aimdhf::LIST_WAVES;
+                g.lket = d_lket.as<int>();
+                g.s64 = (const double*)(d_store.as<char>() + pieces[c].at[k]);
+                g.s32 = nullptr;
+            }
+        upload(d_geo, geo);             // the stream was synchronised when the list was built
+        ensure_digest(1);
+    }
+
+    aimdhf::EriArgs eri_args(int k, long long lo) const {
+        aimdhf::EriArgs ea;
+        ea.recs = d_recs.as<double>();
+        ea.rec_off = d_rec_off.as<long long>();
+        ea.npp = d_npp.as<int>();
+        ea.cls_pairs = d_cls_pairs.as<int>();
+        ea.boys = d_boys.as<double>();
+        ea.lbra = d_lbra.as<int>() + lo;
+        ea.lket = d_lket.as<int>() + lo;
+        ea.out64 = (double*)(d_store.as<char>() + base64[k]);
+        ea.out32 = (float*)(d_store.as<char>() + base32[k]);
+        return ea;
     }
 
     // copies of the global J/K accumulators: one per XCD where the matrices are few
@@ -1066,30 +991,7 @@ static int create_plan(int natm, int nshell, const int64_t* shell_atom, const in
             p->bp_off[i + 1] = p->bp_off[i] + (int)bpl[i].size();
             p->bp_list.insert(p->bp_list.end(), bpl[i].begin(), bpl[i].end());
         }
-        // exchange output blocks (X >= Y) grouped by (l_X, l_Y); a batch digests its dense
-        // tensors instead and needs neither these nor the AO -> shell map
-        if (!p->batched) {
-            std::vector<std::vector<int>> ox(9), oy(9);
-            for (int X = 0; X < nshell; ++X)
-                for (int Y = 0; Y <= X; ++Y) {
-                    int t = p->shell_l[X] * 3 + p->shell_l[Y];
-                    ox[t].push_back(X);
-                    oy[t].push_back(Y);
-                }
-            for (int t = 0; t < 9; ++t) {
-                p->out_off[t + 1] = p->out_off[t] + (int)ox[t].size();
-                p->out_x.insert(p->out_x.end(), ox[t].begin(), ox[t].end());
-                p->out_y.insert(p->out_y.end(), oy[t].begin(), oy[t].end());
-            }
-            for (int s2 = 0; s2 < nshell; ++s2) p->has_l[p->shell_l[s2]] = 1;
-            p->ao_shell.resize(p->shell_ao[nshell]);
-            for (int s2 = 0; s2 < nshell; ++s2)
-                for (int i = p->shell_ao[s2]; i < p->shell_ao[s2 + 1]; ++i) p->ao_shell[i] = s2;
-        }
         // device copies
-        upload(p->d_out_x, p->out_x);
-        upload(p->d_out_y, p->out_y);
-        upload(p->d_ao_shell, p->ao_shell);
         upload(p->d_shell_atom, p->shell_atom);
         upload(p->d_shell_l, p->shell_l);
         upload(p->d_shell_prim, p->shell_prim);
@@ -1313,7 +1215,9 @@ int aimdhf_set_geometry(aimdhf_plan* p, const double* positions, double thr, voi
         });
         HIPCHECK(hipGetLastError());
         auto t0 = Profiler::clock::now();
-        p->build_quartets(thr, p->precision == 1 && p->jk_switch > thr ? p->jk_switch : 0.0, st);
+        // direct mode evaluates in FP64 throughout
+        const double sw = p->precision == 1 && p->jk_switch > thr ? p->jk_switch : 0.0;
+        p->build_quartets(thr, p->jk_mode == 1 && !p->batched ? 0.0 : sw, st);
         p->threshold = thr;
         p->prof.host(85, t0);
         p->stored = false;
@@ -1326,7 +1230,11 @@ int aimdhf_set_geometry(aimdhf_plan* p, const double* positions, double thr, voi
             return AIMDHF_OK;
         }
         bool store = false;
-        if (p->jk_mode != 1 && p->nao < (1 << 14)) {
+        if (p->nao >= (1 << 14)) {
+            p->have_geometry = false;
+            return fail(AIMDHF_E_UNSUPPORTED, "more than 16383 AOs");
+        }
+        if (p->jk_mode != 1) {
             long long limit = p->store_limit;
             if (limit <= 0) {
                 size_t fr = 0, tot = 0;
@@ -1337,7 +1245,8 @@ int aimdhf_set_geometry(aimdhf_plan* p, const double* positions, double thr, voi
         }
         if (!store) {
             t0 = Profiler::clock::now();
-            p->build_owner_lists(thr, true, st);
+            if (p->list_parts == 2) p->build_quartets(thr, 0.0, st);
+            p->build_direct(st);
             p->prof.host(86, t0);
         } else {
             auto t1 = Profiler::clock::now();
@@ -1485,105 +1394,47 @@ int aimdhf_jk_delta(aimdhf_plan* p, int nset, const double* ddens, double* dJ, d
     return jk_from_store(p, nset, ddens, dJ, dK, true, threshold, (hipStream_t)stream);
 }
 
-int aimdhf_jk(aimdhf_plan* p, int nset, const double* dens, double* J, double* K, void* stream) {
-    if (!p || !dens || !J || !K) return fail(AIMDHF_E_ARG, "NULL argument");
-    if (nset < 1 || nset > 2) return fail(AIMDHF_E_ARG, "nset must be 1 or 2");
-    if (!p->have_geometry) return fail(AIMDHF_E_STATE, "no geometry set");
-    hipStream_t st = (hipStream_t)stream;
-    if (p->batched) return jk_from_store(p, nset, dens, J, K, false, 0.0, st);
-    if (p->generic) return jk_generic(p, nset, dens, J, K, st);
-    if (p->stored) return jk_from_store(p, nset, dens, J, K, false, 0.0, st);
+// J and K with the integrals evaluated piece by piece (direct mode)
+static int jk_direct(aimdhf_plan* p, int nset, const double* dens, double* J, double* K, hipStream_t st) {
     try {
-        const size_t nn = (size_t)p->nao * p->nao;
-        p->d_dsym.ensure(sizeof(double) * nset * nn);
-        p->d_jpart.ensure(sizeof(double) * 6 * (size_t)p->npair * nset * 36);
-        p->d_kpart.ensure(sizeof(double) * 9 * nset * nn);
-        p->prof.time(45, st, [&] {
-            aimdhf::launch_symmetrize(dens, nset, p->nao, p->d_dsym.as<double>(), st);
-            aimdhf::launch_zero_d(p->d_kpart.as<double>(), 9 * nset * nn, st);
-        });
-        // J-engine: Hermite densities of the ket streams, then one kernel per (bra class, ket class)
-        aimdhf::DhArgs dh;
-        dh.nao = p->nao;
-        dh.nset = nset;
-        long long ncls_entries[6];
-        for (int c = 0; c < 6; ++c) {
-            dh.pbase[c] = p->pbase[c];
-            dh.dh_base[c] = p->dh_base2[c];
-            ncls_entries[c] = p->pbase[c + 1] - p->pbase[c];
+        p->ensure_digest(nset);
+        const aimdhf::PrepArgs pa = p->prep_args(nset, dens, J, K);
+        p->prof.time(45, st, [&] { aimdhf::launch_jk_prep(pa, st); });
+        for (size_t c = 0; c < p->pieces.size(); ++c) {
+            const aimdhf_plan::Piece& pc = p->pieces[c];
+            // a class is digested on the stream that evaluates it; the pieces share the buffer
+            p->fan.fork(st);
+            int i = 0;
+            for (int k = NQCLASS - 1; k >= 0; --k) {
+                const long long n = pc.hi[k] - pc.lo[k];
+                if (n <= 0) continue;
+                hipStream_t s2 = p->fan.on(i++);
+                aimdhf::EriArgs ea = p->eri_args(k, pc.lo[k]);
+                ea.out64 = (double*)(p->d_store.as<char>() + pc.at[k]);
+                const long long h = p->list_off[k] + p->h64count[k] - pc.lo[k];
+                p->prof.time(46, s2, [&] { aimdhf::launch_eri(k, ea, n, std::min(std::max(h, 0LL), n), 0, 0, s2); });
+                aimdhf::DigestArgs da = p->digest_args(k, nset, false, 0.0);
+                da.geo += c * NQCLASS;
+                p->prof.time(98 + k, s2, [&] { aimdhf::launch_digest(k, da, 256, s2); });
+            }
+            p->fan.join();
         }
-        dh.krec = p->d_krec.as<long long>();
-        dh.kpair = p->d_kpair.as<int>();
-        dh.pair_a = p->d_pair_a.as<int>();
-        dh.pair_b = p->d_pair_b.as<int>();
-        dh.shell_ao = p->d_shell_ao.as<int>();
-        dh.recs = p->d_recs.as<double>();
-        dh.dens = p->d_dsym.as<double>();
-        dh.dh = p->d_dh.as<double>();
-        p->prof.time(46, st, [&] { aimdhf::launch_dh(dh, ncls_entries, st); });
-        aimdhf::JEArgs je;
-        je.npair = p->npair;
-        je.thr = p->threshold;
-        je.cls_pairs = p->d_cls_pairs.as<int>();
-        je.cls_pair_off = p->d_cls_pair_off.as<int>();
-        for (int c = 0; c < 6; ++c) je.ncls_host[c] = p->ncls[c];
-        je.qscr = p->d_qscr.as<double>();
-        je.ket_q = p->d_ket_q.as<double>();
-        for (int c = 0; c < 7; ++c) je.ket_off[c] = p->ket_off[c];
-        je.kpre = p->d_kpre.as<long long>();
-        je.krec = p->d_krec.as<long long>();
-        je.dh = p->d_dh.as<double>();
-        for (int c = 0; c < 6; ++c) je.dh_base[c] = p->dh_base2[c];
-        je.recs = p->d_recs.as<double>();
-        je.rec_off = p->d_rec_off.as<long long>();
-        je.npp = p->d_npp.as<int>();
-        je.boys = p->d_boys.as<double>();
-        je.jpart = p->d_jpart.as<double>();
-        for (int c = 0; c < 6; ++c)
-            if (p->ncls[c] > 0) p->prof.time(c, st, [&] { aimdhf::launch_jeng(c, je, nset, p->nket, st); });
-        aimdhf::JAsmArgs ja;
-        ja.npair = p->npair;
-        ja.nao = p->nao;
-        ja.nset = nset;
-        for (int c = 0; c < 6; ++c) ja.cq_valid[c] = p->nket[c] > 0;
-        ja.pair_a = p->d_pair_a.as<int>();
-        ja.pair_b = p->d_pair_b.as<int>();
-        ja.shell_ao = p->d_shell_ao.as<int>();
-        ja.jpart = p->d_jpart.as<double>();
-        ja.J = J;
-        p->prof.time(45, st, [&] { aimdhf::launch_j_assemble(ja, st); });
-        // exchange owners: one kernel per (l_X, l_Y, l_J, l_L)
-        aimdhf::KOArgs ko;
-        ko.nao = p->nao;
-        ko.nset = nset;
-        ko.thr = p->threshold;
-        for (int t = 0; t < 10; ++t) ko.out_off[t] = p->out_off[t];
-        ko.out_x = p->d_out_x.as<int>();
-        ko.out_y = p->d_out_y.as<int>();
-        ko.part_off = p->d_part_off.as<int>();
-        ko.part_shell = p->d_part_shell.as<int>();
-        ko.part_pair = p->d_part_pair.as<int>();
-        ko.part_q = p->d_part_q.as<double>();
-        ko.pair_a = p->d_pair_a.as<int>();
-        ko.rec_off = p->d_rec_off.as<long long>();
-        ko.recs = p->d_recs.as<double>();
-        ko.npp = p->d_npp.as<int>();
-        ko.shell_ao = p->d_shell_ao.as<int>();
-        ko.boys = p->d_boys.as<double>();
-        ko.dens = p->d_dsym.as<double>();
-        ko.kpart = p->d_kpart.as<double>();
-        for (int t = 0; t < 9; ++t) {
-            int nout = p->out_off[t + 1] - p->out_off[t];
-            if (nout > 0) p->prof.time(6 + t, st, [&] { aimdhf::launch_kown(t, ko, nout, p->has_l, st); });
-        }
-        p->prof.time(45, st, [&] {
-            aimdhf::launch_k_assemble(p->d_kpart.as<double>(), nset, p->nao, p->d_ao_shell.as<int>(), K, st);
-        });
+        p->prof.time(93, st, [&] { aimdhf::launch_jk_finish(pa, st); });
         HIPCHECK(hipGetLastError());
     } catch (const HipError& e) {
         return e.code;
     }
     return AIMDHF_OK;
+}
+
+int aimdhf_jk(aimdhf_plan* p, int nset, const double* dens, double* J, double* K, void* stream) {
+    if (!p || !dens || !J || !K) return fail(AIMDHF_E_ARG, "NULL argument");
+    if (nset < 1 || nset > 2) return fail(AIMDHF_E_ARG, "nset must be 1 or 2");
+    if (!p->have_geometry) return fail(AIMDHF_E_STATE, "no geometry set");
+    hipStream_t st = (hipStream_t)stream;
+    if (p->generic) return jk_generic(p, nset, dens, J, K, st);
+    if (p->batched || p->stored) return jk_from_store(p, nset, dens, J, K, false, 0.0, st);
+    return jk_direct(p, nset, dens, J, K, st);
 }
 
 int aimdhf_one_electron(aimdhf_plan* p, double* S, double* T, double* V, double* M, void* stream) {

@@ -50,7 +50,8 @@ constexpr int OAB_SAME = 1 << 28;
 // What of a digestion depends on the geometry; read from device memory, so a captured
 // launch stays valid when the geometry moves (batched SCF iterations are replayed)
 struct DigestGeo {
-    long long t64, t32;             // list index where the class's FP64 and FP32 parts start
+    long long t64, t32;             // list index of the first FP64 and FP32 block
+    long long lo64, hi64, lo32, hi32;   // list ranges that are held (direct mode: a piece of the list)
     const long long* off;           // list offsets of the class's runs (LIST_WAVES apart)
     const int* lket;
     const double* s64;              // the class's blocks, FP64 part

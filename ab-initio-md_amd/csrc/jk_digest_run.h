@@ -206,6 +206,9 @@ __device__ __forceinline__ void digest_run(const DigestArgs& a, int bi, int part
     const long long run = (long long)part * nb + bi;
     const DigestGeo g = a.geo[QC];
     long long t0 = g.off[run * LIST_WAVES], t1 = g.off[(run + 1) * LIST_WAVES];
+    const long long lo = part ? g.lo32 : g.lo64, hi = part ? g.hi32 : g.hi64;
+    if (t0 < lo) t0 = lo;
+    if (t1 > hi) t1 = hi;
     if (a.nchunk > 1) {
         long long per = (t1 - t0 + a.nchunk - 1) / a.nchunk;
         if (per < a.unit) per = a.unit;

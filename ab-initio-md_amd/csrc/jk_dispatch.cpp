@@ -47,26 +47,6 @@ void launch_grad(const GradArgs& a, const int2* const* lists, const long long* c
     for (int k = 0; k < 21; ++k) fns[k](a, lists[k], counts[k], st);
 }
 
-#define DECLJ(k) void launch_jeng_##k(const JEArgs&, int, const int*, hipStream_t);
-DECLJ(0) DECLJ(1) DECLJ(2) DECLJ(3) DECLJ(4) DECLJ(5)
-#undef DECLJ
-#define DECLK(x, y) void launch_kown_##x##_##y(const KOArgs&, int, const int*, hipStream_t);
-DECLK(0, 0) DECLK(0, 1) DECLK(0, 2) DECLK(1, 0) DECLK(1, 1) DECLK(1, 2) DECLK(2, 0) DECLK(2, 1) DECLK(2, 2)
-#undef DECLK
-
-void launch_jeng(int pclass, const JEArgs& a, int nset, const int* nket_host, hipStream_t st) {
-    typedef void (*Fn)(const JEArgs&, int, const int*, hipStream_t);
-    static const Fn fns[6] = {launch_jeng_0, launch_jeng_1, launch_jeng_2, launch_jeng_3, launch_jeng_4, launch_jeng_5};
-    fns[pclass](a, nset, nket_host, st);
-}
-
-void launch_kown(int type, const KOArgs& a, int nout, const int* has_l, hipStream_t st) {
-    typedef void (*Fn)(const KOArgs&, int, const int*, hipStream_t);
-    static const Fn fns[9] = {launch_kown_0_0, launch_kown_0_1, launch_kown_0_2, launch_kown_1_0, launch_kown_1_1,
-                              launch_kown_1_2, launch_kown_2_0, launch_kown_2_1, launch_kown_2_2};
-    fns[type](a, nout, has_l, st);
-}
-
 #define DECLS(k) void launch_eri_##k(const EriArgs&, long long, long long, long long, long long, hipStream_t); \
     void launch_digest_##k(const DigestArgs&, int, hipStream_t);
 DECLS(0) DECLS(1) DECLS(2) DECLS(3) DECLS(4) DECLS(5) DECLS(6) DECLS(7) DECLS(8) DECLS(9) DECLS(10)

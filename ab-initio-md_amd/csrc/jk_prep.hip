@@ -3,6 +3,7 @@
 // the cleared accumulators before it (one launch), J and K from the
 // accumulators after it (one launch).
 
+#include "aimdhf_internal.h"
 #include "jk_digest.h"
 
 namespace aimdhf {
@@ -147,7 +148,16 @@ __global__ void k_clear_cells(unsigned long long* p, int n) {
     if (i < n) p[i] = 0ull;
 }
 
+__global__ void k_zero_d(double* p, size_t n) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = 0.0;
+}
+
 }  // namespace
+
+void launch_zero_d(double* p, size_t n, hipStream_t st) {
+    if (n) k_zero_d<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st>>>(p, n);
+}
 
 void launch_jk_prep(const PrepArgs& a, hipStream_t st) {
     const int ncell = JK_CELLS * a.nrep * a.nset;

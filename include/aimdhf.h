@@ -121,11 +121,11 @@ int aimdhf_quartets(aimdhf_plan* plan, int64_t* out_host, int64_t cap, int64_t* 
  * Coulomb and exchange matrices of nset densities (device (nset,nao,nao)):
  *   J_mn = sum_ls (mn|ls) D_ls,   K_mn = sum_ls (ml|ns) D_ls
  * of the symmetric part of each D over the screened quartets, bitwise
- * reproducible run to run. Direct mode recomputes the integrals (J-engine in
- * Hermite space for J, per-block exchange owners for K), every output block
- * owned by one wavefront; store mode reads each stored integral once and sums in
- * 64-bit fixed point whose exponent follows the density and the Schwarz bounds
- * (resolution 2^-62 of a bound of the largest element; a density with a NaN or
+ * reproducible run to run. Store mode reads each stored integral once, direct
+ * mode evaluates the list piece by piece into a bounded buffer (at most 1 GiB, an
+ * eighth of the free memory, or max_store_bytes if that is set and above 64 MiB)
+ * and digests each piece; sums are 64-bit fixed point whose exponent follows the
+ * density and the Schwarz bounds (resolution 2^-62 of a bound of the largest element; a density with a NaN or
  * infinity gives NaN in its J and K).
  * Replaces: jk_from_eri (aimd/qc/integrals.py:1009-1044) and, in direct mode,
  * eri_tensor (aimd/qc/integrals.py:986-1006).
@@ -315,11 +315,10 @@ int aimdhf_grad_two(aimdhf_plan* plan, const double* Dc, int nx, const double* D
 /*
  * Kernel timing with HIP events recorded on the caller's stream around every
  * launch while enabled (no counterpart in the reference, whose timings are
- * wall-clock dicts, aimd/backends/hf.py:347-354). Kinds: 0..5 direct J-engine
- * per bra pair class (ss ps pp ds dp dd), 6..14 direct exchange per output
- * type (l_X, l_Y), 21..41 derivative-ERI kernels of the 21 quartet classes,
- * 42 geometry set-up, 43 one-electron integrals, 44 one-electron gradient,
- * 45 J/K prologue and epilogue, 46 Hermite densities, 47 integral store
+ * wall-clock dicts, aimd/backends/hf.py:347-354). Kinds: 21..41
+ * derivative-ERI kernels of the 21 quartet classes, 42 geometry set-up, 43
+ * one-electron integrals, 44 one-electron gradient, 45 J/K prologue, 46 direct
+ * mode's integral evaluation, 47 integral store
  * evaluation, 64..84 derivative-ERI screening pre-pass per class; 85..88 host
  * wall-clock phases (energy list, owner lists, store build incl. its device
  * work, gradient list; milliseconds of the calling thread, not events), 93 J/K

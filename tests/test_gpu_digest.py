@@ -123,3 +123,30 @@ def test_replicas_stay_apart():
         assert torch.equal(batch.J[r], J[r]) and torch.equal(batch.K[r], K[r])
     assert torch.isnan(batch.J[1, 0, :25, :25]).all()
     batch.close()
+
+
+@pytest.mark.parametrize("nset", [1, 2])
+def test_direct_in_pieces(oracle_lib, nset):
+    """Direct mode with its buffer held to 64 MiB (eight waters take several hundred MB, so
+    runs and classes are cut between pieces) against the oracle (1e-11, as the other J/K
+    tests); a difference build and mixed precision change nothing in direct mode."""
+    import torch
+    from tests.conftest import cluster
+    s, x = cluster("water8.xyz")
+    e = _engine(s, x, "6-31g*", "store")
+    assert e.jk_info()["gather_bytes"] > 3 * (64 << 20)
+    D = _dens(e.nao, nset, 5)
+    e.set_jk_mode("direct", 1)
+    e.set_geometry(x)
+    assert not e.jk_info()["stored"]
+    ref = e.jk(D)
+    Jo, Ko = oracle_lib.Pairs(oracle_lib.make_basis(s, x, "6-31g*")).jk_direct(D.cpu().numpy())
+    np.testing.assert_allclose(ref[0].cpu().numpy(), Jo, rtol=0, atol=1e-11)
+    np.testing.assert_allclose(ref[1].cpu().numpy(), Ko, rtol=0, atol=1e-11)
+    for a, b in zip(ref, e.jk_delta(D, 1e-3)):
+        assert torch.equal(a, b)
+    e.set_precision("mixed", 1e-5, 1e-5, 1e-2)
+    e.set_geometry(x)
+    for a, b in zip(ref, e.jk(D)):
+        assert torch.equal(a, b)
+    e.close()
