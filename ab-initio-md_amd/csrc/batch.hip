@@ -15,100 +15,153 @@ namespace {
 // Trace-correcting purification of nmat symmetric ld x ld matrices (ld <= 64), one
 // workgroup per matrix held in LDS for all steps: X0 = (e_max - F) / (e_max -
 // e_min) with F's Gershgorin bounds, then X <- X^2 if tr X > nocc else 2X - X^2,
-// an iterate with |tr X - tr X^2| < tol held (more steps would amplify its
-// rounding errors), and two final unheld steps that square the remaining error.
-// err[i] receives the idempotency error |tr X - tr X^2| before those two steps.
+// up to `steps` times while |tr X - tr X^2| >= tol (more steps would amplify the
+// rounding errors), and two final steps that square the remaining error. err[i]
+// receives the idempotency error |tr X - tr X^2| before those two steps.
 //
 // X^2 on the matrix cores: X sits zero-padded to 64 x 64 in LDS (row stride 65
-// doubles, so the 16 rows one operand load touches fall in distinct banks);
-// wavefront w forms the 16 x 64 row block w of X^2 as four 16 x 16 tiles, each
-// 16 steps of v_mfma_f64_16x16x4f64 over k. Operand and result lanes (measured on
-// gfx950): A(i, k) from lane i + 16 k, B(k, j) from lane j + 16 k, D(i, j) in
-// register i / 4 of lane j + 16 (i % 4). Each result element has one owner lane,
-// which applies the update.
+// doubles, so the 16 rows one operand load touches fall in distinct banks); the
+// 16 x 16 tiles of its upper triangle, up to ceil(ld / 16) a side, go round the four
+// wavefronts (10 tiles, 3 at most in one, at ld > 48) and are written on both sides,
+// each 4 ceil(ld / 16) steps of v_mfma_f64_16x16x4f64 over k. Operand and result
+// lanes (measured on gfx950): A(i, k) from lane i + 16 k, B(k, j) from lane j + 16 k,
+// D(i, j) in register i / 4 of lane j + 16 (i % 4). Both traces are summed by every
+// wavefront for itself in DPP steps, so a step has two barriers.
+// Bound by the serial chain of steps, each the MFMA issue of one CU (1.3 us of 64 x 64)
+// and the latencies of LDS and barriers: 24 matrices of 50 orbitals 268 -> 201 us (full
+// tiles, six barriers and all 62 steps before), one of 19 orbitals 99 -> 56 us.
 constexpr int PUR_THREADS = 256;
 constexpr int PUR_MAXLD = 64;
 constexpr int PUR_LS = PUR_MAXLD + 1;       // LDS row stride (doubles)
+constexpr int PUR_TILES = 3;                // tiles of one wavefront
 
 typedef double v4d __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ double block_sum(double v, double* red) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    return red[0] + red[1] + red[2] + red[3];
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+    return v + __hiloint2double(hi, lo);
+}
+
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// Sum over the wavefront: neighbours, pairs, half rows and rows of 16 lanes, then the four rows
+__device__ __forceinline__ double wave_sum(double v) {
+    v = dpp_add<0xB1>(v);               // quad_perm 1 0 3 2
+    v = dpp_add<0x4E>(v);               // quad_perm 2 3 0 1
+    v = dpp_add<0x141>(v);              // row_half_mirror
+    v = dpp_add<0x140>(v);              // row_mirror
+    return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
 }
 
 __global__ __launch_bounds__(PUR_THREADS) void k_batch_purify(int ld, const double* __restrict__ F,
                                                               const double* __restrict__ nocc, double* __restrict__ P,
                                                               int steps, double tol, double* __restrict__ err) {
     __shared__ double X[PUR_MAXLD * PUR_LS];
-    __shared__ double red[4], lo[4], hi[4];
+    __shared__ double diag2[PUR_MAXLD];
     const int mat = blockIdx.x, t = threadIdx.x, n2 = ld * ld;
+    const int w = t >> 6, lane = t & 63, li = lane & 15, lk = lane >> 4;
+    const int nt = (ld + 15) / 16, ntile = nt * (nt + 1) / 2;
     const double* Fm = F + (size_t)mat * n2;
-    // Gershgorin bounds, thread per row (min / max do not depend on the order)
+    // all loads of F in flight at once, then symmetrised in place
+    double f[16];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int i = 16 * r + (t >> 4), j = 16 * c + (t & 15);
+            f[4 * r + c] = i < ld && j < ld ? Fm[i * ld + j] : 0.0;
+        }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) X[(16 * r + (t >> 4)) * PUR_LS + 16 * c + (t & 15)] = f[4 * r + c];
+    if (t < PUR_MAXLD) diag2[t] = 0.0;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            f[4 * r + c] = 0.5 * (f[4 * r + c] + X[(16 * c + (t & 15)) * PUR_LS + 16 * r + (t >> 4)]);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) X[(16 * r + (t >> 4)) * PUR_LS + 16 * c + (t & 15)] = f[4 * r + c];
+    __syncthreads();
+    // Gershgorin bounds, lane per row, each wavefront for itself (min / max do not depend on the order)
     double mn = 1e300, mx = -1e300;
-    for (int i = t; i < ld; i += PUR_THREADS) {
+    if (lane < ld) {
         double r = 0.0;
-        for (int j = 0; j < ld; ++j) r += j == i ? 0.0 : fabs(Fm[i * ld + j]);
-        mn = fmin(mn, Fm[i * ld + i] - r);
-        mx = fmax(mx, Fm[i * ld + i] + r);
+        const double d = X[lane * PUR_LS + lane];
+#pragma unroll 8
+        for (int j = 0; j < ld; ++j) r += j == lane ? 0.0 : fabs(X[lane * PUR_LS + j]);
+        mn = d - r;
+        mx = d + r;
     }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) {
         mn = fmin(mn, __shfl_xor(mn, o, 64));
         mx = fmax(mx, __shfl_xor(mx, o, 64));
     }
-    if ((t & 63) == 0) {
-        lo[t >> 6] = mn;
-        hi[t >> 6] = mx;
-    }
+    const double inv = 1.0 / (mx - mn);
     __syncthreads();
-    const double emin = fmin(fmin(lo[0], lo[1]), fmin(lo[2], lo[3]));
-    const double emax = fmax(fmax(hi[0], hi[1]), fmax(hi[2], hi[3]));
-    const double inv = 1.0 / (emax - emin);
-    for (int e = t; e < PUR_MAXLD * PUR_LS; e += PUR_THREADS) {
-        const int i = e / PUR_LS, j = e % PUR_LS;
-        X[e] = (i < ld && j < ld) ? ((i == j ? emax : 0.0) - Fm[i * ld + j]) * inv : 0.0;
-    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int i = 16 * r + (t >> 4), j = 16 * c + (t & 15);
+            X[i * PUR_LS + j] = i < ld && j < ld ? ((i == j ? mx : 0.0) - f[4 * r + c]) * inv : 0.0;
+        }
     __syncthreads();
     const double ne = nocc[mat];
-    const int w = t >> 6, lane = t & 63, li = lane & 15, lk = lane >> 4;
-    const int row0 = 16 * w + lk;                   // rows row0 + 4 v (v < 4) of the lane's results
+    // the wavefront's tiles w, w + 4, w + 8 of the upper triangle (row by row)
+    int ti[PUR_TILES], tj[PUR_TILES];
+#pragma unroll
+    for (int s = 0; s < PUR_TILES; ++s) {
+        int q = w + 4 * s, i = 0;
+        while (i < nt && q >= nt - i) q -= nt - i++;
+        ti[s] = __builtin_amdgcn_readfirstlane(i);
+        tj[s] = __builtin_amdgcn_readfirstlane(i + q);
+    }
+    const int mine = __builtin_amdgcn_readfirstlane(w < ntile ? (ntile - w + 3) / 4 : 0);
     double last = 0.0;
     for (int it = 0; it < steps + 2; ++it) {
-        v4d acc[4];
+        v4d acc[PUR_TILES];
 #pragma unroll
-        for (int tj = 0; tj < 4; ++tj) acc[tj] = v4d{0.0, 0.0, 0.0, 0.0};
+        for (int s = 0; s < PUR_TILES; ++s) acc[s] = v4d{0.0, 0.0, 0.0, 0.0};
 #pragma unroll 4
-        for (int k0 = 0; k0 < PUR_MAXLD; k0 += 4) {
-            const double a = X[(16 * w + li) * PUR_LS + k0 + lk];
+        for (int k0 = 0; k0 < 16 * nt; k0 += 4)
 #pragma unroll
-            for (int tj = 0; tj < 4; ++tj) {
-                const double b = X[(k0 + lk) * PUR_LS + 16 * tj + li];
-                acc[tj] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[tj], 0, 0, 0);
-            }
-        }
-        // traces: the diagonal of X, and of X^2 in the wavefront's diagonal tile
-        double dx = 0.0, dx2 = 0.0;
-        if (t < PUR_MAXLD) dx = X[t * PUR_LS + t];
+            for (int s = 0; s < PUR_TILES; ++s)
+                if (s < mine)
+                    acc[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(X[(16 * ti[s] + li) * PUR_LS + k0 + lk],
+                                                                  X[(k0 + lk) * PUR_LS + 16 * tj[s] + li], acc[s], 0, 0, 0);
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
-            if (row0 + 4 * v == 16 * w + li) dx2 += acc[w][v];
-        const double tr = block_sum(dx, red), tr2 = block_sum(dx2, red);
+        for (int s = 0; s < PUR_TILES; ++s)
+            if (s < mine && ti[s] == tj[s])
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    if (lk + 4 * v == li) diag2[16 * ti[s] + li] = acc[s][v];
+        const double dx = X[lane * PUR_LS + lane];
+        __syncthreads();                            // X read by all, diagonal of X^2 complete
+        const double tr = wave_sum(dx), tr2 = wave_sum(diag2[lane]);
+        if (it < steps && fabs(tr - tr2) < tol) it = steps;
         if (it == steps) last = fabs(tr - tr2);
-        const bool hold = it < steps && fabs(tr - tr2) < tol;
         const bool square = tr > ne;
-        __syncthreads();
-        if (!hold)
 #pragma unroll
-            for (int tj = 0; tj < 4; ++tj)
+        for (int s = 0; s < PUR_TILES; ++s)
+            if (s < mine)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    double& x = X[(row0 + 4 * v) * PUR_LS + 16 * tj + li];
-                    x = square ? acc[tj][v] : 2.0 * x - acc[tj][v];
+                    const int i = 16 * ti[s] + lk + 4 * v, j = 16 * tj[s] + li;
+                    const double x = square ? acc[s][v] : 2.0 * X[i * PUR_LS + j] - acc[s][v];
+                    X[i * PUR_LS + j] = x;
+                    if (ti[s] != tj[s]) X[j * PUR_LS + i] = x;
                 }
         __syncthreads();
     }
