@@ -188,8 +188,7 @@ class ReplicaBatch:
         self.Pbuf = torch.zeros((R * 2, n, n), **f64)
         self.perr = torch.zeros(R * 2, **f64)
         self.G = torch.zeros((R, M, M), **f64)
-        self.rhs = torch.zeros((R, M), **f64)
-        self.coef = torch.zeros((R, M), **f64)
+        self.Fx = torch.zeros((R, 2, n, n), **f64)
         self.energy_el = torch.zeros(R, **f64)
         self.e_prev = torch.full((R,), float("nan"), **f64)
         self.err = torch.zeros(R, **f64)
@@ -198,11 +197,10 @@ class ReplicaBatch:
         self.count = torch.zeros(1, dtype=torch.long, device=dev)
         self.nocc_t = torch.tensor(self.nocc.reshape(-1), **f64)
         idx = torch.arange(n, device=dev)
-        real = idx[None, :] < torch.tensor(self.rep_nao, device=dev)[:, None]          # (R, n)
+        self.rep_nao_t = torch.tensor(self.rep_nao, dtype=torch.int32, device=dev)
+        real = idx[None, :] < self.rep_nao_t[:, None]                                   # (R, n)
         self.real = real
         self.pad_diag = torch.diag_embed((~real).to(torch.float64))                     # (R, n, n)
-        self.eye_m = torch.eye(M, **f64)
-        self.slots = torch.arange(M, device=dev)
 
     # ------------------------------------------------------- integrals
     def _set_geometry(self, x: np.ndarray) -> None:
@@ -221,19 +219,13 @@ class ReplicaBatch:
                                for a, b in zip(self.rep_atom[:-1], self.rep_atom[1:])])
 
     def _inv_sqrt(self, S: torch.Tensor, iters: int = 30) -> torch.Tensor:
-        """S^(-1/2) of every replica by the coupled Newton-Schulz iteration (batched products);
-        the residual |X S X - 1| is checked once per geometry on the host."""
-        eye = torch.eye(self.ld, dtype=S.dtype, device=S.device).expand_as(S)
-        c = S.abs().sum(dim=2).amax(dim=1)[:, None, None]
-        Y = S / c
-        Z = eye.clone()
-        for _ in range(iters):
-            Tm = 0.5 * (3.0 * eye - Z @ Y)
-            Y = Y @ Tm
-            Z = Tm @ Z
-        Xs = Z / torch.sqrt(c)
-        Xs = 0.5 * (Xs + Xs.transpose(1, 2))
-        res = float((Xs @ S @ Xs - eye).abs().amax())
+        """S^(-1/2) of every replica by the coupled Newton-Schulz iteration (one launch); the
+        residual |X S X - 1| is checked once per geometry on the host."""
+        Xs = torch.empty_like(S)
+        out = torch.empty((self.nrep, 2), dtype=S.dtype, device=S.device)
+        _lib.check(_lib.lib().aimdhf_small_inv_sqrt(self.nrep, self.ld, _ptr(S), _ptr(Xs), iters, 1e-13, _ptr(out),
+                                                    _stream()))
+        res = float(out[:, 0].amax())
         if not res < 1e-9:
             s, U = torch.linalg.eigh(S)
             if float(s.amin()) < self.lindep:
@@ -273,51 +265,20 @@ class ReplicaBatch:
         """One SCF iteration of every replica on static buffers (captured as a graph)."""
         L = _lib.lib()
         R, n, M = self.nrep, self.ld, self.diis_space
-        D, X, S, H = self.D, self.X, self.S, self.H
-        self._jk(D)
-        Jt = self.J[:, 0] + self.J[:, 1]
-        F = H[:, None] + Jt[:, None] - self.K
-        F = 0.5 * (F + F.transpose(2, 3))
-        self.F.copy_(F)
-        self.energy_el.copy_(0.5 * (D * (H[:, None] + F)).sum(dim=(1, 2, 3)))
-        Xe = X[:, None]
-        FDS = F @ D @ S[:, None]
-        err = Xe.transpose(2, 3) @ (FDS - FDS.transpose(2, 3)) @ Xe
-        self.err.copy_(err.abs().amax(dim=(1, 2, 3)))
-        Fo = Xe.transpose(2, 3) @ F @ Xe
-        # DIIS: push into the ring slot, Gram matrix of the stored errors, anchored system
-        self.Fbuf.index_copy_(1, self.slot, Fo[:, None])
-        self.Ebuf.index_copy_(1, self.slot, err[:, None])
-        Ev = self.Ebuf.view(R, M, -1)
-        G = Ev @ Ev.transpose(1, 2)                                                     # (R, M, M)
-        a = self.slot.view(1, 1, 1).expand(R, M, 1)
-        Gia = torch.gather(G, 2, a)                                                     # (R, M, 1)
-        Gaa = torch.gather(Gia, 1, self.slot.view(1, 1, 1).expand(R, 1, 1))            # (R, 1, 1)
-        Gd = G - Gia - Gia.transpose(1, 2) + Gaa
-        r = (Gaa - Gia)[:, :, 0]
-        valid = (self.slots < self.count) & (self.slots != self.slot)                  # (M,)
-        keep = valid[None, :, None] & valid[None, None, :]
-        Gs = torch.where(keep, Gd, self.eye_m.expand(R, M, M))
-        rs = torch.where(valid[None, :], r, torch.zeros_like(r))
-        self.G.copy_(Gs)
-        self.rhs.copy_(rs)
-        _lib.check(L.aimdhf_batch_diis_solve(R, M, _ptr(self.G), _ptr(self.rhs), _ptr(self.coef), _stream()))
-        c = torch.where(valid[None, :], self.coef, torch.zeros_like(self.coef))
-        anchor = (self.slots[None, :] == self.slot[:, None]).to(c.dtype)                # (1, M)
-        c = c + anchor * (1.0 - c.sum(dim=1, keepdim=True))
-        bad = ~(torch.isfinite(c).all(dim=1) & (c.abs().amax(dim=1) <= 1e4))
-        c = torch.where(bad[:, None], anchor.expand(R, M), c)
-        Fx = (c[:, :, None, None, None] * self.Fbuf).sum(dim=1)                         # (R, 2, n, n)
-        Fx = Fx + PAD_LEVEL * self.pad_diag[:, None]
-        _lib.check(L.aimdhf_batch_purify(R * 2, n, _ptr(Fx.contiguous()), _ptr(self.nocc_t), _ptr(self.Pbuf),
+        vec = 2 * n * n
+        self._jk(self.D)
+        _lib.check(L.aimdhf_small_fock(R, 2, n, _ptr(self.H), _ptr(self.S), _ptr(self.X), _ptr(self.D), _ptr(self.J),
+                                       _ptr(self.K), _ptr(self.F), _ptr(self.Fbuf), _ptr(self.Ebuf), M * vec, vec,
+                                       _ptr(self.slot), _ptr(self.energy_el), _ptr(self.err), _stream()))
+        # DIIS over the ring, the new vector in the slot just written
+        _lib.check(L.aimdhf_small_diis(R, 2, n, M, _ptr(self.slot), _ptr(self.count), _ptr(self.Ebuf),
+                                       _ptr(self.Fbuf), _ptr(self.G), _ptr(self.rep_nao_t), PAD_LEVEL, _ptr(self.Fx),
+                                       _stream()))
+        _lib.check(L.aimdhf_batch_purify(R * 2, n, _ptr(self.Fx), _ptr(self.nocc_t), _ptr(self.Pbuf),
                                          self.purify_steps, 1e-11, _ptr(self.perr), _stream()))
-        Dn = Xe @ self.Pbuf.view(R, 2, n, n) @ Xe.transpose(2, 3)
-        conv = ((self.energy_el - self.e_prev).abs() < self.conv_tol) & (self.err < self.conv_tol_grad)
-        self.frozen |= conv
-        self.D.copy_(torch.where(self.frozen[:, None, None, None], D, Dn))
-        self.e_prev.copy_(self.energy_el)
-        self.slot.copy_((self.slot + 1) % M)
-        self.count.copy_(torch.clamp(self.count + 1, max=M))
+        _lib.check(L.aimdhf_small_density(R, 2, n, _ptr(self.X), _ptr(self.Pbuf), _ptr(self.D), _ptr(self.frozen),
+                                          _ptr(self.energy_el), _ptr(self.err), _ptr(self.e_prev), self.conv_tol,
+                                          self.conv_tol_grad, _ptr(self.slot), _ptr(self.count), M, _stream()))
 
     def _replay(self) -> None:
         if not self.capture:
@@ -340,7 +301,7 @@ class ReplicaBatch:
 
     def _state(self):
         return [self.D, self.F, self.Fbuf, self.Ebuf, self.energy_el, self.e_prev, self.err, self.frozen, self.slot,
-                self.count, self.J, self.K, self.Pbuf, self.perr, self.G, self.rhs, self.coef]
+                self.count, self.J, self.K, self.Pbuf, self.perr, self.G, self.Fx]
 
     def _guess(self) -> torch.Tensor:
         Ds = torch.zeros((self.nrep, 2, self.ld, self.ld), dtype=torch.float64, device=self.device)

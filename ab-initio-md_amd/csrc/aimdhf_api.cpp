@@ -4,6 +4,7 @@
 #include "../../include/aimdhf.h"
 #include "aimdhf_internal.h"
 #include "jk_digest.h"
+#include "scf_small.h"
 
 #include <algorithm>
 #include <chrono>
@@ -1689,6 +1690,58 @@ int aimdhf_batch_purify(int nmat, int ld, const double* F, const double* nocc, d
     aimdhf::launch_batch_purify(nmat, ld, F, nocc, P, steps, tol, err, (hipStream_t)stream);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(AIMDHF_E_HIP, std::string("batch purify: ") + hipGetErrorString(e));
+    return AIMDHF_OK;
+}
+
+int aimdhf_small_fock(int nrep, int nspin, int ld, const double* H, const double* S, const double* X, const double* D,
+                      const double* J, const double* K, double* F, double* Fo, double* E, int64_t rep_stride,
+                      int64_t slot_stride, const int64_t* slot, double* energy, double* err, void* stream) {
+    if (nrep < 0 || nspin < 1 || nspin > 2 || ld <= 0 || ld > 64) return fail(AIMDHF_E_ARG, "bad small_fock arguments");
+    if (nrep == 0) return AIMDHF_OK;
+    if (!H || !S || !X || !D || !J || !K || !F || !Fo || !E || !energy || !err) return fail(AIMDHF_E_ARG, "NULL argument");
+    aimdhf::SmallFock a{nspin, ld, 2.0 / nspin, H, S, X, D, J, K, F, Fo, E, rep_stride, slot_stride,
+                        (const long long*)slot, energy, err};
+    aimdhf::launch_small_fock(a, nrep, (hipStream_t)stream);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(AIMDHF_E_HIP, std::string("small fock: ") + hipGetErrorString(e));
+    return AIMDHF_OK;
+}
+
+int aimdhf_small_diis(int nrep, int nspin, int ld, int m, const int64_t* slot, const int64_t* count, const double* E,
+                      const double* Fo, double* G, const int32_t* rep_nao, double pad, double* Fx, void* stream) {
+    if (nrep < 0 || nspin < 1 || nspin > 2 || ld <= 0 || ld > 64 || m < 1 || m > 12)
+        return fail(AIMDHF_E_ARG, "bad small_diis arguments");
+    if (nrep == 0) return AIMDHF_OK;
+    if (!slot || !count || !E || !Fo || !G || !Fx) return fail(AIMDHF_E_ARG, "NULL argument");
+    aimdhf::SmallDiis a{nspin, ld, m, (const long long*)slot, (const long long*)count, E, Fo, G, rep_nao, pad, Fx};
+    aimdhf::launch_small_diis(a, nrep, (hipStream_t)stream);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(AIMDHF_E_HIP, std::string("small diis: ") + hipGetErrorString(e));
+    return AIMDHF_OK;
+}
+
+int aimdhf_small_density(int nrep, int nspin, int ld, const double* X, const double* P, double* D, uint8_t* frozen,
+                         const double* energy, const double* err, double* e_prev, double conv_e, double conv_g,
+                         int64_t* slot, int64_t* count, int m, void* stream) {
+    if (nrep < 0 || nspin < 1 || nspin > 2 || ld <= 0 || ld > 64) return fail(AIMDHF_E_ARG, "bad small_density arguments");
+    if (nrep == 0) return AIMDHF_OK;
+    if (!X || !P || !D || (frozen && (!energy || !err || !e_prev)) || (slot && (!count || m < 1)))
+        return fail(AIMDHF_E_ARG, "NULL argument");
+    aimdhf::SmallDensity a{nspin, ld, X, P, D, frozen, energy, err, e_prev, conv_e, conv_g, (long long*)slot,
+                           (long long*)count, m};
+    aimdhf::launch_small_density(a, nrep, (hipStream_t)stream);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(AIMDHF_E_HIP, std::string("small density: ") + hipGetErrorString(e));
+    return AIMDHF_OK;
+}
+
+int aimdhf_small_inv_sqrt(int nmat, int ld, const double* S, double* X, int iters, double tol, double* out, void* stream) {
+    if (nmat < 0 || ld <= 0 || ld > 64 || iters < 1 || !(tol >= 0.0)) return fail(AIMDHF_E_ARG, "bad small_inv_sqrt arguments");
+    if (nmat == 0) return AIMDHF_OK;
+    if (!S || !X || !out) return fail(AIMDHF_E_ARG, "NULL argument");
+    aimdhf::launch_small_inv_sqrt(nmat, ld, S, X, iters, tol, out, (hipStream_t)stream);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(AIMDHF_E_HIP, std::string("small inv_sqrt: ") + hipGetErrorString(e));
     return AIMDHF_OK;
 }
 

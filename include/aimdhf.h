@@ -216,6 +216,41 @@ int aimdhf_batch_set_jk_lanes(aimdhf_plan* plan, int lanes);
  */
 int aimdhf_batch_diis_solve(int nrep, int m, const double* G, const double* r, double* c, void* stream);
 
+/*
+ * SCF algebra of small matrices (ld <= 64), one workgroup per replica, products on
+ * the matrix cores; for batches and single small molecules. No plan; every call is
+ * capturable. Replace the dense products around one SCF iteration
+ * (aimd/qc/scf.py:863-923), the Pulay step (scf.py:540-568) and the
+ * orthogonaliser (scf.py:284-303).
+ *
+ * small_fock: F_s = sym(H + (2/nspin) sum J - K_s), electronic energies, E = X^T (F D S -
+ * S D F) X with its largest element err, and Fo = X^T F X; Fo and E of replica r are
+ * written at r rep_stride + *slot slot_stride doubles (slot a device scalar or NULL).
+ * H, S, X (nrep, ld, ld); D, J, K, F (nrep, nspin, ld, ld).
+ *
+ * small_diis: Pulay extrapolation of a ring of m <= 12 vectors E, Fo (nrep, m, nspin,
+ * ld, ld): *count held, the newest in *slot; its row of the Gram matrices G (nrep, m,
+ * m) is computed, the others are kept from earlier calls; coefficients that are not
+ * finite or above 1e4 give the newest vector alone. pad is added to the diagonal past
+ * each replica's rep_nao (NULL: ld).
+ *
+ * small_density: D = X P X^T per spin; with frozen (bytes) a replica whose |energy -
+ * e_prev| < conv_e and err < conv_g is frozen and keeps its D, e_prev is updated;
+ * with slot the ring position and count are advanced.
+ *
+ * small_inv_sqrt: X = S^(-1/2) by Newton-Schulz until |Z Y - 1| < tol or iters steps;
+ * out (nmat, 2): max |X S X - 1| and a lower bound of S's smallest eigenvalue.
+ */
+int aimdhf_small_fock(int nrep, int nspin, int ld, const double* H, const double* S, const double* X, const double* D,
+                      const double* J, const double* K, double* F, double* Fo, double* E, int64_t rep_stride,
+                      int64_t slot_stride, const int64_t* slot, double* energy, double* err, void* stream);
+int aimdhf_small_diis(int nrep, int nspin, int ld, int m, const int64_t* slot, const int64_t* count, const double* E,
+                      const double* Fo, double* G, const int32_t* rep_nao, double pad, double* Fx, void* stream);
+int aimdhf_small_density(int nrep, int nspin, int ld, const double* X, const double* P, double* D, uint8_t* frozen,
+                         const double* energy, const double* err, double* e_prev, double conv_e, double conv_g,
+                         int64_t* slot, int64_t* count, int m, void* stream);
+int aimdhf_small_inv_sqrt(int nmat, int ld, const double* S, double* X, int iters, double tol, double* out, void* stream);
+
 /* err[0] (device) = |tr X - sum_ij X_ij^2|, the idempotency error of a symmetric
  * purification iterate X (n x n, device). Row sums, then their sum in a fixed
  * order (bitwise reproducible); the row sums go through the same device array
