@@ -178,6 +178,12 @@ struct Fan {
         }
         HIPCHECK(hipEventCreateWithFlags(&fork_ev, hipEventDisableTiming));
     }
+    // whether st records a graph, into which the auxiliary streams are not drawn
+    static bool capturing(hipStream_t st) {
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        HIPCHECK(hipStreamIsCapturing(st, &status));
+        return status != hipStreamCaptureStatusNone;
+    }
     void fork(hipStream_t st) {
         base = st;
         if (serial) return;
@@ -199,6 +205,17 @@ struct Fan {
             if (join_ev[i]) (void)hipEventDestroy(join_ev[i]);
         }
         if (fork_ev) (void)hipEventDestroy(fork_ev);
+    }
+};
+
+// The streams of the six one-electron pair classes: all the caller's, or the heaviest
+// classes (d d, d p, d s) apart on the fan's, since each is a chain of a few hundred
+// microseconds in small molecules whose classes do not fill the card
+struct PairStreams {
+    hipStream_t on[6];
+    explicit PairStreams(hipStream_t st) { std::fill(on, on + 6, st); }
+    explicit PairStreams(const Fan& fan) {
+        for (int c = 0; c < 6; ++c) on[c] = fan.on(5 - c);
     }
 };
 
@@ -1459,7 +1476,12 @@ int aimdhf_one_electron(aimdhf_plan* p, double* S, double* T, double* V, double*
             g.M = M;
             p->prof.time(43, st, [&] { aimdhf::launch_gen_oneel(g, p->npair, st); });
         } else {
-            p->prof.time(43, st, [&] { aimdhf::launch_oneel(p->oneel_args(), S, T, M, V, st); });
+            p->prof.time(43, st, [&] {
+                const bool one = Fan::capturing(st);
+                if (!one) p->fan.fork(st);
+                aimdhf::launch_oneel(p->oneel_args(), S, T, M, V, (one ? PairStreams(st) : PairStreams(p->fan)).on);
+                if (!one) p->fan.join();
+            });
         }
         HIPCHECK(hipGetLastError());
     } catch (const HipError& e) {
@@ -1487,7 +1509,13 @@ int aimdhf_grad_one(aimdhf_plan* p, const double* D, const double* W, double* gr
         aimdhf::launch_negate(Wn, nn, Wn, st);
         p->d_gfx.ensure(sizeof(long long) * 6 * p->natm);
         aimdhf::launch_zero64(p->d_gfx.as<long long>(), 6 * p->natm, st);
-        p->prof.time(44, st, [&] { aimdhf::launch_grad_one(p->oneel_args(), Ds, Wn, p->d_gfx.as<long long>(), st); });
+        p->prof.time(44, st, [&] {
+            const bool one = Fan::capturing(st);
+            if (!one) p->fan.fork(st);
+            aimdhf::launch_grad_one(p->oneel_args(), Ds, Wn, p->d_gfx.as<long long>(),
+                                    (one ? PairStreams(st) : PairStreams(p->fan)).on);
+            if (!one) p->fan.join();
+        });
         aimdhf::launch_fx_to_double(p->d_gfx.as<long long>(), 3 * p->natm, grad, st);
         HIPCHECK(hipGetLastError());
     } catch (const HipError& e) {
@@ -1518,7 +1546,7 @@ int aimdhf_grad_one_noalloc(aimdhf_plan* p, const double* D, const double* W, do
     aimdhf::launch_symmetrize(W, 1, p->nao, Wn, st);
     aimdhf::launch_negate(Wn, nn, Wn, st);
     aimdhf::launch_zero64(fx, 6 * (size_t)p->natm, st);     // a fill kernel: the array keeps the last call's sums
-    aimdhf::launch_grad_one(p->oneel_args(), Ds, Wn, fx, st);
+    aimdhf::launch_grad_one(p->oneel_args(), Ds, Wn, fx, PairStreams(st).on);
     aimdhf::launch_fx_to_double(fx, 3 * p->natm, grad, st);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(AIMDHF_E_HIP, std::string("grad_one_noalloc: ") + hipGetErrorString(e));
@@ -1554,10 +1582,10 @@ int aimdhf_grad_one_terms(aimdhf_plan* p, const double* D, const double* W, doub
         // kinetic: overlap/kinetic part with W = 0; nuclear attraction alone; overlap:
         // overlap/kinetic part with D = 0 (the -W S term)
         g.parts = 1;
-        aimdhf::launch_grad_one(g, Ds, Z, fx, st);
-        aimdhf::launch_grad_one(g, Z, Wn, fx + 12 * p->natm, st);
+        aimdhf::launch_grad_one(g, Ds, Z, fx, PairStreams(st).on);
+        aimdhf::launch_grad_one(g, Z, Wn, fx + 12 * p->natm, PairStreams(st).on);
         g.parts = 2;
-        aimdhf::launch_grad_one(g, Ds, Z, fx + 6 * p->natm, st);
+        aimdhf::launch_grad_one(g, Ds, Z, fx + 6 * p->natm, PairStreams(st).on);
         aimdhf::launch_fx_to_double(fx, 3 * p->natm, g_kin, st);
         aimdhf::launch_fx_to_double(fx + 6 * p->natm, 3 * p->natm, g_nuc, st);
         aimdhf::launch_fx_to_double(fx + 12 * p->natm, 3 * p->natm, g_ovl, st);

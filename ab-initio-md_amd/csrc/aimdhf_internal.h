@@ -161,11 +161,12 @@ void launch_symmetrize(const double* D, int nset, int n, double* out, hipStream_
 void launch_grad_one_class(int k, const GradArgs& a, const int2* list, long long nq, hipStream_t st);
 void launch_grad_keep(int k, const GradArgs& a, const int2* list, long long nq, hipStream_t st);
 void launch_pair_dmax(const GradArgs& a, const int* shell_l, double* dmc, double* dmx, hipStream_t st);
-void launch_oneel(const OneElArgs& g, double* S, double* T, double* M, double* V, hipStream_t st);
+// on: the stream of each of the six pair classes
+void launch_oneel(const OneElArgs& g, double* S, double* T, double* M, double* V, const hipStream_t* on);
 // device address of the fixed-size scratch array of the allocation-free entry
 // points on the current device (resolved once per device), and its size
 void* noalloc_scratch(size_t* bytes);
-void launch_grad_one(const OneElArgs& g, const double* D, const double* Wneg, long long* out, hipStream_t st);
+void launch_grad_one(const OneElArgs& g, const double* D, const double* Wneg, long long* out, const hipStream_t* on);
 void launch_negate(const double* W, size_t n, double* out, hipStream_t st);
 void launch_fx_to_double(const long long* fx, int n, double* out, hipStream_t st);
 void launch_grad(const GradArgs& a, const int2* const* lists, const long long* counts, hipStream_t st);

@@ -152,16 +152,18 @@ MD_HD void overlap_type_acc(const ShellView& B, int si, int sj, const double* O,
     }
 }
 
-// V block contributions of point charges c = c0, c0 + cs, ... < nc into v (NC(LI) x NC(LJ))
+// V block contributions of point charges c = c0, c0 + cs, ... < nc and primitive pairs
+// k = k0, k0 + ks, ... (row-major over si's and sj's primitives) into v (NC(LI) x NC(LJ))
 template <int LI, int LJ>
 MD_HD void nuclear_acc(const ShellView& B, int si, int sj, int c0, int cs, int nc, const double* Z, const double* C,
-                       const double* tab, double* v) {
+                       const double* tab, double* v, int k0 = 0, int ks = 1) {
     constexpr int NI = NC(LI), NJ = NC(LJ), L = LI + LJ, NHL = NH(L);
     const int ai = B.atom[si], aj = B.atom[sj];
-    for (int ka = B.prim[si]; ka < B.prim[si + 1]; ++ka) {
-        const double a = B.ex[ka];
-        for (int kb = B.prim[sj]; kb < B.prim[sj + 1]; ++kb) {
-            const double b = B.ex[kb];
+    const int pi0 = B.prim[si], npj = B.prim[sj + 1] - B.prim[sj], npp = (B.prim[si + 1] - pi0) * npj;
+    {
+        for (int k = k0; k < npp; k += ks) {
+            const int ka = pi0 + k / npj, kb = B.prim[sj] + k % npj;
+            const double a = B.ex[ka], b = B.ex[kb];
             const double p = a + b, mu = a * b / p;
             E1T<LI, LJ> E[3];
 #pragma unroll
@@ -261,12 +263,15 @@ MD_HD void ovlkin_grad_acc(const ShellView& B, int n, int si, int sj, const doub
     }
 }
 
-// d/dR sum D V of shells si, sj for operator centres c = c0, c0 + cs, ... < natm
-// (integrals.py:407-501): add(c, d, x) for each centre, gA / gB += the basis-centre
-// terms of atom(si) / atom(sj)
+// d/dR sum D V of shells si, sj for operator centres c = c0 + co, c0 + cs + co, ... < natm
+// and primitive pairs k = k0, k0 + ks, ... (integrals.py:407-501): add(c, d, x) for each
+// centre, called with c >= natm and x = 0 where the round's c0 + ... < natm but the
+// lane's centre is past the end, so lanes of a wavefront with different co and k0 meet
+// there; gA / gB += the basis-centre terms of atom(si) / atom(sj)
 template <int LI, int LJ, class Add>
 MD_HD void nuclear_grad_acc(const ShellView& B, int n, int si, int sj, int c0, int cs, int natm, const double* Z,
-                            const double* D, const double* tab, Add add, double* gA, double* gB) {
+                            const double* D, const double* tab, Add add, double* gA, double* gB, int co = 0,
+                             int k0 = 0, int ks = 1) {
     constexpr int NI = NC(LI), NJ = NC(LJ), L = LI + LJ, NHL = NH(L), NH1 = NH(L + 1);
     const int ai = B.atom[si], aj = B.atom[sj];
     const int oi = B.ao[si], oj = B.ao[sj];
@@ -279,12 +284,14 @@ MD_HD void nuclear_grad_acc(const ShellView& B, int n, int si, int sj, int c0, i
             wd[ia * NJ + ib] = sym * cart_factor(cart_x(LI, ia), cart_y(LI, ia), cart_z(LI, ia)) *
                                cart_factor(cart_x(LJ, ib), cart_y(LJ, ib), cart_z(LJ, ib)) *
                                D[(size_t)(oi + ia) * n + oj + ib];
-    for (int c = c0; c < natm; c += cs) {
+    const int pi0 = B.prim[si], npj = B.prim[sj + 1] - B.prim[sj], npp = (B.prim[si + 1] - pi0) * npj;
+    for (int cb = c0; cb < natm; cb += cs) {
+        const int c = cb + co;
         double gc[3] = {0.0, 0.0, 0.0};
-        for (int ka = B.prim[si]; ka < B.prim[si + 1]; ++ka) {
-            const double a = B.ex[ka];
-            for (int kb = B.prim[sj]; kb < B.prim[sj + 1]; ++kb) {
-                const double b = B.ex[kb];
+        if (c < natm) {
+            for (int k = k0; k < npp; k += ks) {
+                const int ka = pi0 + k / npj, kb = B.prim[sj] + k % npj;
+                const double a = B.ex[ka], b = B.ex[kb];
                 const double p = a + b, mu = a * b / p;
                 E1T<LI + 1, LJ> E[3];
 #pragma unroll

@@ -152,3 +152,29 @@ def test_unsupported_angular_momentum_is_a_value_error():
     b = BasisSet("custom", ["H"], np.zeros((1, 3)), [0], [5], [0, 1], [1.0], [1.0])
     with pytest.raises(ValueError, match="l = 5"):
         Engine(b)
+
+
+@pytest.mark.parametrize("natm", [1, 2, 5, 17, 33, 65])
+def test_one_electron_terms_over_nuclei_and_primitive_pairs(oracle_lib, natm):
+    # every split of a wavefront's lanes over nuclei and primitive pairs: 1, 6, 18 and 36
+    # primitive pairs with 1 ... 65 nuclei. Each sum has natm times a fixed number of terms.
+    import torch
+    s = ["O" if k % 4 == 0 else "H" for k in range(natm)]
+    x = np.array([[2.1 * (k % 4), 2.3 * (k // 4 % 4), 2.5 * (k // 16)] for k in range(natm)])
+    x = x + 0.05 * np.random.default_rng(natm).standard_normal((natm, 3))
+    b, e = _engine(s, x, "6-31g*")
+    n = b.nao
+    S = torch.empty((n, n), dtype=torch.float64, device="cuda")
+    T, V = torch.empty_like(S), torch.empty_like(S)
+    M = torch.empty((3, n, n), dtype=torch.float64, device="cuda")
+    e.one_electron(S, T, V, M)
+    ob = oracle_lib.make_basis(s, x, "6-31g*")
+    for a, o in zip((S, T, V, M), oracle_lib.one_electron(ob)):
+        np.testing.assert_allclose(a.cpu().numpy(), o, rtol=0, atol=1e-12 * max(1, natm / 4))
+    rng = np.random.default_rng(natm + 100)
+    P, W = (0.1 * (a + a.T) for a in rng.standard_normal((2, n, n)))
+    g = e.grad_one(torch.tensor(P, device="cuda"), torch.tensor(W, device="cuda")).cpu().numpy()
+    np.testing.assert_allclose(g, oracle_lib.one_electron_gradient(ob, P, W), rtol=0, atol=1e-11 * max(1, natm / 4))
+    again = e.grad_one(torch.tensor(P, device="cuda"), torch.tensor(W, device="cuda")).cpu().numpy()
+    np.testing.assert_array_equal(g, again)
+    e.close()
