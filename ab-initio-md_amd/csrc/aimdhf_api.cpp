@@ -71,8 +71,10 @@ int ncart(int l) { return (l + 1) * (l + 2) / 2; }
 int nherm(int L) { return (L + 1) * (L + 2) * (L + 3) / 6; }
 constexpr int NQCLASS = 21;
 constexpr int REC_HDR = 8;
-// single molecules up to nset nao^2 of this digest all classes in one launch: measured per
-// build, (1, 19 AOs) 30 against 174 us, (1, 114) 132 against 187; (2, 100) 183 against 169
+// single molecules up to nset nao^2 of this digest all classes in one or two launches:
+// measured per build against 21 launches, (1, 19 AOs) 30 : 174 us, (1, 114) 93 : 187,
+// (2, 100) 128 : 169, (1, 152) 175 : 219; past it the per-class kernels' own thread counts
+// and two densities at once win
 constexpr int SMALL_JK = 200 * 200;
 
 // Boys grid table F_n(k/10), n < 43 (aimd/qc/boys.py:57-75): series for the

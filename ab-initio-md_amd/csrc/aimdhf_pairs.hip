@@ -1,10 +1,5 @@
-// gfx950 kernels of the Hartree-Fock force engine: primitive-pair build,
-// Schwarz bounds, screened quartet lists, and the integral-direct J/K build.
-//
-// One thread evaluates one contracted shell quartet (class-templated, l <= 2)
-// and digests it straight from registers into J and K, accumulated as exact
-// fixed-point integers (md_core.h: fx_split), so the Fock build is bitwise
-// reproducible from run to run whatever order the waves execute in.
+// gfx950 kernels of a new geometry: primitive-pair build, Schwarz bounds and the
+// pair tables that the quartet lists and integral kernels read.
 
 #include "aimdhf_internal.h"
 #include "md_eri.h"

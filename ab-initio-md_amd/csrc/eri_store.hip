@@ -70,6 +70,7 @@ __global__ __launch_bounds__(256) void k_eri(EriArgs a, Real* __restrict__ store
 // quartet's bra primitives, the parts are added in wavefront order. A lane alone walks
 // up to 36 x 36 (6-31G*) or 64 x 64 (cc-pVDZ) dependent primitive quartets, 0.28 us each:
 // 0.36 ms for one water's (ss|ss), 2.5 ms for (H2O)8/cc-pVDZ, most of it this chain
+// (four waters' geometry and first Fock matrix, with the Schwarz bounds split alike: 2.87 -> 1.43 ms)
 template <int LA_, int LB_, int LC_, int LD_, typename Real>
 __global__ __launch_bounds__(64 * WH) void k_eri_split(EriArgs a, Real* __restrict__ store, long long nq) {
     constexpr int NV = SPLIT ? Qt::NAB : BLK;           // values per lane

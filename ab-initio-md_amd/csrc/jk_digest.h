@@ -143,8 +143,8 @@ bool digest_all_fits(int ld, int lds_limit);
 // max_m |q_m|^2 max_l sum_s |D_ls| (the spectral norm of |D| is at most its
 // largest row sum), to a J element by q_max sum_ls q_ls |D_ls| (a fixed-point sum,
 // so the smaller of it and its Cauchy-Schwarz bound q_max |q|_F |D|_F); scaled
-// below 2^62 no sum overflows, and the resolution is 2^-62 of the bound: on
-// (H2O)32/6-31G*, 2e-16 Eh for J (up to 25) and 1e-17 for K (up to 5).
+// below 2^62 no sum overflows, and the resolution is at most 2^-61 of the bound
+// (J and K of (H2O)32/6-31G* agree with two-word sums of 2^-80 resolution to 2e-13).
 __device__ inline int jk_exponent(double bound) {
     if (!(bound > 0.0)) return 0;
     const int e = 61 - ilogb(bound);

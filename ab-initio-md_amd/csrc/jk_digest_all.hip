@@ -47,6 +47,9 @@ void launch_digest_all(const DigestArgs& a, int threads, hipStream_t st) {
         (k < LIGHT ? nl : nh) += a.cls_off[cb + 1] - a.cls_off[cb];
     }
     const size_t lds = sizeof(double) * (HEAD + (size_t)COLW * a.ld);
+    // two launches from the runs on that keep all CUs busy at three wavefronts a SIMD: one
+    // water 30 (one launch) : 39 us (two), 76 AOs 62 : 57, 114 AOs 131 : 94, 128 replicas
+    // 690 : 450 us
     if (nl + nh > 1200) {
         if (nh > 0) k_digest_heavy<<<dim3(nh, a.nparts, a.nset), dim3(threads), lds, st>>>(a);
         if (nl > 0) k_digest_light<<<dim3(nl, a.nparts, a.nset), dim3(threads), lds, st>>>(a);
