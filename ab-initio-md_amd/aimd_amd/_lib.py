@@ -43,6 +43,8 @@ SIGNATURES = {
     "aimdhf_tc2_init": (_I, [_I, _P, _P, _P]),
     "aimdhf_batch_purify": (_I, [_I, _I, _P, _P, _P, _I, _D, _P, _P]),
     "aimdhf_batch_diis_solve": (_I, [_I, _I, _P, _P, _P, _P]),
+    "aimdhf_tc2_sums": (_I, [_I, _P, _P, _P]),
+    "aimdhf_tc2_fused": (_I, [_I, _P, _P, _P, _P, _D, _D, _P]),
     "aimdhf_small_fock": (_I, [_I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _L, _P, _P, _P, _P]),
     "aimdhf_small_diis": (_I, [_I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _D, _P, _P]),
     "aimdhf_small_density": (_I, [_I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _D, _D, _P, _P, _I, _P]),

@@ -180,6 +180,13 @@ def check_nuclear_separation(positions: np.ndarray, atomic_numbers: np.ndarray) 
 SMALL_NAO = 64
 
 
+# Largest matrix whose purification step is one launch of the engine's kernel.
+# Measured per step against the library product and the update: 76 AOs 4.8 : 10.6 us, 304
+# 7.3 : 12.2, 608 15.3 : 29.5, 1024 45.9 : 47.4; 1536 143 : 144, 2048 332 : 275 (the kernel
+# reads every operand from L2, once per 16 x 16 tile).
+TC2_FUSED_NAO = 1024
+
+
 def _ptr(t: torch.Tensor) -> ctypes.c_void_p:
     return ctypes.c_void_p(t.data_ptr())
 
@@ -237,7 +244,7 @@ def inverse_sqrt_newton_schulz(S: torch.Tensor, max_iter: int = 60, tol: float =
     does not fall below 1e-10 within max_iter steps.
     """
     n = S.shape[0]
-    if S.is_cuda and S.dtype == torch.float64 and n <= SMALL_NAO:
+    if S.is_cuda and S.dtype == torch.float64 and n <= SMALL_NAO and not S.requires_grad:
         S = S.contiguous()
         X, out = torch.empty_like(S), torch.empty(2, dtype=S.dtype, device=S.device)
         with torch.cuda.device(S.device):
@@ -266,8 +273,8 @@ class TC2Graph:
     """
     Purification steps of an n x n matrix with nocc electrons captured once as HIP
     graphs, STEPS steps (``replay``) and TAIL_STEPS steps (``tail``) on the same
-    buffers: each step is a dense FP64 product X2 = X X (BLAS) and the engine's
-    fused update (aimdhf_tc2_step), ping-ponging between two static buffers so the
+    buffers: each step is one launch (aimdhf_tc2_fused; above TC2_FUSED_NAO a dense
+    FP64 product X2 = X X and aimdhf_tc2_step), ping-ponging between two static buffers so the
     result of an even number of steps lands back in ``X``. The update kernel needs
     no reduction pass and clears no memory, so replays are exact repeats. The
     replayed steps hold an iterate whose idempotency error is below ``tol``
@@ -285,7 +292,13 @@ class TC2Graph:
         self.needed = 1
         self.X = torch.zeros((n, n), dtype=torch.float64, device=device)
         self.B = torch.empty_like(self.X)
-        self.X2 = torch.empty_like(self.X)
+        # product and update in one launch, or a library product and the update
+        self.fused = n <= TC2_FUSED_NAO
+        if self.fused:
+            t = (n + 15) // 16
+            self.sums = torch.zeros((2, t * (t + 1)), dtype=torch.float64, device=device)
+        else:
+            self.X2 = torch.empty_like(self.X)
         self.err = torch.zeros(1, dtype=torch.float64, device=device)
         side = torch.cuda.Stream(device=device)
         side.wait_stream(torch.cuda.current_stream(device))
@@ -303,7 +316,12 @@ class TC2Graph:
         L = _lib.lib()
         st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
         src, dst = self.X, self.B
-        for _ in range(nsteps):
+        for k in range(nsteps):
+            if self.fused:
+                _lib.check(L.aimdhf_tc2_fused(self.n, _ptr(src), _ptr(dst), _ptr(self.sums[k % 2]),
+                                              _ptr(self.sums[1 - k % 2]), self.nocc, freeze, st))
+                src, dst = dst, src
+                continue
             torch.matmul(src, src, out=self.X2)
             _lib.check(L.aimdhf_tc2_step(self.n, ctypes.c_void_p(src.data_ptr()), ctypes.c_void_p(self.X2.data_ptr()),
                                          ctypes.c_void_p(dst.data_ptr()), self.nocc, freeze, st))
@@ -322,6 +340,8 @@ class TC2Graph:
         F = F.contiguous()
         _lib.check(_lib.lib().aimdhf_tc2_init(self.n, ctypes.c_void_p(F.data_ptr()), ctypes.c_void_p(self.X.data_ptr()),
                                               ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        if self.fused:
+            _lib.check(_lib.lib().aimdhf_tc2_sums(self.n, _ptr(self.X), _ptr(self.sums[0]), _stream()))
 
     def error(self) -> float:
         """|tr X - sum X_ij^2| of the current iterate (one kernel and one read)."""

@@ -1704,6 +1704,24 @@ int aimdhf_tc2_step(int n, const double* X, const double* X2, double* Xout, doub
     return AIMDHF_OK;
 }
 
+int aimdhf_tc2_sums(int n, const double* X, double* sums, void* stream) {
+    if (n <= 0 || n > 16384 || !X || !sums) return fail(AIMDHF_E_ARG, "bad tc2 arguments");
+    aimdhf::launch_tc2_sums(n, X, sums, (hipStream_t)stream);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(AIMDHF_E_HIP, std::string("tc2 sums: ") + hipGetErrorString(e));
+    return AIMDHF_OK;
+}
+
+int aimdhf_tc2_fused(int n, const double* X, double* Xout, const double* sums, double* sums_out, double nocc,
+                     double freeze, void* stream) {
+    if (n <= 0 || n > 16384 || !X || !Xout || X == Xout || !sums || !sums_out || sums == sums_out)
+        return fail(AIMDHF_E_ARG, "bad tc2 arguments");
+    aimdhf::launch_tc2_fused(n, X, Xout, sums, sums_out, nocc, freeze, (hipStream_t)stream);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(AIMDHF_E_HIP, std::string("tc2 fused: ") + hipGetErrorString(e));
+    return AIMDHF_OK;
+}
+
 int aimdhf_batch_set_jk_lanes(aimdhf_plan* p, int lanes) {
     if (!p) return fail(AIMDHF_E_ARG, "NULL plan");
     if (!p->batched) return fail(AIMDHF_E_STATE, "not a batched plan");

@@ -45,4 +45,9 @@ void launch_small_density(const SmallDensity& a, int nrep, hipStream_t st);
 void launch_small_inv_sqrt(int nrep, int ld, const double* S, double* X, int iters, double tol, double* out,
                            hipStream_t st);
 
+// sums: 2 doubles per 16 x 16 tile of the upper triangle
+void launch_tc2_sums(int n, const double* X, double* sums, hipStream_t st);
+void launch_tc2_fused(int n, const double* X, double* Xout, const double* sums, double* sums_out, double nocc,
+                      double freeze, hipStream_t st);
+
 }  // namespace aimdhf

@@ -251,6 +251,16 @@ int aimdhf_small_density(int nrep, int nspin, int ld, const double* X, const dou
                          int64_t* slot, int64_t* count, int m, void* stream);
 int aimdhf_small_inv_sqrt(int nmat, int ld, const double* S, double* X, int iters, double tol, double* out, void* stream);
 
+/*
+ * A purification step with its product in one launch: Xout as aimdhf_tc2_step for
+ * symmetric X (n <= 16384), the traces taken from X's tile sums (T = ceil(n / 16),
+ * T (T + 1) doubles) and Xout's written to sums_out; aimdhf_tc2_sums forms them for a
+ * first X. Xout is exactly symmetric.
+ */
+int aimdhf_tc2_sums(int n, const double* X, double* sums, void* stream);
+int aimdhf_tc2_fused(int n, const double* X, double* Xout, const double* sums, double* sums_out, double nocc,
+                     double freeze, void* stream);
+
 /* err[0] (device) = |tr X - sum_ij X_ij^2|, the idempotency error of a symmetric
  * purification iterate X (n x n, device). Row sums, then their sum in a fixed
  * order (bitwise reproducible); the row sums go through the same device array

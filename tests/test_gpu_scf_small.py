@@ -138,3 +138,29 @@ def test_inverse_square_root(ld):
     assert np.abs(X.cpu().numpy() - ref).max() < 1e-9
     res, low = out.cpu().numpy().T
     assert res.max() < 1e-10 and (low <= lam[:, 0] * (1 + 1e-9)).all() and (low * ld > lam[:, 0] * 0.99).all()
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 65, 304])
+def test_purification_step_in_one_launch(n):
+    import torch
+    from aimd_amd import _lib
+    L = _lib.lib()
+    rng = np.random.default_rng(n)
+    Q, _ = np.linalg.qr(rng.standard_normal((n, n)))
+    X = (Q * rng.uniform(0.0, 1.0, n)) @ Q.T
+    X = 0.5 * (X + X.T)
+    T = (n + 15) // 16
+    Xt = _dev(X)
+    out = torch.full_like(Xt, float("nan"))
+    sums, sums_out = torch.empty((2, 2, T * (T + 1) // 2), dtype=torch.float64, device="cuda")
+    _lib.check(L.aimdhf_tc2_sums(n, _ptr(Xt), _ptr(sums), _stream()))
+    tr, err = np.trace(X), abs(np.trace(X) - (X * X).sum())
+    # |X| <= 1: every sum of n products of one row and one column is below 1
+    tol = 8 * n * EPS
+    for nocc, freeze, ref in ((tr - 0.5, 0.0, X @ X), (tr + 0.5, 0.0, 2 * X - X @ X), (tr, 2 * err + 1.0, X)):
+        _lib.check(L.aimdhf_tc2_fused(n, _ptr(Xt), _ptr(out), _ptr(sums), _ptr(sums_out), nocc, freeze, _stream()))
+        o = out.cpu().numpy()
+        assert np.abs(o - ref).max() <= tol
+        np.testing.assert_array_equal(o, o.T)
+        s = sums_out.sum(dim=1).cpu().numpy()
+        assert abs(s[0] - np.trace(o)) < tol * n and abs(s[1] - (o * o).sum()) < tol * n
