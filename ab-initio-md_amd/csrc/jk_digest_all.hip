@@ -53,7 +53,7 @@ void launch_digest_all(const DigestArgs& a, int threads, hipStream_t st) {
     if (nl + nh > 1200) {
         if (nh > 0) k_digest_heavy<<<dim3(nh, a.nparts, a.nset), dim3(threads), lds, st>>>(a);
         if (nl > 0) k_digest_light<<<dim3(nl, a.nparts, a.nset), dim3(threads), lds, st>>>(a);
-    } else if (nl > 0)
+    } else if (nl + nh > 0)         // either may be zero: a basis of d shells alone has no light runs
         k_digest_all<<<dim3(nl + nh, a.nparts, a.nset), dim3(threads), lds, st>>>(a);
 }
 

@@ -1,0 +1,70 @@
+"""
+The single-read J/K digestion at the edges of its routes: bases of one angular
+momentum.
+"""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _table(l):
+    return {"H": [[l, [1.7, 0.4], [0.6, 0.7]]]}
+
+
+def _points(n, spacing=2.2, seed=0):
+    """n points of a cubic lattice, shaken."""
+    k = int(np.ceil(n ** (1.0 / 3.0)))
+    grid = np.array([[i, j, m] for i in range(k) for j in range(k) for m in range(k)][:n], float)
+    return spacing * grid + 0.2 * np.random.default_rng(seed).standard_normal((n, 3))
+
+
+def _dens(n, nset, seed=0):
+    import torch
+    D = np.random.default_rng(seed).standard_normal((nset, n, n))
+    return torch.tensor(D + D.transpose(0, 2, 1), device="cuda")
+
+
+@pytest.mark.parametrize("nset", [1, 2])
+@pytest.mark.parametrize("l,natm", [(0, 1), (0, 30), (1, 1), (1, 12), (2, 1), (2, 6), (2, 19), (2, 20)])
+def test_bases_of_one_angular_momentum(oracle_lib, l, natm, nset):
+    """One shell per atom, so one pair class and one to six quartet classes (19 and 20 d shells
+    lie on both sides of the rule that launches heavy and light classes apart), against the
+    oracle at 1e-11 as every other J/K test."""
+    from aimd_amd.qc.basis import basis_from_table
+    from aimd_amd.qc.engine import Engine
+    s, x = ["H"] * natm, _points(natm)
+    e = Engine(basis_from_table(s, x, _table(l)))
+    e.set_jk_mode("store")
+    e.set_geometry(x)
+    D = _dens(e.nao, nset, l)
+    J, K = e.jk(D)
+    Jo, Ko = oracle_lib.Pairs(oracle_lib.make_basis(s, x, _table(l))).jk_direct(D.cpu().numpy())
+    assert np.abs(Jo).max() > 1e-3 and np.abs(Ko).max() > 1e-3
+    np.testing.assert_allclose(J.cpu().numpy(), Jo, rtol=0, atol=1e-11)
+    np.testing.assert_allclose(K.cpu().numpy(), Ko, rtol=0, atol=1e-11)
+    e.close()
+
+
+@pytest.mark.parametrize("l", [0, 1, 2])
+def test_batches_of_one_angular_momentum(oracle_lib, monkeypatch, l):
+    import torch
+    import aimd_amd.batch as batch_module
+    from aimd_amd.qc.basis import basis_from_table
+    monkeypatch.setattr(batch_module, "build_basis", lambda s, x, name: basis_from_table(s, x, _table(l)))
+    sizes = [2, 3, 4]
+    xs = [_points(n, seed=n) for n in sizes]
+    batch = batch_module.ReplicaBatch([(["H"] * n, n % 2, 1) for n in sizes], jk_lanes=16)
+    batch._set_geometry(np.concatenate(xs))
+    n = batch.ld
+    D = torch.zeros((len(sizes), 2, n, n), dtype=torch.float64, device="cuda")
+    for r, nr in enumerate(batch.rep_nao):
+        D[r, :, :nr, :nr] = _dens(int(nr), 2, r)
+    batch._jk(D)
+    for r, (nr, x) in enumerate(zip(batch.rep_nao, xs)):
+        ob = oracle_lib.make_basis(["H"] * sizes[r], x, _table(l))
+        Jo, Ko = oracle_lib.Pairs(ob).jk_direct(D[r, :, :nr, :nr].cpu().numpy())
+        np.testing.assert_allclose(batch.J[r, :, :nr, :nr].cpu().numpy(), Jo, rtol=0, atol=1e-11)
+        np.testing.assert_allclose(batch.K[r, :, :nr, :nr].cpu().numpy(), Ko, rtol=0, atol=1e-11)
+    batch.close()
