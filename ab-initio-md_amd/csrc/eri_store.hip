@@ -118,9 +118,17 @@ void launch_part(const EriArgs& a, Real* out, long long n, long long nh, hipStre
     nh = (nh + 63) / 64 * 64;
     if (nh > n) nh = n;
     if constexpr (WH > 1) {
-        if (nh > 0)
+        // a launch takes fewer than 2^32 work-items, and past that the grid wraps without an
+        // error: at most 2^21 workgroups (of up to 1024) at a time
+        constexpr long long SLICE = (1 << 21) / NSPLIT * 64;
+        for (long long q0 = 0; q0 < nh; q0 += SLICE) {
+            EriArgs b = a;
+            b.lbra += q0;
+            b.lket += q0;
+            const long long nq = q0 + SLICE < nh ? SLICE : nh - q0;
             k_eri_split<LA, LB, LC, LD, Real>
-                <<<dim3((unsigned)((nh + 63) / 64 * NSPLIT)), dim3(64 * WH), 0, st>>>(a, out, nh);
+                <<<dim3((unsigned)((nq + 63) / 64 * NSPLIT)), dim3(64 * WH), 0, st>>>(b, out + q0 * BLK, nq);
+        }
     }
     if (n > nh) {
         EriArgs b = a;

@@ -1,6 +1,6 @@
 """
 The single-read J/K digestion at the edges of its routes: bases of one angular
-momentum.
+momentum, integral lists past the size of one launch.
 """
 
 import numpy as np
@@ -68,3 +68,24 @@ def test_batches_of_one_angular_momentum(oracle_lib, monkeypatch, l):
         np.testing.assert_allclose(batch.J[r, :, :nr, :nr].cpu().numpy(), Jo, rtol=0, atol=1e-11)
         np.testing.assert_allclose(batch.K[r, :, :nr, :nr].cpu().numpy(), Ko, rtol=0, atol=1e-11)
     batch.close()
+
+
+def test_more_contracted_quartets_than_one_launch_takes(oracle_lib):
+    """220 hydrogen atoms, STO-3G, no screening: 295 million contracted (ss|ss) quartets in the
+    store, more tiles than a grid of 1024-thread workgroups may have. Ten bohr apart, so
+    that most pairs keep no primitive and the oracle walks them quickly."""
+    from aimd_amd.qc.basis import build_basis
+    from aimd_amd.qc.engine import Engine
+    n = 220
+    s, x = ["H"] * n, _points(n, 10.0)
+    e = Engine(build_basis(s, x, "sto-3g"))
+    e.set_jk_mode("store")
+    e.set_geometry(x, 0.0)
+    npair = n * (n + 1) // 2
+    assert e.quartet_count() == npair * (npair + 1) // 2 > (1 << 32) // 1024 * 64
+    D = _dens(n, 1, 3)
+    J, K = e.jk(D)
+    Jo, Ko = oracle_lib.Pairs(oracle_lib.make_basis(s, x, "sto-3g")).jk_direct(D.cpu().numpy(), 0.0)
+    np.testing.assert_allclose(J.cpu().numpy(), Jo, rtol=0, atol=1e-11)
+    np.testing.assert_allclose(K.cpu().numpy(), Ko, rtol=0, atol=1e-11)
+    e.close()
