@@ -557,54 +557,77 @@ struct aimdhf_plan {
         ensure_digest(1);
     }
 
-    // Direct mode: the list cut into pieces whose integrals fit a bounded buffer (a class is
-    // split at multiples of 64 quartets); a J/K build evaluates and digests piece by piece
+    // Direct mode: the list cut into pieces whose integrals fit a bounded buffer; a J/K build
+    // evaluates and digests piece by piece. Cuts lie between the runs of a class (a lane sums its
+    // share of a whole run in FP64 before it is rounded), and a piece is evaluated from the start of
+    // the tile that its first run begins in (up to 63 quartets again), so neither a quartet's
+    // arithmetic nor a sum depends on where the cuts lie: J and K do not depend on the buffer's size.
     struct Piece {
-        long long lo[NQCLASS], hi[NQCLASS];
+        long long base[NQCLASS], lo[NQCLASS], hi[NQCLASS];     // evaluated from base, digested from lo
         size_t at[NQCLASS];
     };
     std::vector<Piece> pieces;
-    void build_direct(hipStream_t) {
+    void build_direct(hipStream_t st) {
         size_t fr = 0, tot = 0;
         HIPCHECK(hipMemGetInfo(&fr, &tot));
         size_t cap = std::min<size_t>((size_t)1 << 30, std::max<size_t>(fr / 8 + d_store.bytes, (size_t)1 << 20));
         if (store_limit > 0) cap = std::min<size_t>(cap, std::max<size_t>((size_t)store_limit, (size_t)1 << 26));
+        // first quartet of every run, where the list does not fit as a whole
+        std::vector<long long> starts;
+        if (store_need > cap) {
+            starts.resize(runbase[NQCLASS]);
+            aimdhf::launch_run_starts(d_loff.as<long long>(), runbase[NQCLASS], d_lcnt.as<long long>(), st);
+            HIPCHECK(hipGetLastError());
+            HIPCHECK(hipMemcpyAsync(starts.data(), d_lcnt.p, sizeof(long long) * starts.size(), hipMemcpyDeviceToHost, st));
+            HIPCHECK(hipStreamSynchronize(st));
+        }
         pieces.clear();
         Piece cur{};
         size_t used = 0, most = 1;
+        auto close = [&] {
+            if (used > 0) pieces.push_back(cur);
+            cur = Piece{};
+            used = 0;
+        };
         for (int k = 0; k < NQCLASS; ++k) {
             const size_t tile = sizeof(double) * 64 * (size_t)aimdhf::store_block(k);
-            long long pos = list_off[k], left = qcount[k];
-            while (left > 0) {
-                const long long room = (long long)((cap - used) / tile) * 64;
-                if (room == 0) {
-                    pieces.push_back(cur);
-                    cur = Piece{};
-                    used = 0;
-                    continue;
+            const long long end = list_off[k] + qcount[k];
+            const auto r0 = starts.begin() + (starts.empty() ? 0 : runbase[k]);
+            const auto r1 = starts.begin() + (starts.empty() ? 0 : runbase[k + 1]);
+            for (long long pos = list_off[k]; pos < end;) {
+                const long long base = pos - (pos - list_off[k]) % 64;
+                const long long fit = base + (long long)((cap - std::min(used, cap)) / tile) * 64;
+                long long hi = end;
+                if (fit < end) {        // the last run boundary that fits
+                    const auto r = std::upper_bound(r0, r1, fit);
+                    hi = r == r0 ? pos : *(r - 1);
                 }
-                const long long n = std::min(left, room);
+                if (hi <= pos) {
+                    if (used > 0) {
+                        close();
+                        continue;
+                    }
+                    const auto r = std::upper_bound(r0, r1, pos);   // a run longer than the buffer enlarges it
+                    hi = r == r1 ? end : *r;
+                }
+                cur.base[k] = base;
                 cur.lo[k] = pos;
-                cur.hi[k] = pos + n;
+                cur.hi[k] = hi;
                 cur.at[k] = used;
-                used += (size_t)((n + 63) / 64) * tile;
+                used += (size_t)((hi - base + 63) / 64) * tile;
                 most = std::max(most, used);
-                pos += n;
-                left -= n;
-                if (left > 0) {         // one range of a class per piece
-                    pieces.push_back(cur);
-                    cur = Piece{};
-                    used = 0;
-                }
+                pos = hi;
+                if (pos < end) close();         // one range of a class per piece
             }
         }
-        if (used > 0) pieces.push_back(cur);
+        close();
         d_store.ensure(most);
         std::vector<aimdhf::DigestGeo> geo(std::max<size_t>(pieces.size(), 1) * NQCLASS);
         for (size_t c = 0; c < pieces.size(); ++c)
             for (int k = 0; k < NQCLASS; ++k) {
                 aimdhf::DigestGeo& g = geo[c * NQCLASS + k];
-                g.t64 = g.lo64 = pieces[c].lo[k];
+                g.t64 = pieces[c].base[k];
+                g.lo64 = pieces[c].lo[k];
                 g.hi64 = g.t32 = g.lo32 = g.hi32 = pieces[c].hi[k];
                 g.off = d_loff.as<long long>() + runbase[k] * aimdhf::LIST_WAVES;
                 g.lket = d_lket.as<int>();
@@ -1426,12 +1449,12 @@ static int jk_direct(aimdhf_plan* p, int nset, const double* dens, double* J, do
             p->fan.fork(st);
             int i = 0;
             for (int k = NQCLASS - 1; k >= 0; --k) {
-                const long long n = pc.hi[k] - pc.lo[k];
-                if (n <= 0) continue;
+                if (pc.hi[k] <= pc.lo[k]) continue;
+                const long long n = pc.hi[k] - pc.base[k];
                 hipStream_t s2 = p->fan.on(i++);
-                aimdhf::EriArgs ea = p->eri_args(k, pc.lo[k]);
+                aimdhf::EriArgs ea = p->eri_args(k, pc.base[k]);
                 ea.out64 = (double*)(p->d_store.as<char>() + pc.at[k]);
-                const long long h = p->list_off[k] + p->h64count[k] - pc.lo[k];
+                const long long h = p->list_off[k] + p->h64count[k] - pc.base[k];
                 p->prof.time(46, s2, [&] { aimdhf::launch_eri(k, ea, n, std::min(std::max(h, 0LL), n), 0, 0, s2); });
                 aimdhf::DigestArgs da = p->digest_args(k, nset, false, 0.0);
                 da.geo += c * NQCLASS;

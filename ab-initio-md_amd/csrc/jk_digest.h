@@ -124,6 +124,8 @@ struct PickArgs {
     long long at[128];
 };
 void launch_pick(const PickArgs& a, const long long* off, long long* out, hipStream_t st);
+// out[r] = first quartet of run r
+void launch_run_starts(const long long* off, long long nrun, long long* out, hipStream_t st);
 
 // n64 FP64 quartets from the list position of a, n32 FP32 ones after them; the first h64 / h32
 // of each have contracted bras (ERI_HEAVY primitive pairs or more)

@@ -179,6 +179,11 @@ __global__ void k_pick(PickArgs a, const long long* off, long long* out) {
     if ((int)threadIdx.x < a.n) out[threadIdx.x] = off[a.at[threadIdx.x]];
 }
 
+__global__ __launch_bounds__(256) void k_run_starts(const long long* off, long long nrun, long long* out) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i < nrun) out[i] = off[i * LIST_WAVES];
+}
+
 // Screening values by rank, and per replica what bounds J and K: the largest q,
 // the largest sum of q^2 over a row of AO pairs and the sum over all of them
 // (in 2^20 fixed point, rounded up: an integer sum does not depend on the
@@ -239,6 +244,10 @@ void launch_list_scan(const long long* in, long long* out, long long n, long lon
 
 void launch_pick(const PickArgs& a, const long long* off, long long* out, hipStream_t st) {
     k_pick<<<dim3(1), dim3(128), 0, st>>>(a, off, out);
+}
+
+void launch_run_starts(const long long* off, long long nrun, long long* out, hipStream_t st) {
+    if (nrun > 0) k_run_starts<<<dim3((unsigned)((nrun + 255) / 256)), dim3(256), 0, st>>>(off, nrun, out);
 }
 
 void launch_geo_bounds(const GeoArgs& a, hipStream_t st) {

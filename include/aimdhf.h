@@ -122,9 +122,11 @@ int aimdhf_quartets(aimdhf_plan* plan, int64_t* out_host, int64_t cap, int64_t* 
  *   J_mn = sum_ls (mn|ls) D_ls,   K_mn = sum_ls (ml|ns) D_ls
  * of the symmetric part of each D over the screened quartets, bitwise
  * reproducible run to run. Store mode reads each stored integral once, direct
- * mode evaluates the list piece by piece into a bounded buffer (at most 1 GiB, an
- * eighth of the free memory, or max_store_bytes if that is set and above 64 MiB)
- * and digests each piece; sums are 64-bit fixed point whose exponent follows the
+ * mode evaluates the list piece by piece into a bounded buffer and digests each
+ * piece. The buffer takes at most 1 GiB, an eighth of the free memory beyond what
+ * it holds already, and max_store_bytes if that is set (64 MiB at least), or the
+ * run of kets of one bra where that is longer; J and K do not depend on its size.
+ * Sums are 64-bit fixed point whose exponent follows the
  * density and the Schwarz bounds (resolution 2^-62 of a bound of the largest element; a density with a NaN or
  * infinity gives NaN in its J and K).
  * Replaces: jk_from_eri (aimd/qc/integrals.py:1009-1044) and, in direct mode,

@@ -1,10 +1,12 @@
 """
 The single-read J/K digestion at the edges of its routes: bases of one angular
-momentum, integral lists past the size of one launch.
+momentum, integral lists past the size of one launch, direct mode's pieces.
 """
 
 import numpy as np
 import pytest
+
+from tests.conftest import cluster
 
 pytestmark = pytest.mark.gpu
 
@@ -88,4 +90,50 @@ def test_more_contracted_quartets_than_one_launch_takes(oracle_lib):
     Jo, Ko = oracle_lib.Pairs(oracle_lib.make_basis(s, x, "sto-3g")).jk_direct(D.cpu().numpy(), 0.0)
     np.testing.assert_allclose(J.cpu().numpy(), Jo, rtol=0, atol=1e-11)
     np.testing.assert_allclose(K.cpu().numpy(), Ko, rtol=0, atol=1e-11)
+    e.close()
+
+
+@pytest.mark.parametrize("nset", [1, 2])
+def test_direct_mode_does_not_depend_on_its_buffer(nset):
+    """J and K of direct mode bit for bit the same whatever buffer the pieces are cut for: the
+    smallest (64 MiB, runs of some classes longer than what is left of it), others, and one
+    that holds the whole list; and again at the same geometry."""
+    import torch
+    from aimd_amd.qc.basis import build_basis
+    from aimd_amd.qc.engine import Engine
+    s, x = cluster("water8.xyz")
+    e = Engine(build_basis(s, x, "6-31g*"))
+    D = _dens(e.nao, nset, 7)
+    ref = None
+    for limit in (0, 1, 1, 70_000_000, 100_000_000, 0):
+        e.set_jk_mode("direct", limit)
+        e.set_geometry(x)
+        out = e.jk(D)
+        ref = ref or out
+        for a, b in zip(ref, out):
+            assert torch.equal(a, b), limit
+    e.close()
+
+
+def test_direct_mode_with_a_run_longer_than_its_buffer():
+    """One far d shell with coefficients that lift only its quartets over the threshold: its
+    (d d| run holds 240 thousand (s s| kets, 67 MB of integrals, more than the 64 MiB
+    buffer. Direct mode takes the run whole, so it adds what store mode adds, bit for bit."""
+    import torch
+    from aimd_amd.qc.basis import BasisSet
+    from aimd_amd.qc.engine import Engine
+    n = 701
+    x = np.concatenate([_points(n - 1, 1.0), [[400.0, 0.0, 0.0]]])
+    b = BasisSet("custom", ["H"] * n, x, np.arange(n), [0] * (n - 1) + [2], np.arange(n + 1), [0.05] * (n - 1) + [1.0],
+                 [0.07] * (n - 1) + [1e3])
+    e = Engine(b)
+    D = _dens(e.nao, 1, 9)
+    out = []
+    for mode in ("store", "direct"):
+        e.set_jk_mode(mode, 1)
+        e.set_geometry(x, 10.0)
+        out.append(e.jk(D))
+    assert e.class_counts()[0][15] * 36 * 8 > 64 << 20          # (d d|s s)
+    for a, c in zip(*out):
+        assert float(a.abs().max()) > 0.0 and torch.equal(a, c)
     e.close()
