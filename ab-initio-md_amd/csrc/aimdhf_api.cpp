@@ -682,7 +682,7 @@ struct aimdhf_plan {
         }
         a.npao = npao;
         a.kstride = (long long)(mat_elems() * nset);
-        a.oab = d_oab.as<int>();
+        a.oab = d_oab.as<unsigned>();
         a.rank_rep = batched ? d_rank_rep.as<int>() : nullptr;
         a.rep_nao = batched ? d_rep_nao.as<int>() : nullptr;
         a.dens = dens;
@@ -710,7 +710,7 @@ struct aimdhf_plan {
         a.nparts = list_parts;
         a.unit = unit_items;
         a.nchunk = batched ? 1 : (int)std::min<long long>(16, std::max<long long>(1, nk / (8LL * unit_items)));
-        a.oab = d_oab.as<int>();
+        a.oab = d_oab.as<unsigned>();
         a.rank_rep = batched ? d_rank_rep.as<int>() : nullptr;
         a.dsym = d_dsym.as<double>();
         a.dket = d_dket.as<double>();
@@ -994,11 +994,11 @@ static int create_plan(int natm, int nshell, const int64_t* shell_atom, const in
         }
         // AO offsets and replica of every rank, rank range of every (class, replica), and
         // the base of every class's components
-        std::vector<int> oab(p->npair), rank_rep(p->npair), seg(6 * p->nrep + 1, p->npair);
+        std::vector<unsigned> oab(p->npair);
+        std::vector<int> rank_rep(p->npair), seg(6 * p->nrep + 1, p->npair);
         for (int r = p->npair - 1; r >= 0; --r) {
             const int Q = p->cls_pairs[r], a = p->pair_a[Q], b = p->pair_b[Q];
-            oab[r] = (p->shell_ao[a] & aimdhf::OAB_MASK) | (p->shell_ao[b] & aimdhf::OAB_MASK) << 14 |
-                     (a == b ? aimdhf::OAB_SAME : 0);
+            oab[r] = aimdhf::oab_pack(p->shell_ao[a], p->shell_ao[b]);
             rank_rep[r] = p->shell_rep[a];
             seg[p->pair_cls[Q] * p->nrep + rank_rep[r]] = r;
         }
@@ -1248,6 +1248,10 @@ int aimdhf_set_geometry(aimdhf_plan* p, const double* positions, double thr, voi
     hipStream_t st = (hipStream_t)stream;
     p->have_last_store = false;     // the store's buffers may move
     if (p->generic) return set_geometry_generic(p, positions, thr, st);
+    // 16-bit offsets of the quartet list (J, K, the density and its copies of a larger
+    // matrix, 34 GB each, would not fit)
+    if (p->matrix_ld() > aimdhf::MAX_LD)
+        return fail(AIMDHF_E_UNSUPPORTED, "matrices of more than " + std::to_string(aimdhf::MAX_LD) + " AOs");
     try {
         p->pos.assign(positions, positions + 3 * p->natm);
         HIPCHECK(hipMemcpyAsync(p->d_pos.p, positions, sizeof(double) * 3 * p->natm, hipMemcpyHostToDevice, st));
@@ -1273,10 +1277,6 @@ int aimdhf_set_geometry(aimdhf_plan* p, const double* positions, double thr, voi
             return AIMDHF_OK;
         }
         bool store = false;
-        if (p->nao >= (1 << 14)) {
-            p->have_geometry = false;
-            return fail(AIMDHF_E_UNSUPPORTED, "more than 16383 AOs");
-        }
         if (p->jk_mode != 1) {
             long long limit = p->store_limit;
             if (limit <= 0) {

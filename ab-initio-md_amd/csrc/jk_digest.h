@@ -43,9 +43,12 @@ struct EriArgs {
     float* out32;                   // (t / 64) 64 NAB NCD + 64 v + t % 64
 };
 
-// AO offsets of a ranked pair's shells and whether they are the same shell
-constexpr int OAB_MASK = (1 << 14) - 1;
-constexpr int OAB_SAME = 1 << 28;
+// AO offsets of a ranked pair's shells (within the replica), 16 bits each; equal offsets are the same shell
+constexpr int MAX_LD = (1 << 16) - 1;
+__host__ __device__ inline unsigned oab_pack(int first, int second) { return (unsigned)first | (unsigned)second << 16; }
+__host__ __device__ inline int oab_first(unsigned o) { return (int)(o & 0xffffu); }
+__host__ __device__ inline int oab_second(unsigned o) { return (int)(o >> 16); }
+__host__ __device__ inline bool oab_same(unsigned o) { return oab_first(o) == oab_second(o); }
 
 // What of a digestion depends on the geometry; read from device memory, so a captured
 // launch stays valid when the geometry moves (batched SCF iterations are replayed)
@@ -65,7 +68,7 @@ struct DigestArgs {
     int nparts, nchunk, unit;       // pieces a long run is cut into, each of at least unit quartets
     int cls_off[7];                 // rank range and component base (dket / jacc) of each pair class
     long long koff[7];
-    const int* oab;                 // by rank
+    const unsigned* oab;            // by rank
     const int* rank_rep;
     const double* dsym;             // (nrep, nset, ld, ld)
     const double* dket;             // (nset, npao): densities by pair component
@@ -87,7 +90,7 @@ struct PrepArgs {
     int cls_off[7];
     long long koff[7];              // component base of each pair class
     long long npao, kstride;
-    const int* oab;
+    const unsigned* oab;
     const int* rank_rep;
     const int* rep_nao;
     const double* dens;

@@ -96,7 +96,8 @@ __device__ __forceinline__ void digest_part(const DigestArgs& a, const Rows<QC, 
     auto ket_at = [&](int it) { return lket[t0 + (SP > 1 ? it % n : it)]; };
     // the ket and its AO offsets run one item ahead, so that an item's loads and
     // LDS addresses do not wait for them
-    int kr_next = 0, o_next = 0;
+    int kr_next = 0;
+    unsigned o_next = 0;
     if ((int)threadIdx.x < nit) {
         kr_next = ket_at(threadIdx.x);
         o_next = a.oab[kr_next];
@@ -104,7 +105,8 @@ __device__ __forceinline__ void digest_part(const DigestArgs& a, const Rows<QC, 
     for (int it = threadIdx.x; it < nit; it += blockDim.x) {
         const int c0 = SP > 1 ? it / n : 0;
         const int tt = SP > 1 ? it - c0 * n : it;
-        const int kr = kr_next, o = o_next;
+        const int kr = kr_next;
+        const unsigned o = o_next;
         const int it2 = it + blockDim.x;
         if (it2 < nit) {
             kr_next = ket_at(it2);
@@ -112,8 +114,8 @@ __device__ __forceinline__ void digest_part(const DigestArgs& a, const Rows<QC, 
         }
         // a density difference below the threshold for all 64 kets of the wavefront
         if (a.delta && !__any(!(qb * a.rq[kr] < a.dthr))) continue;
-        const int oK = o & OAB_MASK, oL = (o >> 14) & OAB_MASK;
-        double w = o & OAB_SAME ? 0.5 * wbra : wbra;
+        const int oK = oab_first(o), oL = oab_second(o);
+        double w = oab_same(o) ? 0.5 * wbra : wbra;
         if (CB == CK && kr == rank) w *= 0.5;
         const long long t = t0 + tt - tb;
         const Real* __restrict__ p = blocks + (t >> 6) * (64 * BLK) + (t & 63);
@@ -221,12 +223,12 @@ __device__ __forceinline__ void digest_run(const DigestArgs& a, int bi, int part
     const int rep = a.rank_rep ? a.rank_rep[rank] : 0;
     const size_t ld2 = (size_t)a.ld * a.ld;
     const int nao = a.rep_nao ? a.rep_nao[rep] : a.ld;
-    const int o = a.oab[rank];
+    const unsigned o = a.oab[rank];
     double sj[NSET], dm = 0.0;
     Rows<QC, NSET, LDSROWS> R;
     R.ld = a.ld;
-    R.oI = o & OAB_MASK;
-    R.oJ = (o >> 14) & OAB_MASK;
+    R.oI = oab_first(o);
+    R.oJ = oab_second(o);
 #pragma unroll
     for (int s = 0; s < NSET; ++s) {
         const size_t mat = (size_t)rep * a.nset + set0 + s;
@@ -261,7 +263,7 @@ __device__ __forceinline__ void digest_run(const DigestArgs& a, int bi, int part
         sD[i] = a.dket[(set0 + s) * a.npao + kbra + (long long)ab * nb + bi] * (s ? sj[NSET - 1] : sj[0]);
     }
     __syncthreads();
-    const double wbra = o & OAB_SAME ? 0.5 : 1.0;
+    const double wbra = oab_same(o) ? 0.5 : 1.0;
     double jacc[NSET][NAB];
 #pragma unroll
     for (int s = 0; s < NSET; ++s)

@@ -67,8 +67,9 @@ __global__ __launch_bounds__(256) void k_jk_prep(PrepArgs a, int nrow, int npc) 
         const long long e = (long long)(b - nrow) * 256 + threadIdx.x;
         const bool in = e < a.npao;
         const PairComp p = pair_comp(a, in ? e : a.npao - 1);
-        const int o = a.oab[p.rank], nb = nc_of(p.cls);
-        const size_t m = (o & OAB_MASK) + p.comp / nb, n = ((o >> 14) & OAB_MASK) + p.comp % nb;
+        const unsigned o = a.oab[p.rank];
+        const int nb = nc_of(p.cls);
+        const size_t m = oab_first(o) + p.comp / nb, n = oab_second(o) + p.comp % nb;
         const int rep = a.rank_rep ? a.rank_rep[p.rank] : 0;
         const bool one = __all(rep == __shfl(rep, 0, 64));
         for (int s = 0; s < a.nset; ++s) {
@@ -78,7 +79,7 @@ __global__ __launch_bounds__(256) void k_jk_prep(PrepArgs a, int nrow, int npc) 
             if (in) a.dket[s * a.npao + e] = d;
             // sum of q |D| over AO pairs in both orders, in integers (order-independent)
             unsigned long long x = 0;
-            if (in) x = (unsigned long long)ceil(fmin(fabs(d) * a.rq[p.rank] * (o & OAB_SAME ? 1.0 : 2.0), 1e10) * 16777216.0);
+            if (in) x = (unsigned long long)ceil(fmin(fabs(d) * a.rq[p.rank] * (oab_same(o) ? 1.0 : 2.0), 1e10) * 16777216.0);
             unsigned long long* cell = a.dcell + JK_CELLS * mat + 3;
             if (one) {
 #pragma unroll
@@ -121,10 +122,11 @@ __global__ __launch_bounds__(256) void k_jk_finish(PrepArgs a, int nkb) {
     const long long e = (long long)(blockIdx.x - nkb) * 256 + threadIdx.x;
     if (e >= a.npao) return;
     const PairComp p = pair_comp(a, e);
-    const int o = a.oab[p.rank], nb = nc_of(p.cls);
+    const unsigned o = a.oab[p.rank];
+    const int nb = nc_of(p.cls);
     const int i = p.comp / nb, j = p.comp % nb;
-    const bool same = o & OAB_SAME;
-    const size_t m = (o & OAB_MASK) + i, n = ((o >> 14) & OAB_MASK) + j;
+    const bool same = oab_same(o);
+    const size_t m = oab_first(o) + i, n = oab_second(o) + j;
     const size_t rep = a.rank_rep ? a.rank_rep[p.rank] : 0;
     const long long et = same ? e + (long long)((j * nb + i) - p.comp) * p.stride : e;
     for (int s = 0; s < a.nset; ++s) {

@@ -96,7 +96,8 @@ int aimdhf_batch_layout(aimdhf_plan* plan, int* nrep, int* ld, int64_t* tensor_b
  * shell quartets whose contraction-block pairs satisfy Q_P Q_Q >= threshold.
  * In store mode (aimdhf_set_jk_mode) the screened quartets are also evaluated
  * here into a device-resident integral store that every J/K build reads once.
- * Synchronises the stream (the list sizes come back to the host).
+ * Synchronises the stream (the list sizes come back to the host). Matrices of more
+ * than 65535 AOs are refused (l <= 2).
  * Replaces: BasisSet.with_positions (aimd/qc/basis.py:242-246), _build_pairs
  * (aimd/qc/integrals.py:525-599), schwarz_bounds (aimd/qc/integrals.py:970-983)
  * and the screening loop of _eri_tensor_kernel (aimd/qc/integrals.py:900-903);

@@ -1,6 +1,7 @@
 """
 The single-read J/K digestion at the edges of its routes: bases of one angular
-momentum, integral lists past the size of one launch, direct mode's pieces.
+momentum, integral lists past the size of one launch, direct mode's pieces,
+matrices of more than 16384 orbitals.
 """
 
 import numpy as np
@@ -137,3 +138,43 @@ def test_direct_mode_with_a_run_longer_than_its_buffer():
     for a, c in zip(*out):
         assert float(a.abs().max()) > 0.0 and torch.equal(a, c)
     e.close()
+
+
+@pytest.mark.parametrize("mode", ["auto", "direct"])
+def test_more_than_16384_orbitals(mode):
+    """2732 d shells (16392 AOs, 3.7 million pairs), of which the last three sit close together
+    and are the only ones tight enough for the threshold: J and K in their block equal those
+    of the three atoms alone. The screening value of a lone shell grows as the fourth root
+    of its exponent (products of two: 1, 2 and 4 for exponents 1 and 16)."""
+    import torch
+    from aimd_amd.qc.basis import BasisSet
+    from aimd_amd.qc.engine import Engine
+    n, tail = 2732, 3
+    near = np.array([[0.0, 0.0, 0.0], [0.3, 0.1, 0.0], [0.0, 0.2, 0.25]])
+    x = np.concatenate([_points(n - tail, 40.0), near - 100.0])
+    ex = np.where(np.arange(n) < n - tail, 1.0, 16.0)
+
+    def engine(pos, exps):
+        m = len(exps)
+        b = BasisSet("d", ["H"] * m, pos, np.arange(m), np.full(m, 2), np.arange(m + 1), exps, 0.7 * exps ** 1.75)
+        e = Engine(b)
+        e.set_jk_mode(mode)
+        return e
+
+    small = engine(x[-tail:], ex[-tail:])
+    small.set_geometry(x[-tail:], 0.0)
+    q = small.schwarz_bounds()
+    thr = 0.75 * q[0] ** 2
+    small.set_geometry(x[-tail:], thr)
+    e = engine(x, ex)
+    e.set_geometry(x, thr)
+    assert e.nao == 16392 and e.quartet_count() == small.quartet_count() >= 6
+    D = torch.zeros((1, e.nao, e.nao), dtype=torch.float64, device="cuda")
+    m = 6 * tail
+    D[0, -m:, -m:] = _dens(m, 1, 5)[0]
+    J, K = e.jk(D)
+    for got, ref in zip((J, K), small.jk(D[:, -m:, -m:].contiguous())):
+        assert float((got[:, -m:, -m:] - ref).abs().max()) < 1e-12 * float(ref.abs().max())
+        assert float(got[:, :-m].abs().max()) == 0.0
+    e.close()
+    small.close()
