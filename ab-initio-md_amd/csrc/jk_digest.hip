@@ -21,8 +21,8 @@ constexpr int MAXT = QC == 4 || QC == 5 || QC == 8 || QC >= 16 ? 256 : 512;
 constexpr bool BOTH = QC < 5;
 
 template <int QC_, int NSET, bool LDSROWS>
-__global__ __launch_bounds__(MAXT) void k_digest(DigestArgs a) {
-    digest_run<QC_, NSET, LDSROWS>(a, blockIdx.x, blockIdx.y / a.nchunk, blockIdx.y % a.nchunk, blockIdx.z * NSET,
+__global__ __launch_bounds__(MAXT) void k_digest(DigestArgs a, int bra0) {
+    digest_run<QC_, NSET, LDSROWS>(a, bra0 + blockIdx.x, blockIdx.y / a.nchunk, blockIdx.y % a.nchunk, blockIdx.z * NSET,
                                    (int)((blockIdx.y * gridDim.x + blockIdx.x) % a.ncopy));
 }
 
@@ -31,15 +31,18 @@ void launch(const DigestArgs& a, int nb, int threads, hipStream_t st) {
     using S = Dig<QC>;
     const size_t head = sizeof(double) * S::head(NSET);
     const size_t rows = head + sizeof(double) * S::colw(NSET) * (size_t)a.ld;
-    const dim3 grid(nb, a.nparts * a.nchunk, a.nset / NSET);
-    if (rows <= (size_t)a.lds_limit) {
-        if (threads == 256 && rows > 40 * 1024) threads = MAXT;
-        if (rows > 60 * 1024)
-            (void)hipFuncSetAttribute((const void*)k_digest<QC, NSET, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)rows);
-        k_digest<QC, NSET, true><<<grid, dim3(threads), rows, st>>>(a);
-    } else
-        k_digest<QC, NSET, false><<<grid, dim3(threads), head, st>>>(a);
+    const bool fit = rows <= (size_t)a.lds_limit;
+    if (fit && threads == 256 && rows > 40 * 1024) threads = MAXT;
+    if (fit && rows > 60 * 1024)
+        (void)hipFuncSetAttribute((const void*)k_digest<QC, NSET, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)rows);
+    // bras in slices: a grid of 2^32 work-items or more wraps without an error
+    constexpr int SLICE = 1 << 21;
+    for (int b0 = 0; b0 < nb; b0 += SLICE) {
+        const dim3 grid(nb - b0 < SLICE ? nb - b0 : SLICE, a.nparts * a.nchunk, a.nset / NSET);
+        if (fit) k_digest<QC, NSET, true><<<grid, dim3(threads), rows, st>>>(a, b0);
+        else k_digest<QC, NSET, false><<<grid, dim3(threads), head, st>>>(a, b0);
+    }
 }
 
 }  // namespace

@@ -34,8 +34,8 @@ __device__ __forceinline__ void for_segments(const QListArgs& a, int rank, int w
     }
 }
 
-__global__ __launch_bounds__(64 * LIST_WAVES) void k_qlist_count(QListArgs a) {
-    const int rank = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+__device__ __forceinline__ void qlist_count(const QListArgs& a, int rank) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const double qb = a.rq[rank];
     for_segments(a, rank, w, [&](int b0, int b1, long long run, long long nb) {
         long long c0 = 0, c1 = 0;
@@ -65,8 +65,8 @@ __global__ __launch_bounds__(64 * LIST_WAVES) void k_qlist_count(QListArgs a) {
     });
 }
 
-__global__ __launch_bounds__(64 * LIST_WAVES) void k_qlist_fill(QListArgs a) {
-    const int rank = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+__device__ __forceinline__ void qlist_fill(const QListArgs& a, int rank) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const double qb = a.rq[rank];
     const unsigned long long below = lane ? (~0ull >> (64 - lane)) : 0ull;
     for_segments(a, rank, w, [&](int b0, int b1, long long run, long long nb) {
@@ -96,6 +96,14 @@ __global__ __launch_bounds__(64 * LIST_WAVES) void k_qlist_fill(QListArgs a) {
             }
         }
     });
+}
+
+__global__ __launch_bounds__(64 * LIST_WAVES) void k_qlist_count(QListArgs a) {
+    for (int rank = blockIdx.x; rank < a.npair; rank += gridDim.x) qlist_count(a, rank);
+}
+
+__global__ __launch_bounds__(64 * LIST_WAVES) void k_qlist_fill(QListArgs a) {
+    for (int rank = blockIdx.x; rank < a.npair; rank += gridDim.x) qlist_fill(a, rank);
 }
 
 // three-pass exclusive scan: block scans, a scan of the block totals, the add
@@ -225,12 +233,16 @@ __global__ void k_zero_cells(unsigned long long* p, int n) {
 
 }  // namespace
 
+// a grid of 2^32 work-items or more (16.8 million pairs) wraps without an error: workgroups
+// take every GRID_MAX-th pair from there on
+constexpr int GRID_MAX = 1 << 21;
+
 void launch_qlist_count(const QListArgs& a, hipStream_t st) {
-    if (a.npair > 0) k_qlist_count<<<dim3(a.npair), dim3(64 * LIST_WAVES), 0, st>>>(a);
+    if (a.npair > 0) k_qlist_count<<<dim3(a.npair < GRID_MAX ? a.npair : GRID_MAX), dim3(64 * LIST_WAVES), 0, st>>>(a);
 }
 
 void launch_qlist_fill(const QListArgs& a, hipStream_t st) {
-    if (a.npair > 0) k_qlist_fill<<<dim3(a.npair), dim3(64 * LIST_WAVES), 0, st>>>(a);
+    if (a.npair > 0) k_qlist_fill<<<dim3(a.npair < GRID_MAX ? a.npair : GRID_MAX), dim3(64 * LIST_WAVES), 0, st>>>(a);
 }
 
 long long list_scan_blocks(long long n) { return (n + SCAN_B - 1) / SCAN_B; }
