@@ -1405,18 +1405,19 @@ static int jk_from_store(aimdhf_plan* p, int nset, const double* dens, double* J
             for (int k = 0; k < NQCLASS; ++k) p->last_dig[k] = p->digest_args(k, nset, delta, dthr);
             p->prof.time(94, st, [&] { aimdhf::launch_digest_all(da, threads, st); });
         } else {
-            // spread over the fan's streams; a batch's launches stay on the caller's stream, which
-            // may be capturing (its graph outlives calls and must not depend on the plan's
-            // streams), and cover every class, as the graph is replayed at other geometries
-            if (!p->batched) p->fan.fork(st);
+            // spread over the fan's streams; a batch's launches and those that a graph records stay
+            // on the caller's stream (the graph outlives calls and must not depend on the plan's
+            // streams), and a batch's cover every class, as its graph is replayed at other geometries
+            const bool one = p->batched || Fan::capturing(st);
+            if (!one) p->fan.fork(st);
             int i = 0;
             for (int k = NQCLASS - 1; k >= 0; --k) {
                 if (!p->qcount[k] && !p->batched) continue;
                 p->last_dig[k] = p->digest_args(k, nset, delta, dthr);
-                hipStream_t s2 = p->batched ? st : p->fan.on(i++);
+                hipStream_t s2 = one ? st : p->fan.on(i++);
                 p->prof.time(98 + k, s2, [&] { aimdhf::launch_digest(k, p->last_dig[k], threads, s2); });
             }
-            if (!p->batched) p->fan.join();
+            if (!one) p->fan.join();
         }
         p->have_last_store = true;
         p->prof.time(93, st, [&] { aimdhf::launch_jk_finish(pa, st); });
@@ -1443,15 +1444,16 @@ static int jk_direct(aimdhf_plan* p, int nset, const double* dens, double* J, do
         p->ensure_digest(nset);
         const aimdhf::PrepArgs pa = p->prep_args(nset, dens, J, K);
         p->prof.time(45, st, [&] { aimdhf::launch_jk_prep(pa, st); });
+        const bool one = Fan::capturing(st);    // a graph records the caller's stream alone
         for (size_t c = 0; c < p->pieces.size(); ++c) {
             const aimdhf_plan::Piece& pc = p->pieces[c];
             // a class is digested on the stream that evaluates it; the pieces share the buffer
-            p->fan.fork(st);
+            if (!one) p->fan.fork(st);
             int i = 0;
             for (int k = NQCLASS - 1; k >= 0; --k) {
                 if (pc.hi[k] <= pc.lo[k]) continue;
                 const long long n = pc.hi[k] - pc.base[k];
-                hipStream_t s2 = p->fan.on(i++);
+                hipStream_t s2 = one ? st : p->fan.on(i++);
                 aimdhf::EriArgs ea = p->eri_args(k, pc.base[k]);
                 ea.out64 = (double*)(p->d_store.as<char>() + pc.at[k]);
                 const long long h = p->list_off[k] + p->h64count[k] - pc.base[k];
@@ -1460,7 +1462,7 @@ static int jk_direct(aimdhf_plan* p, int nset, const double* dens, double* J, do
                 da.geo += c * NQCLASS;
                 p->prof.time(98 + k, s2, [&] { aimdhf::launch_digest(k, da, 256, s2); });
             }
-            p->fan.join();
+            if (!one) p->fan.join();
         }
         p->prof.time(93, st, [&] { aimdhf::launch_jk_finish(pa, st); });
         HIPCHECK(hipGetLastError());

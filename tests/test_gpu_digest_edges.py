@@ -1,7 +1,7 @@
 """
 The single-read J/K digestion at the edges of its routes: bases of one angular
 momentum, integral lists past the size of one launch, direct mode's pieces,
-matrices of more than 16384 orbitals.
+matrices of more than 16384 orbitals, builds that a graph records.
 """
 
 import numpy as np
@@ -178,3 +178,36 @@ def test_more_than_16384_orbitals(mode):
         assert float(got[:, :-m].abs().max()) == 0.0
     e.close()
     small.close()
+
+
+@pytest.mark.parametrize("nset", [1, 2])
+@pytest.mark.parametrize("mode", ["direct", "store"])
+def test_builds_recorded_in_a_graph(mode, nset):
+    """A captured build replayed with other densities, with eager builds and waits between the
+    replays, equals the eager one bit for bit (two densities of 152 orbitals take the
+    launches per class, one the launch of all classes)."""
+    import torch
+    from aimd_amd.qc.basis import build_basis
+    from aimd_amd.qc.engine import Engine
+    s, x = cluster("water8.xyz")
+    e = Engine(build_basis(s, x, "6-31g*"))
+    e.set_jk_mode(mode, 1 if mode == "direct" else 0)
+    e.set_geometry(x)
+    D = _dens(e.nao, nset)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        e.jk(D)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = e.jk(D)
+    for seed in range(1, 5):
+        D.copy_(_dens(e.nao, nset, seed))
+        ref = e.jk(D)
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(out, ref):
+            assert torch.equal(a, b), seed
+    del graph
+    e.close()
