@@ -1045,9 +1045,10 @@ class SCFSolver:
         J, K = I.engine.jk(Ds) if jk is None else jk
         F, err, Fo = (torch.empty_like(Ds) for _ in range(3))
         em = torch.empty(2, dtype=torch.float64, device=Ds.device)
-        _lib.check(_lib.lib().aimdhf_small_fock(
-            1, Ds.shape[0], Ds.shape[1], _ptr(I.H), _ptr(I.S), _ptr(X), _ptr(Ds), _ptr(J), _ptr(K), _ptr(F),
-            _ptr(Fo), _ptr(err), 0, 0, None, _ptr(em), ctypes.c_void_p(em.data_ptr() + 8), _stream()))
+        with torch.cuda.device(Ds.device):
+            _lib.check(_lib.lib().aimdhf_small_fock(
+                1, Ds.shape[0], Ds.shape[1], _ptr(I.H), _ptr(I.S), _ptr(X), _ptr(Ds), _ptr(J), _ptr(K), _ptr(F),
+                _ptr(Fo), _ptr(err), 0, 0, None, _ptr(em), ctypes.c_void_p(em.data_ptr() + 8), _stream()))
         return F, err, Fo, em
 
     def _next_density_small(self, Fo: torch.Tensor, X: torch.Tensor, nocc: torch.Tensor, Ds: torch.Tensor,
@@ -1058,9 +1059,10 @@ class SCFSolver:
         P, Dn = torch.empty_like(Ds), torch.empty_like(Ds)
         perr = torch.empty(nspin, dtype=torch.float64, device=Ds.device)
         L = _lib.lib()
-        _lib.check(L.aimdhf_batch_purify(nspin, n, _ptr(Fo), _ptr(nocc), _ptr(P), steps, tol, _ptr(perr), _stream()))
-        _lib.check(L.aimdhf_small_density(1, nspin, n, _ptr(X), _ptr(P), _ptr(Dn), None, None, None, None, 0.0, 0.0,
-                                          None, None, 0, _stream()))
+        with torch.cuda.device(Ds.device):
+            _lib.check(L.aimdhf_batch_purify(nspin, n, _ptr(Fo), _ptr(nocc), _ptr(P), steps, tol, _ptr(perr), _stream()))
+            _lib.check(L.aimdhf_small_density(1, nspin, n, _ptr(X), _ptr(P), _ptr(Dn), None, None, None, None, 0.0,
+                                              0.0, None, None, 0, _stream()))
         return Dn if all(e < tol for e in perr.tolist()) else None
 
     def _fock(self, I: SCFIntegrals, Ds: torch.Tensor, jk: tuple | None = None) -> torch.Tensor:

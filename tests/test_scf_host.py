@@ -157,3 +157,34 @@ def test_incremental_fock_defaults_follow_the_precision():
     assert Solver(precision="mixed").incremental
     assert Solver(incremental_fock=True).incremental
     assert not Solver(precision="mixed", incremental_fock=False).incremental
+
+
+def test_small_scf_algebra_launches_on_the_device_of_its_tensors(monkeypatch):
+    # the stream and every launch are taken inside a guard for the tensors' device, whatever the current one
+    from types import SimpleNamespace
+    active, seen = [], []
+
+    class Guard:
+        def __init__(self, device):
+            self.device = device
+
+        def __enter__(self):
+            active.append(self.device)
+
+        def __exit__(self, *_):
+            active.pop()
+
+    class Recorder:
+        def __getattr__(self, name):
+            return lambda *args: seen.append((name, list(active))) or 0
+
+    monkeypatch.setattr(torch.cuda, "device", Guard)
+    monkeypatch.setattr(S._lib, "lib", Recorder)
+    monkeypatch.setattr(S, "_stream", lambda: seen.append(("stream", list(active))))
+    solver = object.__new__(S.SCFSolver)
+    Ds = torch.zeros((2, 4, 4), dtype=torch.float64)
+    I = SimpleNamespace(H=Ds[0], S=Ds[0])
+    solver._fock_small(I, Ds[0], Ds, (Ds, Ds))
+    solver._next_density_small(Ds, Ds[0], torch.ones(2, dtype=torch.float64), Ds)
+    assert [n for n, _ in seen if n != "stream"] == ["aimdhf_small_fock", "aimdhf_batch_purify", "aimdhf_small_density"]
+    assert all(a == [Ds.device] for _, a in seen) and len(seen) == 6
