@@ -63,6 +63,13 @@ constexpr int NT_MAX = NT<double> > NT<float> ? NT<double> : NT<float>;
 constexpr int GRAD_LDS_WORDS = 3600;
 // most parts a bra's (or, in a ket pass, a ket's) primitive pairs are cut into
 constexpr int MAXPART = pc_lo() == 0 || pc_hi() <= 1 ? (pc_hi() == 0 ? 16 : pc_hi() == 1 ? 8 : 4) : pc_hi() <= 3 ? 4 : 2;
+// and the items, parts counted, up to which they are: sixteen wavefronts a CU for bras with
+// many primitive pairs, where a shorter chain pays over several rounds ((ss|ss) of four waters
+// 0.92 -> 0.24 ms); bras of a d shell have one to three, and cut items past a round of one
+// wavefront a SIMD only come twice ((dd|dd) of (H2O)11 0.10 -> 0.18 ms, (dp|ps) of five waters
+// 0.15 -> 0.19). Candidates are counted, about a third of which the screening drops; (dd|pp)
+// cut spills so much more that it gains below 5000 items only
+constexpr long long CUT_ITEMS = pc_hi() <= 3 || QC == 10 ? 262144 : pc_hi() == 4 ? 131072 : QC == 17 ? 16384 : 98304;
 
 __device__ __forceinline__ void lds_add(long long* lds, int atom, int d, double x) {
     long long h, l;
@@ -210,9 +217,9 @@ __global__ __launch_bounds__(256) void k_grad_scatter(const unsigned char* __res
     if (k == 2) sel32[o2 + __popcll(m2 & below)] = (int)q;
 }
 
-// part `part` of np primitive pairs; false if it is empty
-__device__ __forceinline__ bool prim_part(int np, int part, int nparts, int& b0, int& nb) {
-    const int ch = (np + nparts - 1) / nparts;
+// part `part` of 2^lparts of np primitive pairs; false if it is empty
+__device__ __forceinline__ bool prim_part(int np, int part, int lparts, int& b0, int& nb) {
+    const int ch = (np + (1 << lparts) - 1) >> lparts;
     b0 = part * ch;
     nb = b0 + ch < np ? ch : np - b0;
     return nb > 0;
@@ -221,10 +228,10 @@ __device__ __forceinline__ bool prim_part(int np, int part, int nparts, int& b0,
 // The folded item for ket columns KC0 .. KC0+FOLD<Real>-1 of quartet pq: A, B and C
 // derivatives from one pass, D by translational invariance
 template <int KC0, typename Real>
-__device__ __forceinline__ void fold_item(const GradArgs& a, int2 pq, int part, int nparts, const double* btab,
+__device__ __forceinline__ void fold_item(const GradArgs& a, int2 pq, int part, int lparts, const double* btab,
                                           long long* lds) {
     int b0, nb;
-    if (!prim_part(a.npp[pq.x], part, nparts, b0, nb)) return;
+    if (!prim_part(a.npp[pq.x], part, lparts, b0, nb)) return;
     const int sA = a.pair_a[pq.x], sB = a.pair_b[pq.x], sC = a.pair_a[pq.y], sD = a.pair_b[pq.y];
     const int aA = a.shell_atom[sA], aB = a.shell_atom[sB], aC = a.shell_atom[sC], aD = a.shell_atom[sD];
     double deg = 0.5;
@@ -253,9 +260,9 @@ __device__ __forceinline__ void fold_item(const GradArgs& a, int2 pq, int part, 
 }
 
 // Work item = (selected quartet, pass column group), derivative integrals in Real
-template <int Q, typename Real>
+template <int Q, typename Real, bool PARTS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(grad_waves<Real>()))) void k_grad_class(
-    GradArgs a, const int2* __restrict__ list, const int* __restrict__ sel, const int* __restrict__ nsel, int nparts) {
+    GradArgs a, const int2* __restrict__ list, const int* __restrict__ sel, const int* __restrict__ nsel, int lparts) {
     extern __shared__ long long lds_acc[];
     __shared__ double btab[BOYS_NGRID * BOYS_SROW];
     // per-atom sums staged in LDS when they fit next to the Boys slice, else added
@@ -268,19 +275,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(grad_waves<
     // items wave by wave: the 64 lanes of a wave take 64 consecutive selected
     // quartets and one pass / column group, so the pass dispatch is uniform
     constexpr int NTR = NT<Real>;
-    const int ntp = NTR * nparts;
-    const long long ns = *nsel, nitems = (ns + 63) / 64 * 64 * ntp;
+    if constexpr (!PARTS) lparts = 0;
+    const long long ns = *nsel, nitems = ((ns + 63) / 64 * 64 * NTR) << lparts;
     for (long long it = (long long)blockIdx.x * blockDim.x + threadIdx.x; it < nitems;
          it += (long long)gridDim.x * blockDim.x) {
-        const long long g = it >> 6;
-        const int jp = (int)(g % ntp), j = jp / nparts, part = jp - j * nparts;
-        const long long qi = g / ntp * 64 + (it & 63);
+        const long long g = it >> (6 + lparts);
+        const int part = (int)(it >> 6) & ((1 << lparts) - 1), j = (int)(g % NTR);
+        const long long qi = g / NTR * 64 + (it & 63);
         if (qi >= ns) continue;
         const int2 pq = list[sel[qi]];
         if constexpr (FOLD<Real> > 0) {
             static_for<0, NTR>([&](auto jj) {
                 constexpr int J = decltype(jj)::value;
-                if (j == J) fold_item<J * FOLD<Real>, Real>(a, pq, part, nparts, btab, lds);
+                if (j == J) fold_item<J * FOLD<Real>, Real>(a, pq, part, lparts, btab, lds);
             });
             continue;
         }
@@ -299,7 +306,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(grad_waves<
         const double* rb = a.recs + a.rec_off[pq.x];
         const double* rk = a.recs + a.rec_off[pq.y];
         int b0, nb;
-        if (!prim_part(a.npp[bra ? pq.x : pq.y], part, nparts, b0, nb)) continue;
+        if (!prim_part(a.npp[bra ? pq.x : pq.y], part, lparts, b0, nb)) continue;
         double g1[3], g2[3];
         if (bra) {
             const int kc0 = j * NCB;
@@ -355,6 +362,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(grad_waves<
 #define CAT2(a, b) a##b
 #define CAT(a, b) CAT2(a, b)
 
+// the class's FP64 items uncut, where that needs a kernel of its own (compiled apart with
+// -DAIMDHF_GRAD_WHOLE). With the bounds of a part the register allocator spills more in
+// these classes: (H2O)16/6-31G* (dp|ps) 0.650 -> 0.668 ms, (dd|pp) 0.404 -> 0.492, (dd|dd)
+// 0.212 -> 0.286; the others stay within 1% (all with the item index taken apart by
+// shifts; a division by the number of items and parts cost the light classes 1%)
+constexpr bool WHOLE = QC == 11 || QC == 17 || QC == 20;
+void CAT(launch_grad_whole_, AIMDHF_QCLASS)(const GradArgs& a, const int2* list, int blocks, size_t shm, hipStream_t st);
+
+#ifdef AIMDHF_GRAD_WHOLE
+void CAT(launch_grad_whole_, AIMDHF_QCLASS)(const GradArgs& a, const int2* list, int blocks, size_t shm, hipStream_t st) {
+    k_grad_class<QC, double, false><<<dim3(blocks), dim3(256), shm, st>>>(a, list, a.sel64, a.nsel, 0);
+}
+#else
+
 // pre-pass + scan + ordered scatter (a.bcnt / a.boff hold 2 ints per 256 quartets)
 void CAT(launch_grad_keep_, AIMDHF_QCLASS)(const GradArgs& a, const int2* list, long long nq, hipStream_t st) {
     if (nq <= 0) return;
@@ -369,19 +390,25 @@ void CAT(launch_grad_keep_, AIMDHF_QCLASS)(const GradArgs& a, const int2* list, 
 void CAT(launch_grad_class_, AIMDHF_QCLASS)(const GradArgs& a, const int2* list, long long nq, hipStream_t st) {
     // primitive parts per item: a lane's loop over a contracted quartet (36 x 36 for
     // (ss|ss) in 6-31G*, 64 x 64 in cc-pVDZ) is what a small system waits for; with too few
-    // items to fill the card it is cut into parts (their sums are exact integers). Up to
-    // 16 parts, while the items stay below 16 wavefronts a CU
+    // items to fill the card it is cut into parts (their sums are exact integers)
     long long items = nq * NT_MAX;
     if (items <= 0) return;
-    int nparts = 1;
-    while (nparts < MAXPART && items * nparts * 2 <= 262144) nparts *= 2;
-    items *= nparts;
+    int lparts = 0;
+    while ((1 << lparts) < MAXPART && items << (lparts + 1) <= CUT_ITEMS) ++lparts;
+    items <<= lparts;
     long long blocks = (items + 255) / 256;
     if (blocks > 1024) blocks = 1024;
     const size_t shm = 6 * a.natm <= GRAD_LDS_WORDS ? sizeof(long long) * 6 * a.natm : 0;
-    k_grad_class<QC, double><<<dim3((unsigned)blocks), dim3(256), shm, st>>>(a, list, a.sel64, a.nsel, nparts);
+    bool whole = false;
+    if constexpr (WHOLE) {
+        whole = lparts == 0;
+        if (whole) CAT(launch_grad_whole_, AIMDHF_QCLASS)(a, list, (int)blocks, shm, st);
+    }
+    if (!whole)
+        k_grad_class<QC, double, true><<<dim3((unsigned)blocks), dim3(256), shm, st>>>(a, list, a.sel64, a.nsel, lparts);
     if (a.fp32_switch > 0.0)
-        k_grad_class<QC, float><<<dim3((unsigned)blocks), dim3(256), shm, st>>>(a, list, a.sel32, a.nsel + 1, nparts);
+        k_grad_class<QC, float, true><<<dim3((unsigned)blocks), dim3(256), shm, st>>>(a, list, a.sel32, a.nsel + 1, lparts);
 }
+#endif
 
 }  // namespace aimdhf
