@@ -7,10 +7,10 @@ Per geometry of the whole batch:
 * one set-up (pairs, Schwarz bounds, screened quartets of every replica) and
   one integral-evaluation launch per quartet class for all replicas;
 * an SCF whose iteration is one captured HIP graph for all replicas: J/K of
-  every replica in one or two launches, Fock matrices, energies and commutators as
-  batched products, Pulay DIIS with its small systems solved on the device
-  (one launch), and the aufbau densities of every replica and spin by
-  purification in one launch; one host read per iteration checks convergence;
+  every replica in one or two launches, then one launch each for the Fock
+  matrices, energies and commutators, the Pulay step, the aufbau projectors of
+  every replica and spin by purification, and the densities with the
+  convergence test; one host read per iteration checks convergence;
 * forces of every replica from one one-electron-gradient launch and one
   derivative-ERI launch per class.
 

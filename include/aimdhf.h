@@ -127,9 +127,11 @@ int aimdhf_quartets(aimdhf_plan* plan, int64_t* out_host, int64_t cap, int64_t* 
  * piece. The buffer takes at most 1 GiB, an eighth of the free memory beyond what
  * it holds already, and max_store_bytes if that is set (64 MiB at least), or the
  * run of kets of one bra where that is longer; J and K do not depend on its size.
- * Sums are 64-bit fixed point whose exponent follows the
- * density and the Schwarz bounds (resolution 2^-62 of a bound of the largest element; a density with a NaN or
- * infinity gives NaN in its J and K).
+ * Sums are 64-bit fixed point whose exponent follows the density and the Schwarz
+ * bounds: each J and each K has one absolute resolution, 2^-61 of a bound of its
+ * largest element, so an element 1e-6 of that keeps 12 digits, and one dominant
+ * element of the density costs all the others theirs. A density with a NaN or an
+ * infinity gives NaN in its J and K.
  * Replaces: jk_from_eri (aimd/qc/integrals.py:1009-1044) and, in direct mode,
  * eri_tensor (aimd/qc/integrals.py:986-1006).
  */
@@ -206,8 +208,9 @@ int aimdhf_batch_purify(int nmat, int ld, const double* F, const double* nocc, d
 /*
  * Lanes (16, 32 or 64; default 64): a workgroup of a batched plan's J/K has four
  * threads per lane, for batches of small replicas whose runs of kets would
- * leave larger workgroups idle. Results do not depend on it. A tuning knob with no counterpart in the
- * reference; aimd_amd.batch.ReplicaBatch.autotune times the choices.
+ * leave larger workgroups idle. J depends on it in its last bits (a lane adds its
+ * share of a bra's J in FP64). A tuning knob with no counterpart in the reference;
+ * aimd_amd.batch.ReplicaBatch.autotune times the choices.
  */
 int aimdhf_batch_set_jk_lanes(aimdhf_plan* plan, int lanes);
 
@@ -283,7 +286,7 @@ int aimdhf_set_streams(aimdhf_plan* plan, int concurrent);
 /*
  * Least quartets (64 .. 65536, default 1024) a workgroup of the store-mode J/K
  * digestion takes from a long run of kets. A tuning knob with no counterpart in
- * the reference; results do not depend on it.
+ * the reference; J depends on it in its last bits.
  */
 int aimdhf_set_store_units(aimdhf_plan* plan, int items);
 
