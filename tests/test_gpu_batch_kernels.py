@@ -1,8 +1,8 @@
 """
 The batched-replica kernels on their own: the purification (X^2 on the FP64
 matrix cores) against the exact aufbau projector of random gapped Fock
-matrices, and the batched J/K digestion at every lanes-per-element choice
-against the single-molecule engine's J/K of each replica.
+matrices, the Pulay solve against numpy, and the batched J/K digestion at every
+workgroup size against the single-molecule engine's J/K of each replica.
 """
 
 import ctypes
@@ -51,6 +51,33 @@ def test_batched_purification_is_the_aufbau_projector(ld):
     print(f"ld {ld}: max |P - projector| {dev_max:.2e}, idempotency errors {err.cpu().numpy().max():.1e}", flush=True)
     assert dev_max < 1e-10
     np.testing.assert_allclose(np.trace(Pg, axis1=1, axis2=2), nocc, rtol=0, atol=1e-10)
+
+
+@pytest.mark.parametrize("m", [1, 2, 7, 12])
+def test_batched_pulay_solve(m):
+    """Random symmetric systems, one with an unused slot (an identity row with r = 0) and one
+    with a null direction, whose unknown is 0; elimination loses about m eps cond."""
+    import torch
+    from aimd_amd import _lib
+    rng = np.random.default_rng(m)
+    n = 5
+    A = rng.standard_normal((n, m, m + 3))
+    G = A @ A.transpose(0, 2, 1)
+    r = rng.standard_normal((n, m))
+    if m > 1:
+        G[1, -1, :] = G[1, :, -1] = 0.0
+        G[1, -1, -1], r[1, -1] = 1.0, 0.0
+        G[2, -1, :] = G[2, :, -1] = 0.0
+        r[2, -1] = 0.0
+    ref = np.stack([np.linalg.lstsq(G[i], r[i], rcond=None)[0] for i in range(n)])
+    Gt, rt = torch.tensor(G, device="cuda"), torch.tensor(r, device="cuda")
+    c = torch.empty_like(rt)
+    _lib.check(_lib.lib().aimdhf_batch_diis_solve(n, m, _ptr(Gt), _ptr(rt), _ptr(c), _stream()))
+    for i in range(n):
+        w = np.linalg.svd(G[i], compute_uv=False)
+        cond = w[0] / w[w > 1e-13 * w[0]].min()
+        tol = 100 * m * np.finfo(float).eps * cond * max(1.0, np.abs(ref[i]).max())
+        assert np.abs(c[i].cpu().numpy() - ref[i]).max() < tol
 
 
 def test_batched_jk_at_every_lane_choice_matches_the_single_molecule_engine():

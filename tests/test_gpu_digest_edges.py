@@ -1,13 +1,14 @@
 """
 The single-read J/K digestion at the edges of its routes: bases of one angular
 momentum, integral lists past the size of one launch, direct mode's pieces,
-matrices of more than 16384 orbitals, builds that a graph records.
+matrices of more than 16384 orbitals, builds that a graph records, what difference
+builds leave out, densities with one dominant element.
 """
 
 import numpy as np
 import pytest
 
-from tests.conftest import cluster
+from tests.conftest import cluster, water_dimer
 
 pytestmark = pytest.mark.gpu
 
@@ -210,4 +211,79 @@ def test_builds_recorded_in_a_graph(mode, nset):
         for a, b in zip(out, ref):
             assert torch.equal(a, b), seed
     del graph
+    e.close()
+
+
+@pytest.mark.parametrize("name,nset", [("dimer", 1), ("water8", 2)])
+def test_difference_build_skips_only_what_is_below_the_threshold(name, nset):
+    """What a screened build leaves out, element by element, is at most the sum of |integral
+    bounds| |dD| over the products below the threshold (Schwarz bounds and densities as given,
+    not a count times the threshold); something is left out, and everything is when the threshold
+    is above every product. The bounds tell a threshold that is off by a thousand. One launch
+    for all classes (dimer) and launches per class."""
+    import torch
+    from aimd_amd.qc.basis import build_basis
+    from aimd_amd.qc.engine import Engine
+    s, x = water_dimer() if name == "dimer" else cluster("water8.xyz")
+    b = build_basis(s, x, "6-31g*")
+    assert b.nblock == b.nshell
+    e = Engine(b)
+    e.set_jk_mode("store")
+    e.set_geometry(x)
+    D = 1e-3 * _dens(e.nao, nset, 11)
+    i = torch.arange(b.nshell)
+    pair = torch.where(i[:, None] >= i[None], i[:, None] * (i[:, None] + 1) // 2 + i[None],
+                       i[None] * (i[None] + 1) // 2 + i[:, None])
+    ao = torch.as_tensor(b.ao_shell.copy())
+    Q = torch.as_tensor(e.schwarz_bounds())[pair][ao][:, ao].cuda()
+    full = e.jk_delta(D, 0.0)
+    thr = 1e-8
+    part = e.jk_delta(D, thr)
+    off = e.jk_delta(D, 1e3 * thr)
+    for s_ in range(nset):
+        a = D[s_].abs()
+        bound_j, bound_k = torch.empty_like(a), torch.empty_like(a)
+        for m in range(e.nao):
+            T = Q[m][:, None, None] * Q[None]               # (second index of the bra, k, l)
+            T = torch.where(T * a.max() < thr, T, torch.zeros_like(T))
+            bound_j[m] = (T * a[None]).sum(dim=(1, 2))
+            # (m k|n l) D_kl: T indexed (k, n, l)
+            bound_k[m] = (T * a[:, None, :]).sum(dim=(0, 2))
+        for f, p, o, bound in ((full[0][s_], part[0][s_], off[0][s_], bound_j),
+                               (full[1][s_], part[1][s_], off[1][s_], bound_k)):
+            left = (f - p).abs()
+            print(name, nset, s_, "left out", float(left.max()), "bound", float(bound.max()), flush=True)
+            assert float(left.max()) > 0.0
+            slack = 1e-14 * float(f.abs().max())
+            assert bool((left <= bound + slack).all())
+            assert bool(((f - o).abs() > bound + slack).any())
+    for z in e.jk_delta(D, 1.001 * float(Q.max()) ** 2 * float(D.abs().max())):
+        assert float(z.abs().max()) == 0.0
+    e.close()
+
+
+def test_one_dominant_density_element(oracle_lib):
+    """The fixed-point words of a build have one resolution for every element, 2^-61 of a bound of
+    the largest: with one density element of 1e10 the others keep an absolute error of that size
+    (and of the FP64 lane sums, 2^-53 of the same bound), not a relative one."""
+    from aimd_amd.qc.basis import build_basis
+    from aimd_amd.qc.engine import Engine
+    s, x = water_dimer()
+    b = build_basis(s, x, "6-31g*")
+    e = Engine(b)
+    e.set_jk_mode("store")
+    e.set_geometry(x)
+    D = _dens(e.nao, 1, 13)
+    D[0, 2, 2] = 1e10
+    J, K = e.jk(D)
+    Dh = D.cpu().numpy()
+    Jo, Ko = oracle_lib.Pairs(oracle_lib.make_basis(s, x, "6-31g*")).jk_direct(Dh)
+    q = e.schwarz_bounds()
+    i = np.arange(b.nshell)
+    hi, lo = np.maximum(i[:, None], i), np.minimum(i[:, None], i)
+    Q = q[hi * (hi + 1) // 2 + lo][np.ix_(b.ao_shell, b.ao_shell)]
+    a = np.abs(Dh[0])
+    bound_j, bound_k = Q.max() * (Q * a).sum(), (Q ** 2).sum(axis=1).max() * a.sum(axis=1).max()
+    assert np.abs(J.cpu().numpy() - Jo).max() < b.nao * 2.0 ** -53 * bound_j
+    assert np.abs(K.cpu().numpy() - Ko).max() < b.nao * 2.0 ** -53 * bound_k
     e.close()

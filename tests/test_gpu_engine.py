@@ -107,8 +107,8 @@ def test_one_electron_and_gradient_terms(oracle_lib, mol, basis, mult):
 @pytest.mark.parametrize("mode,precision", [("store", "fp64"), ("store", "mixed"), ("direct", "fp64")])
 def test_density_difference_builds(oracle_lib, mode, precision):
     """J/K of a density difference (incremental Fock): linear against the oracle
-    with nothing screened, exactly zero when every unit is screened out, and
-    FP32 digestion in mixed precision within FP32 rounding of the FP64 result."""
+    with nothing screened, exactly zero when every quartet is screened out, and in mixed
+    precision (integrals below the switch held in FP32) within FP32 rounding of it."""
     import torch
     from aimd_amd.qc.basis import build_basis
     from aimd_amd.qc.engine import Engine
@@ -126,7 +126,7 @@ def test_density_difference_builds(oracle_lib, mode, precision):
     dt = torch.tensor(dD, device="cuda")
     dJ, dK = e.jk_delta(dt, 0.0)
     Jo, Ko = oracle_lib.Pairs(oracle_lib.make_basis(s, x, "6-31g*")).jk_direct(dD)
-    # FP64: the oracle's 1e-11 at unit density, scaled; FP32 digestion: ~1e-7 relative per term
+    # FP64: the oracle's 1e-11 at unit density, scaled; FP32 integrals: ~1e-7 relative per term
     tol = (2e-5 if precision == "mixed" else 1e-10) * scale
     np.testing.assert_allclose(dJ.cpu().numpy(), Jo, rtol=0, atol=tol)
     np.testing.assert_allclose(dK.cpu().numpy(), Ko, rtol=0, atol=tol)
