@@ -237,7 +237,6 @@ struct aimdhf_plan {
     double threshold = 0.0;
     std::vector<long long> qcount;   // per class
     std::vector<long long> q64count; // per class, quartets with q_P q_Q >= the FP32 switch (listed first)
-    std::vector<long long> g64count;
     long long qtotal = 0;
 
     DevBuf d_shell_atom, d_shell_l, d_shell_prim, d_shell_ao, d_prim_exp, d_prim_coef, d_pos;
@@ -270,7 +269,6 @@ struct aimdhf_plan {
     DevBuf d_store;
     // least quartets a workgroup of the J/K digestion takes from a long run
     int unit_items = 1024;
-    double delta_fp32_max = 1e-3;   // accepted; every difference build sums in FP64
     DevBuf d_gdmax;                 // per shell pair density maxima for the gradient screening
     long long* h_pin = nullptr;     // pinned host words for the totals and the error flag
     // batched plans: independent molecules (replicas) sharing one plan; shells and
@@ -280,7 +278,7 @@ struct aimdhf_plan {
     int nrep = 1, bld = 0;
     int batch_jk_lanes = 64;        // batched J/K digestion: four threads per lane of this and workgroup
     std::vector<int> rep_shell, rep_atom, rep_nao, shell_rep, shell_first, shell_pair0, pair_lo;
-    long long tens_total = 0;       // elements of one dense n_r^4 tensor per replica (aimdhf_batch_layout)
+    long long tens_total = 0;       // elements of one dense n_r^4 tensor per replica, none of which exists (aimdhf_batch_layout)
     DevBuf d_shell_rep, d_shell_first, d_shell_pair0, d_pair_lo, d_rep_atom, d_rep_nao;
     // elements of one stack of matrices (nao^2, or nrep ld^2 for a batch)
     size_t mat_elems() const { return batched ? (size_t)nrep * bld * bld : (size_t)nao * nao; }
@@ -389,35 +387,28 @@ struct aimdhf_plan {
         return g;
     }
 
-    // Class-binned list of unique shell quartets with q_P q_Q >= thr into buf;
+    // List of unique shell quartets with q_P q_Q >= thr into buf, binned by class and cost;
     // counts[k] receives the per-class sizes. Synchronises the stream.
-    // Screened quartet list binned by class, precision part (q_P q_Q >= sw
-    // first) and cost; counts per class, n64 per class the part >= sw.
-    void build_list(double thr, double sw, DevBuf& buf, std::vector<long long>& counts, std::vector<long long>& n64,
-                    hipStream_t st) {
+    void build_list(double thr, DevBuf& buf, std::vector<long long>& counts, hipStream_t st) {
         aimdhf::PairArgs g = pair_args();
-        const int nb = aimdhf::list_bins(sw), nv = NQCLASS * nb;
+        const int nb = aimdhf::NCOSTBIN, nv = NQCLASS * nb;
         d_counts.ensure(sizeof(int) * (size_t)npair * nv);
         d_offsets.ensure(sizeof(long long) * ((size_t)npair * nv + 2 * nv));
         long long* offs = d_offsets.as<long long>();
         long long* totals = offs + (size_t)npair * nv;
         long long* base = totals + nv;
-        aimdhf::launch_count_quartets(g, thr, sw, d_counts.as<int>(), offs, totals, base, st);
+        aimdhf::launch_count_quartets(g, thr, d_counts.as<int>(), offs, totals, base, st);
         HIPCHECK(hipGetLastError());
         std::vector<long long> tot(nv);
         HIPCHECK(hipMemcpyAsync(tot.data(), totals, sizeof(long long) * nv, hipMemcpyDeviceToHost, st));
         HIPCHECK(hipStreamSynchronize(st));
         counts.assign(NQCLASS, 0);
-        n64.assign(NQCLASS, 0);
         long long total = 0;
         for (int k = 0; k < NQCLASS; ++k)
-            for (int b = 0; b < nb; ++b) {
-                counts[k] += tot[k * nb + b];
-                if (b < aimdhf::NCOSTBIN) n64[k] += tot[k * nb + b];
-            }
+            for (int b = 0; b < nb; ++b) counts[k] += tot[k * nb + b];
         for (long long c : counts) total += c;
         buf.ensure(sizeof(int2) * std::max<long long>(total, 1));
-        aimdhf::launch_fill_quartets(g, thr, sw, offs, base, buf.as<int2>(), st);
+        aimdhf::launch_fill_quartets(g, thr, offs, base, buf.as<int2>(), st);
         HIPCHECK(hipGetLastError());
     }
 
@@ -1646,7 +1637,7 @@ int aimdhf_grad_two(aimdhf_plan* p, const double* Dc, int nx, const double* Dx, 
         double gbound = 4.0 * (mc * mc + std::fabs(kfac) * nx * mx * mx);
         double lthr = gbound > 0.0 ? thr / gbound : 0.0;
         auto t0 = Profiler::clock::now();
-        p->build_list(lthr, 0.0, p->d_glist, p->gcount, p->g64count, st);
+        p->build_list(lthr, p->d_glist, p->gcount, st);
         p->prof.host(88, t0);
         p->d_gfx.ensure(sizeof(long long) * 6 * p->natm);
         aimdhf::launch_zero64(p->d_gfx.as<long long>(), 6 * p->natm, st);
@@ -1858,7 +1849,6 @@ int aimdhf_set_precision(aimdhf_plan* p, int mode, double jk_switch, double grad
     p->precision = mode;
     p->jk_switch = jk_switch;
     p->grad_switch = grad_switch;
-    p->delta_fp32_max = delta_switch;
     return AIMDHF_OK;
 }
 

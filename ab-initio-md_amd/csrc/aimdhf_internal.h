@@ -111,15 +111,11 @@ void launch_zero_d(double* p, size_t n, hipStream_t st);
 
 void launch_build_pairs(const PairArgs& g, hipStream_t st);
 void launch_schwarz(const PairArgs& g, const int* ncls_host, hipStream_t st);
-// quartet lists: per class, NCOSTBIN bins of primitive-quartet cost (heaviest first)
+// gradient quartet lists: per class, NCOSTBIN bins of primitive-quartet cost (heaviest first)
 constexpr int NCOSTBIN = 5;
-// list bins of a class: the quartets with q_P q_Q >= sw (FP64) in cost bins,
-// then those below sw (FP32 in mixed precision) in cost bins
-constexpr int NLBIN = 2 * NCOSTBIN;
-void launch_count_quartets(const PairArgs& g, double thr, double sw, int* counts, long long* offs, long long* totals,
+void launch_count_quartets(const PairArgs& g, double thr, int* counts, long long* offs, long long* totals,
                            long long* base, hipStream_t st);
-int list_bins(double sw);
-void launch_fill_quartets(const PairArgs& g, double thr, double sw, const long long* offs, const long long* base, int2* list,
+void launch_fill_quartets(const PairArgs& g, double thr, const long long* offs, const long long* base, int2* list,
                           hipStream_t st);
 // ---------------------------------------------------------------- runtime-l path (l <= GEN_LMAX)
 constexpr int GEN_LMAX = 4;
@@ -169,7 +165,6 @@ void* noalloc_scratch(size_t* bytes);
 void launch_grad_one(const OneElArgs& g, const double* D, const double* Wneg, long long* out, const hipStream_t* on);
 void launch_negate(const double* W, size_t n, double* out, hipStream_t st);
 void launch_fx_to_double(const long long* fx, int n, double* out, hipStream_t st);
-void launch_grad(const GradArgs& a, const int2* const* lists, const long long* counts, hipStream_t st);
 double device_absmax(const double* x, size_t n, double* scratch, hipStream_t st);
 void launch_jk_finalize(const long long* fx, int nset, int n, double* J, double* K, hipStream_t st);
 

@@ -110,25 +110,18 @@ __device__ __forceinline__ int qclass(int cp, int cq) {
     return hi * (hi + 1) / 2 + lo;
 }
 
-// Within a class, quartets are further binned by precision (q_P q_Q >= sw
-// first: FP64; then below sw: FP32 in mixed precision) and cost npp_P * npp_Q
-// (kept primitive pairs), heaviest bin first, so the lanes of a wavefront run
-// loops of similar length; within a bin the order is P-major, Q ascending.
+// Within a class, quartets are further binned by cost npp_P * npp_Q (kept
+// primitive pairs), heaviest bin first, so the lanes of a wavefront run loops
+// of similar length; within a bin the order is P-major, Q ascending.
 __device__ __forceinline__ int cost_bin(int c) {
     return c > 256 ? 0 : c > 64 ? 1 : c > 16 ? 2 : c > 4 ? 3 : 4;
 }
 
-// list bin of a kept quartet: precision part, then cost bin
-__device__ __forceinline__ int list_bin(double qq, double sw, int cost) {
-    return (qq < sw ? NCOSTBIN : 0) + cost_bin(cost);
-}
-
 // One wavefront per pair P, lanes over Q <= P in chunks of 64: counts per
-// (class, list bin) into counts[vc * npair + P], vc = class * NB + bin, with
-// NB = NLBIN (precision split at sw) or NCOSTBIN (no split). Per (partner
+// (class, cost bin) into counts[vc * npair + P], vc = class * NCOSTBIN + bin. Per (partner
 // class, bin) histogram in LDS (integer adds: order-independent).
-template <int NB>
-__global__ __launch_bounds__(64) void k_count_quartets(PairArgs g, double thr, double sw, int* counts) {
+__global__ __launch_bounds__(64) void k_count_quartets(PairArgs g, double thr, int* counts) {
+    constexpr int NB = NCOSTBIN;
     __shared__ int hist[6 * NB];
     const int P = blockIdx.x;
     const int lane = threadIdx.x;
@@ -141,8 +134,7 @@ __global__ __launch_bounds__(64) void k_count_quartets(PairArgs g, double thr, d
     for (int Q = lo + lane; Q <= P; Q += 64) {
         const double qq = qp * g.qscr[Q];
         if (qq < thr) continue;
-        atomicAdd(&hist[g.pair_cls[Q] * NB + (NB == NLBIN ? list_bin(qq, sw, np * g.npp[Q]) : cost_bin(np * g.npp[Q]))],
-                  1);
+        atomicAdd(&hist[g.pair_cls[Q] * NB + cost_bin(np * g.npp[Q])], 1);
     }
     __syncthreads();
     for (int vc = lane; vc < NQCLASS * NB; vc += 64) {
@@ -199,9 +191,9 @@ __global__ void k_scan_totals(const long long* totals, int n, long long* base) {
 
 // Ordered fill: per 64-partner chunk, one ballot per key present (the chunk's
 // lanes grouped by (partner class, bin)), running offsets in LDS.
-template <int NB>
-__global__ __launch_bounds__(64) void k_fill_quartets(PairArgs g, double thr, double sw, const long long* offs,
+__global__ __launch_bounds__(64) void k_fill_quartets(PairArgs g, double thr, const long long* offs,
                                                       const long long* base, int2* list) {
+    constexpr int NB = NCOSTBIN;
     __shared__ long long o[6 * NB];
     const int P = blockIdx.x;
     const int lane = threadIdx.x;
@@ -219,9 +211,7 @@ __global__ __launch_bounds__(64) void k_fill_quartets(PairArgs g, double thr, do
         const int Q = Q0 + lane;
         const double qq = Q <= P ? qp * g.qscr[Q] : 0.0;
         const bool in = Q <= P && !(qq < thr);
-        const int key = in ? g.pair_cls[Q] * NB +
-                                 (NB == NLBIN ? list_bin(qq, sw, np * g.npp[Q]) : cost_bin(np * g.npp[Q]))
-                           : -1;
+        const int key = in ? g.pair_cls[Q] * NB + cost_bin(np * g.npp[Q]) : -1;
         unsigned long long active = __ballot(in);
         while (active) {
             const int kk = __shfl(key, __ffsll((long long)active) - 1, 64);
@@ -310,24 +300,17 @@ void launch_schwarz(const PairArgs& g, const int* ncls_host, hipStream_t st) {
     if (g.nbpair) k_block_q<<<GRID(g.nbpair, 64), 0, st>>>(g);
 }
 
-// columns per class: NLBIN with a precision split (sw > 0), else NCOSTBIN
-int list_bins(double sw) { return sw > 0.0 ? NLBIN : NCOSTBIN; }
-
-void launch_count_quartets(const PairArgs& g, double thr, double sw, int* counts, long long* offs, long long* totals,
+void launch_count_quartets(const PairArgs& g, double thr, int* counts, long long* offs, long long* totals,
                            long long* base, hipStream_t st) {
     if (!g.npair) return;
-    const int nb = list_bins(sw);
-    if (nb == NLBIN) k_count_quartets<NLBIN><<<dim3(g.npair), dim3(64), 0, st>>>(g, thr, sw, counts);
-    else k_count_quartets<NCOSTBIN><<<dim3(g.npair), dim3(64), 0, st>>>(g, thr, sw, counts);
-    k_scan_columns<<<dim3(NQCLASS * nb), dim3(1024), 0, st>>>(counts, g.npair, offs, totals);
-    k_scan_totals<<<dim3(1), dim3(1), 0, st>>>(totals, NQCLASS * nb, base);
+    k_count_quartets<<<dim3(g.npair), dim3(64), 0, st>>>(g, thr, counts);
+    k_scan_columns<<<dim3(NQCLASS * NCOSTBIN), dim3(1024), 0, st>>>(counts, g.npair, offs, totals);
+    k_scan_totals<<<dim3(1), dim3(1), 0, st>>>(totals, NQCLASS * NCOSTBIN, base);
 }
 
-void launch_fill_quartets(const PairArgs& g, double thr, double sw, const long long* offs, const long long* base,
-                          int2* list, hipStream_t st) {
-    if (!g.npair) return;
-    if (list_bins(sw) == NLBIN) k_fill_quartets<NLBIN><<<dim3(g.npair), dim3(64), 0, st>>>(g, thr, sw, offs, base, list);
-    else k_fill_quartets<NCOSTBIN><<<dim3(g.npair), dim3(64), 0, st>>>(g, thr, sw, offs, base, list);
+void launch_fill_quartets(const PairArgs& g, double thr, const long long* offs, const long long* base, int2* list,
+                          hipStream_t st) {
+    if (g.npair) k_fill_quartets<<<dim3(g.npair), dim3(64), 0, st>>>(g, thr, offs, base, list);
 }
 
 // per shell pair (thread per pair): largest |D| over its block, for Dc and each Dx

@@ -35,18 +35,6 @@ void launch_grad_keep(int k, const GradArgs& a, const int2* list, long long nq, 
     fns[k](a, list, nq, st);
 }
 
-void launch_grad(const GradArgs& a, const int2* const* lists, const long long* counts, hipStream_t st) {
-    typedef void (*Fn)(const GradArgs&, const int2*, long long, hipStream_t);
-    static const Fn fns[21] = {
-        launch_grad_class_0, launch_grad_class_1, launch_grad_class_2, launch_grad_class_3,
-        launch_grad_class_4, launch_grad_class_5, launch_grad_class_6, launch_grad_class_7,
-        launch_grad_class_8, launch_grad_class_9, launch_grad_class_10, launch_grad_class_11,
-        launch_grad_class_12, launch_grad_class_13, launch_grad_class_14, launch_grad_class_15,
-        launch_grad_class_16, launch_grad_class_17, launch_grad_class_18, launch_grad_class_19,
-        launch_grad_class_20};
-    for (int k = 0; k < 21; ++k) fns[k](a, lists[k], counts[k], st);
-}
-
 #define DECLS(k) void launch_eri_##k(const EriArgs&, long long, long long, long long, long long, hipStream_t); \
     void launch_digest_##k(const DigestArgs&, int, hipStream_t);
 DECLS(0) DECLS(1) DECLS(2) DECLS(3) DECLS(4) DECLS(5) DECLS(6) DECLS(7) DECLS(8) DECLS(9) DECLS(10)
