@@ -11,13 +11,16 @@ namespace aimdhf {
 
 namespace {
 constexpr int QC = AIMDHF_QCLASS;
-// threads of a workgroup: where its rows leave room for few workgroups on a CU, 512;
-// the classes that need more than 128 registers a lane stay at 256 (measured on 32
-// waters, 6-31G*: class 6 674 -> 509 us, class 10 504 -> 350, class 18 194 -> 247)
+// threads of a workgroup: where its rows leave room for few workgroups on a CU, 512; the
+// classes that need more than 128 registers a lane spill there and stay at 256. Alone,
+// 256 : 512 threads, 6-31G*: (H2O)32 class 6 393 : 330 us, class 10 300 : 226, class 18
+// 159 : 258; (H2O)16 class 10 49 : 42, class 15 54 : 43, class 16 75 : 120; the whole build
+// of (H2O)32 4.31 ms with 256 in every class, 4.52 with 512, 4.19 so
 constexpr int MAXT = QC == 4 || QC == 5 || QC == 8 || QC >= 16 ? 256 : 512;
 // two densities in one workgroup (each integral read once) where the sums of both fit
-// the registers, else a workgroup each: UHF (H2O)8/cc-pVDZ 0.59 ms per build, against
-// 0.66 with both up to class 11 and 0.78 up to class 15
+// the registers, else a workgroup each: per build with each alone, so, and both up to
+// class 9: (H2O)32 6-31G* 8.22, 8.06, 8.19 ms; (H2O)16 1.22, 1.17, 1.21; cc-pVDZ (H2O)12
+// 1.48, 1.40, 1.40; (H2O)8 0.52, 0.51, 0.55 (up to class 15 0.78)
 constexpr bool BOTH = QC < 5;
 
 template <int QC_, int NSET, bool LDSROWS>

@@ -126,8 +126,8 @@ __device__ __forceinline__ void fx_add(long long* acc, int atom, int d, double x
 // otherwise be one chain; LDS staging when use_lds (6 * natm * 8 bytes of dynamic
 // shared memory). Bound by the serial chain of one wavefront (d d: 130 KB of straight
 // code), so the classes also run on streams of their own: with the lane split a step of
-// one water molecule 4.93 -> 4.59 ms, of 12 replicas 9.87 -> 9.59 ms, the forces of five
-// (UHF) from 1.06 to 1.16 times the rate of one class after the other.
+// one water molecule 4.93 -> 4.59 ms, of 12 replicas 9.87 -> 9.59 ms; the gradient alone,
+// class after class, of five waters in cc-pVDZ 0.73 -> 0.57 ms, of 16 in 6-31G* 0.86 -> 0.81.
 template <int LI, int LJ>
 __global__ __launch_bounds__(256) void k_grad_one_cls(OneElArgs g, const int* pairs, int np, const double* D,
                                                       const double* Wneg, long long* out, int use_lds) {
