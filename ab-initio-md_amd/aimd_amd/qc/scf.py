@@ -1060,9 +1060,10 @@ class SCFSolver:
         perr = torch.empty(nspin, dtype=torch.float64, device=Ds.device)
         L = _lib.lib()
         with torch.cuda.device(Ds.device):
-            _lib.check(L.aimdhf_batch_purify(nspin, n, _ptr(Fo), _ptr(nocc), _ptr(P), steps, tol, _ptr(perr), _stream()))
+            st = _stream()
+            _lib.check(L.aimdhf_batch_purify(nspin, n, _ptr(Fo), _ptr(nocc), _ptr(P), steps, tol, _ptr(perr), st))
             _lib.check(L.aimdhf_small_density(1, nspin, n, _ptr(X), _ptr(P), _ptr(Dn), None, None, None, None, 0.0,
-                                              0.0, None, None, 0, _stream()))
+                                              0.0, None, None, 0, st))
         return Dn if all(e < tol for e in perr.tolist()) else None
 
     def _fock(self, I: SCFIntegrals, Ds: torch.Tensor, jk: tuple | None = None) -> torch.Tensor:
