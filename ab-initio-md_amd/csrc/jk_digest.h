@@ -159,7 +159,11 @@ __device__ inline double jk_bound_k(const unsigned long long* g, const unsigned 
     return __longlong_as_double((long long)g[1]) * __longlong_as_double((long long)d[0]);
 }
 __device__ inline double jk_bound_j(const unsigned long long* g, const unsigned long long* d, int n) {
-    const double cs = sqrt((double)g[2] * (1.0 / 1048576.0) * n * __longlong_as_double((long long)d[1]));
+    // |q|_F^2: the fixed-point sum, whose words neither saturate nor wrap while n times the
+    // largest row is below their range, or that bound (larger integrals; and much smaller
+    // ones, of which the sum only counts the rounded-up units)
+    const double rows = n * __longlong_as_double((long long)g[1]), fq = (double)g[2] * (1.0 / 1048576.0);
+    const double cs = sqrt((rows < 1e12 && fq < rows ? fq : rows) * (n * __longlong_as_double((long long)d[1])));
     const double sum = (double)d[3] * (1.0 / 16777216.0);
     // the fixed-point sum cannot have wrapped while the other bound is below its range
     return __longlong_as_double((long long)g[0]) * (cs < 1e9 && sum < cs ? sum : cs);

@@ -2,7 +2,7 @@
 The single-read J/K digestion at the edges of its routes: bases of one angular
 momentum, integral lists past the size of one launch, direct mode's pieces,
 matrices of more than 16384 orbitals, builds that a graph records, what difference
-builds leave out, densities with one dominant element.
+builds leave out, densities with one dominant element, coefficients of any magnitude.
 """
 
 import numpy as np
@@ -287,3 +287,24 @@ def test_one_dominant_density_element(oracle_lib):
     assert np.abs(J.cpu().numpy() - Jo).max() < b.nao * 2.0 ** -53 * bound_j
     assert np.abs(K.cpu().numpy() - Ko).max() < b.nao * 2.0 ** -53 * bound_k
     e.close()
+
+
+@pytest.mark.parametrize("power", [6, 10, 12, 40, -30])
+def test_coefficients_of_any_magnitude(power):
+    """Contraction coefficients scaled by c = 2^power scale every integral, J and K by c^4, whatever the
+    magnitude of the Schwarz bounds that set the words' exponents (q grows as c^2: the sum of its
+    squares passes 1e12 at 2^10)."""
+    from aimd_amd.qc.basis import BasisSet, build_basis
+    from aimd_amd.qc.engine import Engine
+    s, x = water_dimer()
+    b = build_basis(s, x, "6-31g*")
+    D = _dens(b.nao, 2, 17)
+    out = []
+    for c in (1.0, 2.0 ** power):
+        e = Engine(BasisSet("scaled", s, x, b.shell_atom, b.shell_l, b.shell_prim, b.prim_exp, c * b.prim_coef))
+        e.set_jk_mode("store")
+        e.set_geometry(x, 1e-12 * c ** 4)
+        out.append(e.jk(D))
+        e.close()
+    for ref, got in zip(*out):
+        assert float((got / 2.0 ** (4 * power) - ref).abs().max()) < 1e-13 * float(ref.abs().max())
