@@ -1386,6 +1386,7 @@ int aimdhf_grad_quartets(aimdhf_plan* p, int64_t* out, int64_t cap, int64_t* cou
 static int jk_from_store(aimdhf_plan* p, int nset, const double* dens, double* J, double* K, bool delta, double dthr,
                          hipStream_t st) {
     try {
+        p->have_last_store = false;     // a failed allocation below leaves the last build's arguments stale
         p->ensure_digest(nset);
         const aimdhf::PrepArgs pa = p->prep_args(nset, dens, J, K);
         p->prof.time(45, st, [&] { aimdhf::launch_jk_prep(pa, st); });

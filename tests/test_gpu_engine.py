@@ -178,3 +178,21 @@ def test_one_electron_terms_over_nuclei_and_primitive_pairs(oracle_lib, natm):
     again = e.grad_one(torch.tensor(P, device="cuda"), torch.tensor(W, device="cuda")).cpu().numpy()
     np.testing.assert_array_equal(g, again)
     e.close()
+
+
+def test_replay_of_a_digestion_kernel_needs_a_build():
+    """Timing replays take the arguments of the last build at the current geometry: refused before one
+    and after a new geometry; they leave later builds as they were."""
+    import torch
+    s, x = water_dimer()
+    b, e = _engine(s, x, "6-31g*", "store")
+    D = torch.tensor(np.random.default_rng(5).standard_normal((1, b.nao, b.nao)), device="cuda")
+    for _ in range(2):
+        with pytest.raises(RuntimeError):
+            e.profile_replay(98)
+        ref = e.jk(D)
+        assert e.profile_replay(98, 3) > 0.0
+        for a, c in zip(ref, e.jk(D)):
+            assert torch.equal(a, c)
+        e.set_geometry(x)
+    e.close()
