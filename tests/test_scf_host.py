@@ -179,6 +179,7 @@ def test_small_scf_algebra_launches_on_the_device_of_its_tensors(monkeypatch):
             return lambda *args: seen.append((name, list(active))) or 0
 
     monkeypatch.setattr(torch.cuda, "device", Guard)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
     monkeypatch.setattr(S._lib, "lib", Recorder)
     monkeypatch.setattr(S, "_stream", lambda: seen.append(("stream", list(active))))
     solver = object.__new__(S.SCFSolver)
